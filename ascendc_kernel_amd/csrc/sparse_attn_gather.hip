@@ -3,7 +3,9 @@
 // of sparse_attn_ref, reference/task1_v0_ref.py:5-24; duplicates and masked
 // slots handled exactly like the gather there).
 //
-// One workgroup per token, one wave per 32 heads (ceil(h/32) waves). The slots are
+// Two kernels, chosen by gather_split: this file's sa_gather_kernel (many tokens of more
+// than 32 heads) and sa_gather_split_kernel (few tokens, or at most 32 heads). The former:
+// one workgroup per token, one wave per 32 heads (ceil(h/32) waves). The slots are
 // processed in blocks of 32. The selected kv rows (256 B each) of a block are
 // copied straight from global memory into LDS by global_load_lds_dwordx4 (no
 // register staging), into a ring of kRing block buffers: kRing - 1 blocks are in
@@ -62,7 +64,7 @@ __device__ __forceinline__ int out_ch(int dt, int i) {
 __device__ __forceinline__ int swz(int r, int c) { return r * 16 + (c ^ (r & 15)); }
 
 template <int NW, typename IdxT>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW >= 2 ? 2 : 1)))
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 void sa_gather_kernel(GatherParams p) {
   const IdxT* const idx = static_cast<const IdxT*>(p.idx);
   __shared__ u32x4 ring[kRing][kKB * 16];  // kRing blocks of 32 gathered rows (8 KB each)
@@ -381,6 +383,334 @@ void sa_gather_kernel(GatherParams p) {
   }
 }
 
+// One workgroup per (token, 32 heads), whose slot blocks are divided among SP waves: wave
+// w takes blocks w, w + SP, ... . Every wave copies its own blocks into its own two LDS
+// buffers, so the block loop has no barrier; blocks without a valid slot are skipped.
+// Each wave starts its running max at the sink and keeps its own sum and O^T; at the end
+// these go to LDS (O^T over the wave's own buffers) and every wave adds up and normalises
+// 64 / SP of the 64 register rows over all SP states (in fp32, one rounding to bf16).
+//
+// What bounds it: with few tokens the latency of the slot list, the rows and one block
+// after the other (~0.8 us each), which the split divides; 8 tokens of 64 heads, 512 slots
+// of 8192 rows: 16.4 us with the blocks in sequence (sa_gather_kernel), 8.3 us with SP 4;
+// 2048 slots: 52.9 us, 17.1 us with SP 8. With many tokens SP 1 serves up to 32 heads:
+// 17 KB of LDS per wave instead of the 4-buffer ring's 33 KB keeps two waves on each SIMD
+// (4,800 tokens of 16 heads, 256 slots: 57.1 -> 42.4 us). SP 2 was the best choice
+// nowhere by more than 8 %.
+constexpr int kSplitRing = 2;
+
+template <int SP, typename IdxT>
+__global__ __launch_bounds__(64 * SP) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void sa_gather_split_kernel(GatherParams p) {
+  static_assert(SP == 1 || SP == 4 || SP == 8, "slot ranges per workgroup");
+  const IdxT* const idx = static_cast<const IdxT*>(p.idx);
+  __shared__ u32x4 ring[SP][kSplitRing][kKB * 16];
+  __shared__ float ml[SP][2][64];   // per wave and lane: running max, partial sum
+  extern __shared__ int32_t slot[];  // the token's slot indices (masked -> -1)
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wi = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ngrp = (p.H + 31) >> 5;  // head groups of 32 (the last may be half full)
+  // Blocks go to the 8 XCDs round-robin: the head groups of a token, which read the same
+  // rows, take blocks of one XCD, and where sa_gather_kernel pins a batch to an XCD so
+  // does this map. The grid is rounded up to 8 tokens; surplus blocks leave at once.
+  const unsigned xcd = blockIdx.x & 7u, slotno = (blockIdx.x >> 3) / (unsigned)ngrp;
+  const int hbase = 32 * (int)((blockIdx.x >> 3) - slotno * (unsigned)ngrp);
+  const int64_t tok = p.xpb > 0
+      ? (int64_t)(xcd % (unsigned)p.B) * p.M + (int64_t)slotno * p.xpb + xcd / (unsigned)p.B
+      : (int64_t)slotno * 8 + xcd;
+  if (tok >= p.B * p.M) return;
+  const int b = (int)(tok / p.M);
+  const int col = lane & 31;
+  const int hf = lane >> 5;
+  const bool hvalid = hbase + col < p.H;
+
+  // As in sa_gather_kernel: every global read of the token is issued before the first wait.
+  bf16x8 qf[8];
+  {
+    const uint16_t* qrow = p.q + (tok * p.H + (hvalid ? hbase + col : 0)) * kD + 8 * hf;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+      qf[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(qrow + 16 * ks));
+  }
+  const float sink_raw = p.sink[hvalid ? hbase + col : 0];
+  const int nblk = (p.TOPK + kKB - 1) / kKB;
+  auto slot_chunk = [&](const int s0) {
+    int v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int s = s0 + 64 * SP * u + tid;
+      v[u] = slot_index(idx, tok * p.TOPK + min(s, p.TOPK - 1));
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int s = s0 + 64 * SP * u + tid;
+      if (s < nblk * kKB) slot[s] = (s < p.TOPK && v[u] < p.NKV) ? v[u] : -1;
+    }
+  };
+  slot_chunk(0);
+  for (int s0 = 4 * 64 * SP; s0 < nblk * kKB; s0 += 4 * 64 * SP) slot_chunk(s0);
+  __syncthreads();
+
+  const i32x4 rsrc = make_rsrc(p.kv + (int64_t)b * p.NKV * kD, (uint32_t)p.NKV * (uint32_t)(kD * 2));
+  const uint32_t ring_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) u32x4*)&ring[wi][0][0];
+  // Copy block blk into buffer rs: unit u holds rows 4u .. 4u+3, lane l row 4u + l/16, chunk
+  // position l%16 (logical chunk (l%16) ^ (row & 15)); a masked row reads zeros.
+  auto issue = [&](const int blk, const int rs) {
+    int rv[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) rv[u] = slot[blk * kKB + 4 * u + (lane >> 4)];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int r = 4 * u + (lane >> 4);
+      lds_dma16(rsrc, (uint32_t)rv[u] * (uint32_t)(kD * 2) + 16u * (uint32_t)((lane & 15) ^ (r & 15)),
+                ring_lds + 8192u * (uint32_t)rs + 1024u * (uint32_t)u);
+    }
+  };
+  // The first block from blk on (in steps of SP) that holds a valid slot, or nblk; its
+  // valid slots in vm.
+  auto next_block = [&](int blk, uint32_t& vm) {
+    for (; blk < nblk; blk += SP) {
+      vm = (uint32_t)__ballot(slot[blk * kKB + (lane & 31)] >= 0);
+      if (vm != 0u) return blk;
+    }
+    vm = 0u;
+    return nblk;
+  };
+  f32x16 o[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) o[dt] = f32x16{};
+  const float sink_l2 = hvalid ? sink_raw * kLog2e : 0.f;
+  const float c2 = p.scale_log2;
+  float m_run = fmaxf(sink_l2, -FLT_MAX);  // floored as in sa_gather_kernel
+  float l_run = 0.f;
+  uint32_t neg_lo_bits = kNegLoBits, neg_hi_bits = kNegHiBits;
+  asm volatile("" : "+s"(neg_lo_bits), "+s"(neg_hi_bits));
+  const bf16v2 neg_lo = __builtin_bit_cast(bf16v2, neg_lo_bits);
+  const bf16v2 neg_hi = __builtin_bit_cast(bf16v2, neg_hi_bits);
+
+  uint32_t vm_cur, vm_nxt = 0u;
+  int cur = next_block(wi, vm_cur);
+  int nxt = nblk;
+  if (cur < nblk) {
+    issue(cur, 0);
+    nxt = next_block(cur + SP, vm_nxt);
+    if (nxt < nblk) issue(nxt, 1);
+  }
+  // The compiler-tracked loads are consumed here, so that its own vmcnt(0) for them (which
+  // also covers the copies just issued) stays out of the loop.
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) asm volatile("" ::"v"(qf[ks]));
+  asm volatile("" ::"v"(m_run));
+
+  // One block, which sits in buffer j.
+  auto step = [&](const int j) {
+    if (nxt < nblk) wait_vmcnt<8>();  // only the next block's copies may be outstanding
+    else wait_vmcnt<0>();
+    asm volatile("" ::: "memory");
+    const u32x4* kvl = ring[wi][j];
+    f32x16 s = {};
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      const bf16x8 a = __builtin_bit_cast(bf16x8, kvl[swz(lane & 31, 2 * ks + hf)]);
+      s = mfma32x32x16(a, qf[ks], s);
+    }
+    if (vm_cur != 0xffffffffu) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = 8 * (r >> 2) + 4 * hf + (r & 3);
+        if (!((vm_cur >> key) & 1u)) s[r] = -INFINITY;
+      }
+    }
+    float bmax = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) bmax = fmaxf(bmax, s[r]);
+    bmax *= c2;
+    {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(bmax), __float_as_uint(bmax),
+                                                       false, false);
+      bmax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    }
+    const bool raise = bmax > m_run + kRaise;
+    if (__ballot(raise) != 0) {
+      const float m_new = raise ? bmax : m_run;
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+      m_run = m_new;
+    }
+    float pe[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) pe[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c2, -m_run));
+#pragma unroll
+    for (int r = 0; r < 16; ++r) l_run += pe[r];
+    bf16x8 phi[2], plo[2];
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      u32x4 wh, wl;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float p0 = pe[8 * st + 2 * w], p1 = pe[8 * st + 2 * w + 1];
+        const uint32_t h = pack_bf2(p0, p1);
+        wh[w] = h;
+        const bf16v2 hv = __builtin_bit_cast(bf16v2, h);
+        wl[w] = pack_bf2(__builtin_amdgcn_fdot2_f32_bf16(hv, neg_lo, p0, false),
+                         __builtin_amdgcn_fdot2_f32_bf16(hv, neg_hi, p1, false));
+      }
+      phi[st] = __builtin_bit_cast(bf16x8, wh);
+      plo[st] = __builtin_bit_cast(bf16x8, wl);
+    }
+    const int u = lane & 15, g16 = (lane >> 4) & 1;
+    const uint16_t* kvh = reinterpret_cast<const uint16_t*>(kvl);
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        const int ch = out_ch(dt, 16 * g16 + 4 * (u & 3));
+        const int r0 = 16 * st + 4 * hf + (u >> 2);
+        const int r1 = r0 + 8;
+        const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_s16x4_ptr)(kvh + swz(r0, ch >> 3) * 8 + (ch & 7)));
+        const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_s16x4_ptr)(kvh + swz(r1, ch >> 3) * 8 + (ch & 7)));
+        const s16x8 v01 = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+        const bf16x8 a = __builtin_bit_cast(bf16x8, v01);
+        o[dt] = mfma32x32x16(a, plo[st], o[dt]);
+        o[dt] = mfma32x32x16(a, phi[st], o[dt]);
+      }
+    }
+    // Buffer j is free once its last reads have returned: refill it with the block
+    // after the next.
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    uint32_t vm_2 = 0u;
+    int nxt2 = nblk;
+    if (nxt < nblk) {
+      nxt2 = next_block(nxt + SP, vm_2);
+      if (nxt2 < nblk) issue(nxt2, j);
+    }
+    cur = nxt;
+    vm_cur = vm_nxt;
+    nxt = nxt2;
+    vm_nxt = vm_2;
+  };
+  while (cur < nblk) {
+    step(0);
+    if (cur >= nblk) break;
+    step(1);
+  }
+
+  if constexpr (SP == 1) {
+    // One state: normalise it and transpose it through the wave's own buffers (chunk c of
+    // head col at swz(col, c)), so that every store writes four whole rows.
+    l_run += __shfl_xor(l_run, 32, 64);
+    const float rz = 1.0f / (l_run + __builtin_amdgcn_exp2f(sink_l2 - m_run));
+    u32x4* obuf = &ring[0][0][0];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      u32x4 w;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        w[k] = pack_bf2(o[c >> 1][8 * (c & 1) + 2 * k] * rz, o[c >> 1][8 * (c & 1) + 2 * k + 1] * rz);
+      obuf[swz(col, 8 * hf + c)] = w;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    u32x4* dst = reinterpret_cast<u32x4*>(p.out + (tok * p.H + hbase) * kD);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int r = 4 * k + (lane >> 4), c = lane & 15;
+      if (hbase + r < p.H) st_nt(dst + r * 16 + c, obuf[swz(r, c)]);
+    }
+    return;
+  }
+  // The states of all waves: O^T register rows 4k .. 4k+3 of a lane at [k][lane].
+  u32x4* mine = &ring[wi][0][0];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const f32x4 v = {o[dt][4 * k], o[dt][4 * k + 1], o[dt][4 * k + 2], o[dt][4 * k + 3]};
+      mine[(4 * dt + k) * 64 + lane] = __builtin_bit_cast(u32x4, v);
+    }
+  ml[wi][0][lane] = m_run;
+  ml[wi][1][lane] = l_run;
+  __syncthreads();
+  float mx = m_run;
+#pragma unroll
+  for (int w = 0; w < SP; ++w) mx = fmaxf(mx, ml[w][0][lane]);
+  float z = __builtin_amdgcn_exp2f(sink_l2 - mx);
+  float f[SP];
+#pragma unroll
+  for (int w = 0; w < SP; ++w) {
+    f[w] = __builtin_amdgcn_exp2f(ml[w][0][lane] - mx);
+    z += (ml[w][1][col] + ml[w][1][col + 32]) * f[w];
+  }
+  const float rz = 1.0f / z;
+  // Wave wi finishes 8 / SP chunks of 8 channels per lane (chunk c = register rows
+  // 8c .. 8c+7 = channels 64 hf + 8 c .. +7 of head col).
+#pragma unroll
+  for (int i = 0; i < 8 / SP; ++i) {
+    const int c = (8 / SP) * wi + i;
+    f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < SP; ++w) {
+      const f32x4 v0 = __builtin_bit_cast(f32x4, (&ring[w][0][0])[(2 * c) * 64 + lane]);
+      const f32x4 v1 = __builtin_bit_cast(f32x4, (&ring[w][0][0])[(2 * c + 1) * 64 + lane]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        a0[k] += v0[k] * f[w];
+        a1[k] += v1[k] * f[w];
+      }
+    }
+    const u32x4 w = {pack_bf2(a0[0] * rz, a0[1] * rz), pack_bf2(a0[2] * rz, a0[3] * rz),
+                     pack_bf2(a1[0] * rz, a1[1] * rz), pack_bf2(a1[2] * rz, a1[3] * rz)};
+    if (hvalid)
+      *reinterpret_cast<u32x4*>(p.out + (tok * p.H + hbase + col) * kD + 64 * hf + 8 * c) = w;
+  }
+}
+
+// Waves per (token, 32 heads) of sa_gather_split_kernel, or 0 for sa_gather_kernel, for
+// `groups` = tokens x head groups of nblk slot blocks on cu CUs. Measured at 16 .. 128
+// heads, 32 .. 2048 slots and 8 .. 8192 groups (256 CUs; us, sequential -> split):
+//  up to one group per CU the split takes the CU's waves: 8 from 32 blocks on (1024 slots:
+//    35.0 -> 12.5, four waves 13.3), 4 from 4 blocks on (128 slots: 7.3 -> 5.5), else one
+//    (64 slots: 5.8 -> 5.1);
+//  up to two groups per CU, 4 waves from 8 blocks on (512 slots, 512 groups: 16.8 -> 13.1);
+//    with fewer blocks the states cost what the split saves (128 slots: 7.7 -> 8.4);
+//  beyond that, 64 and more heads stay sequential, where the waves of a token share each
+//    row's copy (512 slots, 1536 groups: 23.3, one wave 27.6), and up to 32 heads take one
+//    wave (512 slots, 8192 groups: 153.8 -> 108), or 4 where the slot list would leave
+//    room for fewer than 7 one-wave workgroups per CU (2048 slots, 3072 groups: one wave
+//    181, four 169).
+int gather_split(int64_t groups, int nw, int64_t nblk, int cu) {
+  if (groups <= cu) return nblk >= 32 ? 8 : nblk >= 4 ? 4 : 1;
+  if (groups <= 2 * (int64_t)cu && nblk >= 8) return 4;
+  if (nw > 1) return 0;
+  return nblk >= 48 ? 4 : 1;
+}
+
+template <typename IdxT>
+int launch_split(const GatherParams& p, int sp, unsigned blocks, size_t smem, hipStream_t stream) {
+  switch (sp) {
+#define DSA_GATHER_CASE(n)                                                                          \
+  case n:                                                                                           \
+    if (dsa_host::ensure_dyn_lds((const void*)sa_gather_split_kernel<n, IdxT>, (int)smem) != DSA_OK) \
+      return DSA_ERR_LAUNCH;                                                                        \
+    hipLaunchKernelGGL((sa_gather_split_kernel<n, IdxT>), dim3(blocks), dim3(64 * n), smem, stream, p); \
+    break;
+    DSA_GATHER_CASE(1)
+    DSA_GATHER_CASE(4)
+    DSA_GATHER_CASE(8)
+#undef DSA_GATHER_CASE
+    default:
+      return DSA_ERR_UNSUPPORTED;
+  }
+  return hipGetLastError() == hipSuccess ? DSA_OK : DSA_ERR_LAUNCH;
+}
+
 }  // namespace
 
 int dsa_sparse_attn_gather_launch(const void* q, const void* kv, const void* idx, bool idx64,
@@ -405,21 +735,29 @@ int dsa_sparse_attn_gather_launch(const void* q, const void* kv, const void* idx
   p.TOPK = (int32_t)topk;
   p.scale_log2 = scale * kLog2e;
   p.xpb = (b <= 8 && 8 % b == 0 && m % (8 / b) == 0) ? (int32_t)(8 / b) : 0;
-  const dim3 grid((unsigned)tokens);
   // Dynamic LDS: the slot list, padded to whole blocks.
-  const size_t smem = (size_t)((topk + kKB - 1) / kKB) * kKB * sizeof(int32_t);
+  const int64_t nblk = (topk + kKB - 1) / kKB;
+  const size_t smem = (size_t)nblk * kKB * sizeof(int32_t);
   const int nw = (int)((h + 31) / 32);
   if (nw < 1 || nw > 4) return DSA_ERR_UNSUPPORTED;
+  int cu = 0;
+  if (dsa_host::device_cu_count(&cu) != DSA_OK) return DSA_ERR_DEVICE;
+  const int sp = gather_split(tokens * nw, nw, nblk, cu);
+  if (sp > 0) {
+    const int64_t blocks = (tokens + 7) / 8 * 8 * nw;
+    if (blocks > INT32_MAX) return DSA_ERR_SHAPE;
+    return idx64 ? launch_split<int64_t>(p, sp, (unsigned)blocks, smem, stream)
+                 : launch_split<int32_t>(p, sp, (unsigned)blocks, smem, stream);
+  }
+  const dim3 grid((unsigned)tokens);
   if (idx64) {
     switch (nw) {
-      case 1: hipLaunchKernelGGL((sa_gather_kernel<1, int64_t>), grid, dim3(64), smem, stream, p); break;
       case 2: hipLaunchKernelGGL((sa_gather_kernel<2, int64_t>), grid, dim3(128), smem, stream, p); break;
       case 3: hipLaunchKernelGGL((sa_gather_kernel<3, int64_t>), grid, dim3(192), smem, stream, p); break;
       default: hipLaunchKernelGGL((sa_gather_kernel<4, int64_t>), grid, dim3(256), smem, stream, p); break;
     }
   } else {
     switch (nw) {
-      case 1: hipLaunchKernelGGL((sa_gather_kernel<1, int32_t>), grid, dim3(64), smem, stream, p); break;
       case 2: hipLaunchKernelGGL((sa_gather_kernel<2, int32_t>), grid, dim3(128), smem, stream, p); break;
       case 3: hipLaunchKernelGGL((sa_gather_kernel<3, int32_t>), grid, dim3(192), smem, stream, p); break;
       default: hipLaunchKernelGGL((sa_gather_kernel<4, int32_t>), grid, dim3(256), smem, stream, p); break;

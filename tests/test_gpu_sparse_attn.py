@@ -263,6 +263,40 @@ def test_gather_shapes_and_masks(gpu, case):
     _compare(out, ref, f"gather{case}")
 
 
+# The edges of the split of a token's slot blocks over waves (256 CUs; groups = tokens x
+# ceil(h / 32), blocks of 32 slots): one block and its remainders, 3 / 4 blocks, 31 / 32
+# blocks, 256 / 257 groups, 512 / 513 groups with 7 / 8 blocks, up to 32 heads beyond that
+# with 47 / 48 blocks, token counts that are no multiple of 8, half-filled head groups.
+SPLIT_CASES = [
+    # b, m, h, n_kv, topk
+    (1, 1, 64, 70, 1), (1, 3, 16, 40, 31), (3, 1, 128, 100, 33), (1, 5, 48, 400, 96), (1, 5, 48, 400, 97),
+    (8, 1, 64, 2000, 992), (8, 1, 64, 2000, 993), (1, 2, 112, 3000, 2048),
+    (2, 64, 64, 300, 200), (1, 129, 64, 300, 200), (1, 257, 32, 300, 100), (1, 256, 16, 900, 1024),
+    (1, 128, 128, 300, 224), (4, 32, 112, 300, 225), (1, 171, 80, 300, 260), (3, 171, 32, 300, 225),
+    (1, 515, 16, 300, 300), (2, 260, 32, 1600, 1504), (2, 260, 32, 1600, 1505),
+]
+
+
+@pytest.mark.parametrize("case", SPLIT_CASES)
+def test_gather_split_edges(gpu, case):
+    """Every form of the split against the oracle, with whole blocks masked (among them the
+    only block of some waves), a token without any slot, and int64 slots giving the int32
+    result bit for bit."""
+    b, m, h, n_kv, topk = case
+    _say("gather split case", case)
+    q, kv, idx, sink = _case(b, m, h, n_kv, topk, 33, 0.1, 1.0)
+    idx[..., 32:64] = -1
+    idx[:, 1::3, 96:200] = -1
+    idx[0, 0] = -1
+    out = _native.sparse_attn_fwd(q, kv, idx, sink, 128 ** -0.5, _native.DSA_SA_GATHER)
+    ref = torch.cat([osa.sparse_attn_ref(q[:, i:i + 64], kv, sink, idx[:, i:i + 64], 128 ** -0.5)
+                     for i in range(0, m, 64)], dim=1)
+    _compare(out, ref, f"split{case}")
+    assert torch.count_nonzero(out[0, 0]) == 0
+    out64 = _native.sparse_attn_fwd(q, kv, idx.long(), sink, 128 ** -0.5, _native.DSA_SA_GATHER)
+    assert torch.equal(out64.view(torch.int16), out.view(torch.int16))
+
+
 @pytest.mark.parametrize("variant", [_native.DSA_SA_GATHER, _native.DSA_SA_MULTIPLICITY])
 def test_neg_inf_sink_masked_leading_block(gpu, variant):
     """A -inf sink on half the heads with the first slot blocks of every token masked: no
