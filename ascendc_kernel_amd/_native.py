@@ -14,7 +14,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 DSA_SA_AUTO = 0
 DSA_SA_MULTIPLICITY = 1
@@ -42,6 +42,7 @@ EXPORTS = (
     "dsa_indexer_q_proj",
     "dsa_indexer_pack_projection_weights",
     "dsa_indexer_projections",
+    "dsa_indexer_projections_splitk",
     "dsa_indexer_decode_projections",
 )
 
@@ -130,10 +131,12 @@ def load() -> ctypes.CDLL:
     lib.dsa_indexer_pack_projection_weights.restype = ctypes.c_int
     lib.dsa_indexer_pack_projection_weights.argtypes = [
         _c_vp, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64, _c_vp, _c_vp, _c_vp]
-    lib.dsa_indexer_projections.restype = ctypes.c_int
-    lib.dsa_indexer_projections.argtypes = [
-        _c_vp, _c_vp, _c_vp, ctypes.c_int32, _c_vp, _c_vp, _c_vp, _c_vp,
-        _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp]
+    for name in ("dsa_indexer_projections", "dsa_indexer_projections_splitk"):
+        fn = getattr(lib, name)
+        fn.restype = ctypes.c_int
+        fn.argtypes = [
+            _c_vp, _c_vp, _c_vp, ctypes.c_int32, _c_vp, _c_vp, _c_vp, _c_vp,
+            _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp]
     lib.dsa_indexer_decode_projections.restype = ctypes.c_int
     lib.dsa_indexer_decode_projections.argtypes = [
         _c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp]
@@ -496,9 +499,10 @@ PROJ_SLOT_Q, PROJ_SLOT_WL = 4, 7
 
 def prepare_indexer_projections(qr: torch.Tensor, wq_packed: torch.Tensor, freqs_cis: Optional[torch.Tensor],
                                 x: torch.Tensor, wproj_packed: torch.Tensor, head_dim: int, rope_head_dim: int,
-                                rope_mode: int = DSA_ROPE_TORCH_ROCM):
-    """Checks and marshals dsa_indexer_projections; returns (Launch, q_shape, wl_shape, keep)
-    with the outputs in the argument slots PROJ_SLOT_Q and PROJ_SLOT_WL."""
+                                rope_mode: int = DSA_ROPE_TORCH_ROCM, splitk: bool = False):
+    """Checks and marshals dsa_indexer_projections (packed weights) or, with splitk,
+    dsa_indexer_projections_splitk (the Linear weights as they are); returns (Launch, q_shape,
+    wl_shape, keep) with the outputs in the argument slots PROJ_SLOT_Q and PROJ_SLOT_WL."""
     load()
     if qr.dim() != 3 or x.dim() != 3 or qr.shape[:2] != x.shape[:2]:
         raise ValueError(f"qr {tuple(qr.shape)} and x {tuple(x.shape)} do not match")
@@ -509,7 +513,11 @@ def prepare_indexer_projections(qr: torch.Tensor, wq_packed: torch.Tensor, freqs
     n = wq_packed.shape[0]
     n_w = wproj_packed.shape[0]
     if wq_packed.shape[1] != k or wproj_packed.shape[1] != dim:
-        raise ValueError("packed weights do not match qr / x")
+        raise ValueError("weights do not match qr / x")
+    if splitk:
+        if wq_packed.dtype != torch.bfloat16 or wproj_packed.dtype != torch.bfloat16:
+            raise TypeError("the weights must be bfloat16")
+        wq_packed, wproj_packed = wq_packed.detach().contiguous(), wproj_packed.detach().contiguous()
     qr = qr.contiguous()
     x = x.contiguous()
     fr = _freqs_view(freqs_cis, s, rope_head_dim) if freqs_cis is not None else None
@@ -517,18 +525,20 @@ def prepare_indexer_projections(qr: torch.Tensor, wq_packed: torch.Tensor, freqs
     args = [qr.data_ptr(), wq_packed.data_ptr(), fr.data_ptr() if fr is not None else None, int(rope_mode),
             None, x.data_ptr(), wproj_packed.data_ptr(), None,
             b * s, n, k, dim, n_w, head_dim, rope_head_dim, max(s, 1), stream_handle(dev)]
-    return (Launch("dsa_indexer_projections", args), (b, s, n // head_dim, head_dim), (b, s, n_w),
+    fn = "dsa_indexer_projections_splitk" if splitk else "dsa_indexer_projections"
+    return (Launch(fn, args), (b, s, n // head_dim, head_dim), (b, s, n_w),
             (qr, x, wq_packed, wproj_packed, fr))
 
 
 def indexer_projections(qr: torch.Tensor, wq_packed: torch.Tensor, freqs_cis: Optional[torch.Tensor],
                         x: torch.Tensor, wproj_packed: torch.Tensor, head_dim: int, rope_head_dim: int,
-                        rope_mode: int = DSA_ROPE_TORCH_ROCM):
+                        rope_mode: int = DSA_ROPE_TORCH_ROCM, splitk: bool = False):
     """Both indexer projections in one launch: q = RoPE(qr . wq^T) as bf16
     [b, s, n/head_dim, head_dim] and wl = x . wproj^T as bf16 [b, s, n_w], from the
-    packed weights of ``pack_projection_weights``. qr: bf16 [b, s, 256]; x: bf16 [b, s, dim]."""
+    packed weights of ``pack_projection_weights``. qr: bf16 [b, s, 256]; x: bf16 [b, s, dim].
+    splitk: in hipBLASLt's split-k order, from the weights as they are."""
     launch, q_shape, wl_shape, _keep = prepare_indexer_projections(qr, wq_packed, freqs_cis, x, wproj_packed,
-                                                                   head_dim, rope_head_dim, rope_mode)
+                                                                   head_dim, rope_head_dim, rope_mode, splitk)
     q = torch.empty(q_shape, dtype=torch.bfloat16, device=qr.device)
     wl = torch.empty(wl_shape, dtype=torch.bfloat16, device=qr.device)
     launch.set(PROJ_SLOT_Q, q.data_ptr())

@@ -355,6 +355,7 @@ __device__ __forceinline__ void q_role(const SProjParams& p, int blk, uint8_t* s
     else
       t0 = t1 - tail;
   }
+  if (t0 >= t1) return;  // (workgroup-uniform)
   const int n0 = cg * kSCh;
   const __amdgpu_buffer_rsrc_t qrs = buf_rsrc(p.q, (uint32_t)p.M * (uint32_t)p.N * 2u);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
@@ -388,8 +389,6 @@ __device__ __forceinline__ void q_role(const SProjParams& p, int blk, uint8_t* s
       __syncthreads();
     }
   }
-  if (t0 >= t1) return;  // (workgroup-uniform)
-
   QTileCopier<RD> cp;
   cp.init(p, smem, wis, lane, t0);
   cp.issue(t0, 0);
@@ -537,7 +536,7 @@ constexpr uint32_t kWChainBytes = kWTok * kWDim * 2;
 
 struct WProjParams {
   const uint16_t* x;  // [M, 1024]
-  const u32x4* wp;    // packed weights_proj fragments [32 k-steps][64 lanes]
+  const u32x4* wp;    // weights_proj: packed fragments [32 k-steps][64 lanes], or its [16, 1024] rows
   uint16_t* wl;       // [M, 16]
   int32_t M;
   int32_t nwaves;     // waves of the w role in the grid
@@ -546,16 +545,23 @@ struct WProjParams {
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // wl for chains of 16 tokens: acc = W (16 heads x 32 k, A operand) . x^T (32 k x 16
-// tokens, B operand) over the k-steps 0..31 in order, one accumulator per chain, rounded
-// once to bf16: the natural k order, which is F.linear's on torch-ROCm where hipBLASLt
-// runs a kernel without split-k for this shape. W's fragments sit in LDS (32 KB); all 32
-// x fragments of the next chain (16 B per lane and k-step) are in flight while the
-// current chain's products run. Rows at or past M read as zero and are not stored.
+// tokens, B operand) over the k-steps 0..31 in order, rounded once to bf16. kSplit false:
+// one accumulator, the natural k order, which is F.linear's on torch-ROCm where hipBLASLt
+// runs a kernel without split-k for this shape. kSplit true: four accumulators, step ks
+// into accumulator ks % 4, summed in order: hipBLASLt's local split of k over 4 waves in
+// depth blocks of 128. W's fragments sit in LDS (32 KB, from the packed copy or from W's
+// rows); all 32 x fragments of the next chain (16 B per lane and k-step) are in flight
+// while the current chain's products run. Rows at or past M read as zero and are not
+// stored.
+template <bool kSplit, bool kPacked>
 __device__ __forceinline__ void w_role(const WProjParams& p, int wblk, uint8_t* smem) {
   const int tid = threadIdx.x, lane = tid & 63, wi = tid >> 6;
   u32x4* wls = reinterpret_cast<u32x4*>(smem);
 #pragma unroll
-  for (int i = 0; i < kWSteps * 64 / 256; ++i) wls[tid + 256 * i] = p.wp[tid + 256 * i];
+  for (int i = 0; i < kWSteps * 64 / 256; ++i) {
+    const int e = tid + 256 * i;  // fragment e: row e % 16, chunk 4 (e / 64) + (e / 16) % 4 of W
+    wls[e] = kPacked ? p.wp[e] : p.wp[(e & 15) * (kWDim / 8) + 4 * (e >> 6) + ((e >> 4) & 3)];
+  }
   __syncthreads();
   const int gw = wblk * 4 + wi;
   const int nch = (p.M + kWTok - 1) / kWTok;
@@ -578,14 +584,17 @@ __device__ __forceinline__ void w_role(const WProjParams& p, int wblk, uint8_t* 
     // read, product, next chain's load) is pinned so that only a few W fragments are
     // live beside the 32 x fragments.
     constexpr int kWPre = 4;
-    f32x4 acc = f32x4{};
+    constexpr int kAcc = kSplit ? 4 : 1;
+    f32x4 acc[kAcc];
+#pragma unroll
+    for (int i = 0; i < kAcc; ++i) acc[i] = f32x4{};
     bf16x8 wa[kWSteps];
 #pragma unroll
     for (int ks = 0; ks < kWPre; ++ks) wa[ks] = __builtin_bit_cast(bf16x8, wls[ks * 64 + lane]);
 #pragma unroll
     for (int ks = 0; ks < kWSteps; ++ks) {
       if (ks + kWPre < kWSteps) wa[ks + kWPre] = __builtin_bit_cast(bf16x8, wls[(ks + kWPre) * 64 + lane]);
-      acc = mfma16x16x32(wa[ks], __builtin_bit_cast(bf16x8, xf[ks]), acc);
+      acc[ks % kAcc] = mfma16x16x32(wa[ks], __builtin_bit_cast(bf16x8, xf[ks]), acc[ks % kAcc]);
       // The next chain's fragment ks (beyond the resource, i.e. no memory access, after the last chain).
       xf[ks] = __builtin_amdgcn_raw_buffer_load_b128(xr, more ? (int)(nb + 64u * ks) : (int)0xfffffff0u, 0, 0);
     }
@@ -597,10 +606,15 @@ __device__ __forceinline__ void w_role(const WProjParams& p, int wblk, uint8_t* 
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                            // MFMA
       __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                            // VMEM read
     }
+    f32x4 tot = acc[0];
+#pragma unroll
+    for (int i = 1; i < kAcc; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tot[r] = __fadd_rn(tot[r], acc[i][r]);
     // Lane (n = lane % 16, g = lane / 16) holds heads 4g .. 4g + 3 of token 16c + n.
     const uint32_t t = (uint32_t)c * kWTok + (uint32_t)(lane & 15);
     const uint32_t off = t < (uint32_t)p.M ? t * (uint32_t)(kWHeads * 2) + (uint32_t)(lane >> 4) * 8u : 0xfffffff0u;
-    __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf2(acc[0], acc[1]), pack_bf2(acc[2], acc[3])}, orr, (int)off,
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf2(tot[0], tot[1]), pack_bf2(tot[2], tot[3])}, orr, (int)off,
                                           0, 0);
   }
 }
@@ -617,17 +631,23 @@ struct Proj2Params {
 // the other way round the q role's first tile came ~5 us later). Each w-role block,
 // once its chains are done, computes the last tail16/16 of the q tiles of the run with
 // its own index (on the same XCD), so that both roles end together.
-template <int RD, int RM>
+// kSplitK (dsa_indexer_projections_splitk): both weights as their rows, wl in hipBLASLt's
+// split-k order. The rows are staged through LDS where the packed form loads straight into
+// registers, which costs 0.5 us (1000 tokens: 5.1 us) to 2 us (12,000 tokens: 18.4 us);
+// packing would make a write to the weights through .data stale at token counts where it
+// is not, and the first call on new weights slower. Fewer w-role workgroups of 4 chains
+// per wave group and more q ones: slower up to 4096 tokens (1000: 7.3 us).
+template <int RD, int RM, bool kSplitK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void ix_proj2_kernel(Proj2Params p) {
   extern __shared__ __align__(16) uint8_t smem[];
   const int b = blockIdx.x;
   if (b < p.nq) {
-    q_role<RD, RM, true>(p.q, b, smem, p.wtail ? 1 : 0);
+    q_role<RD, RM, !kSplitK>(p.q, b, smem, p.wtail ? 1 : 0);
   } else {
-    w_role(p.w, b - p.nq, smem);
+    w_role<kSplitK, !kSplitK>(p.w, b - p.nq, smem);
     if (p.wtail) {
       __syncthreads();  // the w role's LDS (W fragments) becomes the q role's ring
-      q_role<RD, RM, true>(p.q, b - p.nq, smem, 2);
+      q_role<RD, RM, !kSplitK>(p.q, b - p.nq, smem, 2);
     }
   }
 }
@@ -677,7 +697,7 @@ int launch_k256(const ProjParams& a, void* stream) {
 constexpr int kProj2QPerCu = 1;
 constexpr int kProj2Tail16 = 4;
 
-template <int RD, int RM>
+template <int RD, int RM, bool kSplitK>
 int launch_proj2(SProjParams q, WProjParams w, void* stream) {
   using C = SCfg<RD>;
   int cus = 0;
@@ -694,9 +714,95 @@ int launch_proj2(SProjParams q, WProjParams w, void* stream) {
   p.w = w;
   p.nq = (int32_t)qblocks;
   p.wtail = kProj2Tail16 > 0 ? 1 : 0;
-  void (*fn)(Proj2Params) = ix_proj2_kernel<RD, RM>;
+  void (*fn)(Proj2Params) = ix_proj2_kernel<RD, RM, kSplitK>;
   if (dsa_host::ensure_dyn_lds((const void*)fn, C::kLds) != DSA_OK) return DSA_ERR_LAUNCH;
   hipLaunchKernelGGL(fn, dim3((unsigned)(qblocks + wblocks)), dim3(256), (size_t)C::kLds, (hipStream_t)stream, p);
+  return hipGetLastError() == hipSuccess ? DSA_OK : DSA_ERR_LAUNCH;
+}
+
+// Up to 16 tokens: hipBLASLt splits k over 4 waves for both products here (depth blocks of
+// 128: chain c takes the c-th 32 k of every block in ascending k, the chains are added as
+// ((c0 + c1) + c2) + c3 and rounded once). A q workgroup covers 64 channels, 16 per wave,
+// each wave running its four chains of 2 products with all 16 loads in flight; the last
+// workgroup computes wl, one chain of 8 products per wave, the chains meeting in LDS.
+// Bound by the latency of one load and the launch: 3.2-3.6 us for 1..16 tokens, beside
+// 3.9 + 4.2 us for hipBLASLt's two kernels and ~20 us of host time for each F.linear.
+constexpr int kSmallTok = 16;
+
+template <int RD, int RM>
+__global__ __launch_bounds__(256) void ix_proj_small_kernel(Proj2Params p) {
+  __shared__ f32x4 red[4][64];
+  const int lane = threadIdx.x & 63, wi = threadIdx.x >> 6;
+  const int col = lane & 15, g = lane >> 4;  // token (B column) / W row, k slice 8g .. 8g + 7
+  const int M = p.q.M, tok = min(col, M - 1);  // columns >= M compute on a valid row and are not stored
+  const bool is_q = (int)blockIdx.x < p.nq;
+  const int n0 = 64 * (int)blockIdx.x + 16 * wi;  // q: first of the wave's 16 channels
+  // 8 steps of 32 k: q, steps 0..7 of k 256 (chain s % 4); wl, steps wi + 4 s of k 1024.
+  const int K = is_q ? kSK : kWDim, k0 = 8 * g + (is_q ? 0 : 32 * wi), ks = is_q ? 32 : 128;
+  const uint16_t* wrow = (is_q ? p.q.w + (int64_t)(n0 + col) * K : reinterpret_cast<const uint16_t*>(p.w.wp) + col * K) + k0;
+  const uint16_t* xrow = (is_q ? p.q.x : p.w.x) + (int64_t)tok * K + k0;
+  bf16x8 a[8], b[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    a[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(wrow + s * ks));
+    b[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(xrow + s * ks));
+  }
+  float4 cs = float4{1.f, 0.f, 1.f, 0.f};
+  const int hd = n0 / 64, pj = (n0 % 64 - (64 - RD) + 4 * g) >> 1;  // head dim 64; complex index of the first pair
+  const bool rot = RD > 0 && is_q && n0 % 64 >= 64 - RD;
+  if constexpr (RD > 0) {
+    if (rot) cs = *reinterpret_cast<const float4*>(p.q.freqs + ((int64_t)(tok % p.q.S) * (RD / 2) + pj) * 2);
+  }
+  __builtin_amdgcn_sched_barrier(0);  // every load in flight before the first product
+  if (!is_q) {
+    f32x4 acc = f32x4{};
+#pragma unroll
+    for (int s = 0; s < 8; ++s) acc = mfma16x16x32(a[s], b[s], acc);
+    red[wi][lane] = acc;
+    __syncthreads();
+    if (wi == 0 && col < M) {
+      f32x4 t = red[0][lane];
+#pragma unroll
+      for (int c = 1; c < 4; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t[r] = __fadd_rn(t[r], red[c][lane][r]);
+      *reinterpret_cast<u32x2*>(p.w.wl + col * kWHeads + 4 * g) = u32x2{pack_bf2(t[0], t[1]), pack_bf2(t[2], t[3])};
+    }
+    return;
+  }
+  f32x4 acc[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) acc[c] = mfma16x16x32(a[c], b[c], f32x4{});
+#pragma unroll
+  for (int c = 0; c < 4; ++c) acc[c] = mfma16x16x32(a[c + 4], b[c + 4], acc[c]);
+  f32x4 t = acc[0];
+#pragma unroll
+  for (int c = 1; c < 4; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t[r] = __fadd_rn(t[r], acc[c][r]);
+  // Lane (col, g): channels n0 + 4g .. + 3 of token col.
+  u32x2 u = {pack_bf2(t[0], t[1]), pack_bf2(t[2], t[3])};
+  if constexpr (RD > 0) {
+    if (rot) {
+      const uint32_t nb = ((uint32_t)tok * (uint32_t)p.q.H + (uint32_t)hd) * (uint32_t)(RD / 2) + (uint32_t)pj;
+      float re, im;
+      rope_pair_sel<RM>(bf_lo(u[0]), bf_hi(u[0]), cs.x, cs.y, nb, re, im);
+      u[0] = pack_bf2(re, im);
+      rope_pair_sel<RM>(bf_lo(u[1]), bf_hi(u[1]), cs.z, cs.w, nb + 1, re, im);
+      u[1] = pack_bf2(re, im);
+    }
+  }
+  if (col < M) *reinterpret_cast<u32x2*>(p.q.q + (int64_t)col * p.q.N + n0 + 4 * g) = u;
+}
+
+template <int RD, int RM>
+int launch_small(const SProjParams& q, const WProjParams& w, void* stream) {
+  Proj2Params p;
+  p.q = q;
+  p.w = w;
+  p.nq = q.N / 64;
+  p.wtail = 0;
+  hipLaunchKernelGGL((ix_proj_small_kernel<RD, RM>), dim3((unsigned)p.nq + 1), dim3(256), 0, (hipStream_t)stream, p);
   return hipGetLastError() == hipSuccess ? DSA_OK : DSA_ERR_LAUNCH;
 }
 
@@ -800,10 +906,13 @@ extern "C" int dsa_indexer_pack_projection_weights(const void* wq, int64_t n, in
   return hipGetLastError() == hipSuccess ? DSA_OK : DSA_ERR_LAUNCH;
 }
 
-extern "C" int dsa_indexer_projections(const void* qr, const void* wq_packed, const void* freqs_cis,
-                                       int32_t rope_mode, void* q, const void* x, const void* wproj_packed,
-                                       void* wl, int64_t m, int64_t n, int64_t k, int64_t dim, int64_t n_w,
-                                       int64_t head_dim, int64_t rd, int64_t s_len, void* stream) {
+namespace {
+
+// Both projection entry points (the weights packed, or as their rows).
+int projections(const void* qr, const void* wq, const void* freqs_cis, int32_t rope_mode, void* q,
+                const void* x, const void* wproj, void* wl, int64_t m, int64_t n, int64_t k,
+                int64_t dim, int64_t n_w, int64_t head_dim, int64_t rd, int64_t s_len, bool splitk,
+                void* stream) {
   if (m < 0 || n <= 0 || k <= 0 || dim <= 0 || n_w <= 0 || head_dim <= 0 || s_len <= 0) return DSA_ERR_SHAPE;
   if (n % head_dim != 0 || m % s_len != 0) return DSA_ERR_SHAPE;
   if (k != kSK || n % kSCh != 0 || head_dim != 64 || dim != kWDim || n_w != kWHeads)
@@ -818,14 +927,14 @@ extern "C" int dsa_indexer_projections(const void* qr, const void* wq_packed, co
   if (m > INT32_MAX / 2 || m * n > (int64_t)UINT32_MAX / 2 || m * dim * 2 > (int64_t)UINT32_MAX - 2 * kWChainBytes)
     return DSA_ERR_UNSUPPORTED;
   if (m == 0) return DSA_OK;
-  if (!qr || !wq_packed || !q || !x || !wproj_packed || !wl) return DSA_ERR_NULL;
-  if (!dsa_host::aligned16(qr) || !dsa_host::aligned16(wq_packed) || !dsa_host::aligned16(q) ||
-      !dsa_host::aligned16(x) || !dsa_host::aligned16(wproj_packed) || ((uintptr_t)wl & 7u) ||
+  if (!qr || !wq || !q || !x || !wproj || !wl) return DSA_ERR_NULL;
+  if (!dsa_host::aligned16(qr) || !dsa_host::aligned16(wq) || !dsa_host::aligned16(q) ||
+      !dsa_host::aligned16(x) || !dsa_host::aligned16(wproj) || ((uintptr_t)wl & 7u) ||
       (freqs_cis != nullptr && ((uintptr_t)freqs_cis & 15u)))
     return DSA_ERR_ALIGN;
   SProjParams qp;
   qp.x = (const uint16_t*)qr;
-  qp.w = (const uint16_t*)wq_packed;
+  qp.w = (const uint16_t*)wq;
   qp.q = (uint16_t*)q;
   qp.freqs = (const float*)freqs_cis;
   qp.M = (int32_t)m;
@@ -836,11 +945,41 @@ extern "C" int dsa_indexer_projections(const void* qr, const void* wq_packed, co
   qp.tail16 = 0;
   WProjParams wp;
   wp.x = (const uint16_t*)x;
-  wp.wp = (const u32x4*)wproj_packed;
+  wp.wp = (const u32x4*)wproj;
   wp.wl = (uint16_t*)wl;
   wp.M = (int32_t)m;
   wp.nwaves = 0;
-  if (freqs_cis == nullptr) return launch_proj2<0, 0>(qp, wp, stream);
-  return rope_mode == DSA_ROPE_CPU ? launch_proj2<32, DSA_ROPE_CPU>(qp, wp, stream)
-                                   : launch_proj2<32, DSA_ROPE_TORCH_ROCM>(qp, wp, stream);
+  const bool cpu = rope_mode == DSA_ROPE_CPU;
+  if (splitk && m <= kSmallTok) {
+    if (freqs_cis == nullptr) return launch_small<0, 0>(qp, wp, stream);
+    return cpu ? launch_small<32, DSA_ROPE_CPU>(qp, wp, stream)
+               : launch_small<32, DSA_ROPE_TORCH_ROCM>(qp, wp, stream);
+  }
+  if (splitk) {
+    if (freqs_cis == nullptr) return launch_proj2<0, 0, true>(qp, wp, stream);
+    return cpu ? launch_proj2<32, DSA_ROPE_CPU, true>(qp, wp, stream)
+               : launch_proj2<32, DSA_ROPE_TORCH_ROCM, true>(qp, wp, stream);
+  }
+  if (freqs_cis == nullptr) return launch_proj2<0, 0, false>(qp, wp, stream);
+  return cpu ? launch_proj2<32, DSA_ROPE_CPU, false>(qp, wp, stream)
+             : launch_proj2<32, DSA_ROPE_TORCH_ROCM, false>(qp, wp, stream);
+}
+
+}  // namespace
+
+extern "C" int dsa_indexer_projections(const void* qr, const void* wq_packed, const void* freqs_cis,
+                                       int32_t rope_mode, void* q, const void* x, const void* wproj_packed,
+                                       void* wl, int64_t m, int64_t n, int64_t k, int64_t dim, int64_t n_w,
+                                       int64_t head_dim, int64_t rd, int64_t s_len, void* stream) {
+  return projections(qr, wq_packed, freqs_cis, rope_mode, q, x, wproj_packed, wl, m, n, k, dim, n_w, head_dim,
+                     rd, s_len, false, stream);
+}
+
+extern "C" int dsa_indexer_projections_splitk(const void* qr, const void* wq, const void* freqs_cis,
+                                              int32_t rope_mode, void* q, const void* x, const void* wproj,
+                                              void* wl, int64_t m, int64_t n, int64_t k, int64_t dim,
+                                              int64_t n_w, int64_t head_dim, int64_t rd, int64_t s_len,
+                                              void* stream) {
+  return projections(qr, wq, freqs_cis, rope_mode, q, x, wproj, wl, m, n, k, dim, n_w, head_dim, rd, s_len,
+                     true, stream);
 }

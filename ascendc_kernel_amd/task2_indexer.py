@@ -10,13 +10,14 @@ so a seeded construction yields the reference's weights.
 
 forward = the two projections, then one gfx950 kernel for the score, the
 relu-weighted head sum, the causal mask and the top-k (``dsa_indexer_score_topk``).
-The projections run as one kernel launch (``dsa_indexer_projections``: q with RoPE,
-and the head weights), as the query-projection kernel beside ``F.linear``, as one
-decode launch for 1..16 tokens (``dsa_indexer_decode_projections``, both products in
-hipBLASLt's split-k order; the score kernel applies RoPE), or as two ``F.linear`` (the
-reference's own op; the score kernel then applies RoPE), whichever ``projection_route``
-picks: a kernel only where its rounding was measured equal to ``F.linear`` on this
-torch-ROCm build. Inputs must be on the HIP device;
+The projections run as one kernel launch (``dsa_indexer_projections`` or, in the order
+of hipBLASLt's split k, ``dsa_indexer_projections_splitk``: q with RoPE, and the head
+weights), as the query-projection kernel beside ``F.linear``, as one decode launch for
+1..16 tokens (``dsa_indexer_decode_projections``, both products in hipBLASLt's split-k
+order; the score kernel applies RoPE), or as two ``F.linear`` (the reference's own op; the
+score kernel then applies RoPE), whichever ``splitk_route`` and ``projection_route`` pick:
+a kernel only where its rounding was measured equal to ``F.linear`` on this torch-ROCm
+build. Inputs must be on the HIP device;
 unsupported configurations raise.
 """
 from __future__ import annotations
@@ -155,6 +156,13 @@ Q_PROJ_MIN_TOKENS = 64
 DECODE_MAX_TOKENS = 16
 DECODE_SHAPE = (1536, 8192, 7168, 64)
 
+#: Token counts up to which torch-ROCm's F.linear of the 16-head shapes (wq_b 256 -> 1024,
+#: weights_proj 1024 -> 16) sums k as dsa_indexer_projections_splitk does, apart from the
+#: counts of WL_EQUAL: hipBLASLt splits weights_proj's k over 4 waves up to here and wq_b's
+#: up to 16 tokens (measured for every count by tests/golden/measure_projection_ranges.py).
+SPLITK_MAX_TOKENS = 16384
+SPLITK_SHAPE = (256, 1024, 1024, 16)
+
 _build_ok: dict = {}
 
 
@@ -193,6 +201,16 @@ def projection_route(m: int, q_lora_rank: int, rope_head_dim: int, head_dim: int
     return "q"
 
 
+def splitk_route(m: int, q_lora_rank: int, rope_head_dim: int, head_dim: int, n_q: int, dim: int,
+                 n_w: int, bf16: bool, on_gpu: bool, build_ok: bool) -> bool:
+    """Whether one launch of dsa_indexer_projections_splitk (q with RoPE, and weights_proj)
+    gives F.linear's bits for m = b * s tokens: the 16-head shapes on the measured build, where
+    weights_proj's k is split and wq_b's is either split (up to 16 tokens) or in natural order."""
+    return (bf16 and on_gpu and build_ok and 1 <= m <= SPLITK_MAX_TOKENS
+            and (q_lora_rank, n_q, dim, n_w) == SPLITK_SHAPE and rope_head_dim == 32 and head_dim == 64
+            and (m <= 16 or _within(m, Q_EQUAL)) and not _within(m, WL_EQUAL))
+
+
 class Model(nn.Module):
     """Drop-in for ``Model`` of reference/task2_v0_ref.py:106-144."""
 
@@ -223,12 +241,17 @@ class Model(nn.Module):
         self._packed = None
 
     def route(self, x: torch.Tensor, qr: torch.Tensor) -> str:
-        """projection_route for these inputs ('both', 'q', 'decode' or 'torch')."""
+        """The projections' path for these inputs: 'splitk' (splitk_route), else what
+        projection_route picks ('both', 'q', 'decode' or 'torch')."""
         wq, wp = self.wq_b.weight, self.weights_proj.weight
-        return projection_route(
-            qr.shape[0] * qr.shape[1], qr.shape[-1], self.rope_head_dim, self.head_dim, wq.shape[0], x.shape[-1],
-            wp.shape[0], qr.dtype == x.dtype == wq.dtype == wp.dtype == torch.bfloat16,
-            qr.is_cuda and x.is_cuda, qr.is_cuda and _measured_build(qr.device))
+        args = (qr.shape[0] * qr.shape[1], qr.shape[-1], self.rope_head_dim, self.head_dim, wq.shape[0],
+                x.shape[-1], wp.shape[0], qr.dtype == x.dtype == wq.dtype == wp.dtype == torch.bfloat16,
+                qr.is_cuda and x.is_cuda, qr.is_cuda and _measured_build(qr.device))
+        if splitk_route(*args):
+            # (F.linear takes any alignment, the kernel 16 bytes; a copy made contiguous is aligned.)
+            if all(t.data_ptr() % 16 == 0 or not t.is_contiguous() for t in (x, qr, wq, wp, self.freqs_cis)):
+                return "splitk"
+        return projection_route(*args)
 
     def forward(self, x: torch.Tensor, qr: torch.Tensor, start_pos: int, offset: int) -> torch.Tensor:
         # Steady state (the Ascend ModelNew binds a no-argument launch of the whole forward
@@ -266,20 +289,11 @@ class Model(nn.Module):
         self._packed = None
         self._plan = None
 
-    def _q_proj_fused(self, qr: torch.Tensor) -> bool:
-        """Whether q comes from a projection kernel (dsa_indexer_q_proj or
-        dsa_indexer_projections) rather than F.linear + RoPE in the score kernel."""
-        wq, wp = self.wq_b.weight, self.weights_proj.weight
-        return projection_route(
-            qr.shape[0] * qr.shape[1], qr.shape[-1], self.rope_head_dim, self.head_dim, wq.shape[0], self.dim,
-            wp.shape[0], qr.dtype == wq.dtype == torch.bfloat16, qr.is_cuda,
-            qr.is_cuda and _measured_build(qr.device)) in ("both", "q")
-
 
 class _IndexerPlan:
     """Everything Model.forward launches for one set of inputs, prepared once. Intermediate q
-    and wl buffers of the kernel paths are kept and reused by later calls of the plan: the
-    plan is keyed on the stream, and on one stream a call's projections start only after
+    and wl buffers of the 'both', 'decode' and 'q' paths are kept and reused by later calls of
+    the plan: the plan is keyed on the stream, and on one stream a call's projections start only after
     the previous call's score kernel has read them."""
 
     def __init__(self, model: Model, x: torch.Tensor, qr: torch.Tensor, start_pos: int, offset: int, key):
@@ -303,17 +317,25 @@ class _IndexerPlan:
         score_kw = dict(rope_head_dim=rd, n_cand=n_cand, k_out=k_out, ratio=ratio, causal=start_pos == 0,
                         offset=offset, rope_mode=mode)
         self.proj = None
-        if self.route == "both":
+        if self.route == "both" or self.route == "splitk":
             # q = RoPE(qr . wq_b^T) and wl = x . weights_proj^T in one launch
-            # (task2_v0_ref.py:129-132), bit-equal to F.linear + apply_rotary_emb here.
-            wq_p, wp_p = model.packed_weights()
+            # (task2_v0_ref.py:129-132), bit-equal to F.linear + apply_rotary_emb here: 'both'
+            # in ascending k from packed weights, 'splitk' in hipBLASLt's split order from the
+            # weights in place.
+            splitk = self.route == "splitk"
+            wq_k, wp_k = (self.wq, self.wp) if splitk else model.packed_weights()
             self.proj, q_shape, wl_shape, self.proj_keep = _native.prepare_indexer_projections(
-                qr, wq_p, freqs, x, wp_p, hd, rd, mode)
-            self.q = torch.empty(q_shape, dtype=torch.bfloat16, device=x.device)
-            self.wl = torch.empty(wl_shape, dtype=torch.bfloat16, device=x.device)
-            self.proj.set(_native.PROJ_SLOT_Q, self.q.data_ptr())
-            self.proj.set(_native.PROJ_SLOT_WL, self.wl.data_ptr())
-            self.score = _native.prepare_indexer_score_topk(self.q, kv, self.wl, w_scale, None, **score_kw)
+                qr, wq_k, freqs, x, wp_k, hd, rd, mode, splitk)
+            q = torch.empty(q_shape, dtype=torch.bfloat16, device=x.device)
+            wl = torch.empty(wl_shape, dtype=torch.bfloat16, device=x.device)
+            self.score = _native.prepare_indexer_score_topk(q, kv, wl, w_scale, None, **score_kw)
+            if splitk:  # q and wl of a call: one fresh buffer, wl after q (whole 2 KB rows)
+                self.q_bytes = 2 * q.numel()
+                self.qwl_words = q.numel() + wl.numel()
+            else:
+                self.q, self.wl = q, wl
+                self.proj.set(_native.PROJ_SLOT_Q, q.data_ptr())
+                self.proj.set(_native.PROJ_SLOT_WL, wl.data_ptr())
         elif self.route == "decode":
             # q = qr . wq_b^T and wl = x . weights_proj^T in one launch, in hipBLASLt's
             # rounding at decode sizes (task2_v0_ref.py:129,132); RoPE in the score kernel.
@@ -343,7 +365,16 @@ class _IndexerPlan:
         if self.empty is not None:
             return torch.empty(*self.empty, 0, dtype=torch.int64, device=self.device)
         launch = self.score.launch
-        if self.route == "both" or self.route == "decode":
+        if self.route == "splitk":
+            qwl = self.x.new_empty(self.qwl_words)
+            q_ptr = qwl.data_ptr()
+            wl_ptr = q_ptr + self.q_bytes
+            self.proj.set(_native.PROJ_SLOT_Q, q_ptr)
+            self.proj.set(_native.PROJ_SLOT_WL, wl_ptr)
+            self.proj()
+            launch.set(_native.SCORE_SLOT_Q, q_ptr)
+            launch.set(_native.SCORE_SLOT_WL, wl_ptr)
+        elif self.route == "both" or self.route == "decode":
             self.proj()
         elif self.route == "q":
             self.proj()
@@ -354,7 +385,7 @@ class _IndexerPlan:
             wl = F.linear(self.x, self.wp)
             launch.set(_native.SCORE_SLOT_Q, q.data_ptr())
             launch.set(_native.SCORE_SLOT_WL, wl.data_ptr())
-        # (The fresh q / wl tensors of the torch paths are released when this returns; the
+        # (The fresh q / wl tensors of the splitk and torch paths are released when this returns; the
         # caching allocator hands their memory only to later work on this stream.)
         return self.score.run()
 

@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define DSA_ABI_VERSION 4
+#define DSA_ABI_VERSION 5
 
 #define DSA_OK 0
 #define DSA_ERR_NULL (-1)        /* a required pointer is NULL */
@@ -334,6 +334,21 @@ int dsa_indexer_projections(const void* qr, const void* wq_packed, const void* f
                             int32_t rope_mode, void* q, const void* x, const void* wproj_packed,
                             void* wl, int64_t m, int64_t n, int64_t k, int64_t dim, int64_t n_w,
                             int64_t head_dim, int64_t rd, int64_t s_len, void* stream);
+
+/*
+ * dsa_indexer_projections (reference/task2_v0_ref.py:129-132) in the k order of hipBLASLt's
+ * local split: in depth blocks of 128, chain c of 4 accumulates the c-th 32 k of every block
+ * in ascending k in fp32, the chains are added as ((c0 + c1) + c2) + c3 and rounded once to
+ * bf16. wl takes that order at every m, q for m <= 16 (ascending k above), which is how
+ * torch-ROCm's F.linear sums these shapes below about 16,384 tokens (the drop-in Model calls
+ * this entry point only at token counts where that was measured). Arguments and requirements
+ * are those of dsa_indexer_projections, except that the weights are the Linear weights as
+ * they are: wq bf16 [n, k], wproj bf16 [n_w, dim].
+ */
+int dsa_indexer_projections_splitk(const void* qr, const void* wq, const void* freqs_cis,
+                                   int32_t rope_mode, void* q, const void* x, const void* wproj,
+                                   void* wl, int64_t m, int64_t n, int64_t k, int64_t dim, int64_t n_w,
+                                   int64_t head_dim, int64_t rd, int64_t s_len, void* stream);
 
 /*
  * The indexer's two projections for a few tokens (decode), in one launch, without RoPE

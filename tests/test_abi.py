@@ -283,6 +283,15 @@ def test_projections_host_checks():
     assert _proj(lib, m=2 ** 21, s=2 ** 21) == -3   # 32-bit buffer offsets
 
 
+def test_splitk_projections_host_checks():
+    """dsa_indexer_projections_splitk refuses what dsa_indexer_projections does."""
+    lib = _native.load()
+    f = lambda m=16, qr=16, wq=16, n=1024, k=256, s=16, wl=16: lib.dsa_indexer_projections_splitk(
+        qr, wq, 16, 1, 16, 16, 16, wl, m, n, k, 1024, 16, 64, 32, s, None)
+    assert f(m=-1) == f(m=17) == f(n=1000) == -2 and f(k=512) == -3 and f(m=0) == 0
+    assert f(qr=None) == f(wl=None) == -1 and f(qr=8) == f(wq=2) == f(wl=4) == -6
+
+
 def test_pack_projection_weights_host_checks():
     lib = _native.load()
     f = lib.dsa_indexer_pack_projection_weights

@@ -195,3 +195,87 @@ def test_q_proj_more_token_counts(gpu, b, m):
     w, qr, fr, ref, ref_rope = _case(k, n, d, rd, b, m, 11 + m, gpu)
     got = _native.indexer_q_proj(qr, w, fr, d, rd)
     assert _ne(got, ref_rope) == 0
+
+
+# ---------------------------------------------------------------- hipBLASLt's split-k order
+def _planted(m, n, k, g, dev):
+    """x [m, k], w [n, k] whose products come in cancelling pairs of powers of two at positions
+    all rows share, the rest ~ N(0, 1): the sums are small beside their parts, so that a sum
+    taken in another order shows in several percent of the rounded outputs."""
+    perm = torch.randperm(k, generator=g, device=dev)
+    npair = int(k * 0.9) // 2
+    a, b = perm[:npair], perm[npair:2 * npair]
+
+    def powers(rows):
+        s = torch.where(torch.rand(rows, npair, generator=g, device=dev) < 0.5, -1.0, 1.0)
+        return s * torch.exp2(torch.randint(0, 8, (rows, npair), generator=g, device=dev).float())
+
+    x, w = torch.randn(m, k, generator=g, device=dev), torch.randn(n, k, generator=g, device=dev)
+    x[:, a], w[:, a] = powers(m), powers(n)
+    x[:, b], w[:, b] = x[:, a], -w[:, a]
+    return x.to(torch.bfloat16), w.to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("b,s", [(1, 1), (3, 5), (2, 8), (1, 17), (1, 31), (4, 8), (1, 33), (3, 1003), (1, 5000),
+                                 (1, 15360), (1, 15518), (2, 8192)])
+def test_splitk_projections_equal_f_linear(gpu, b, s):
+    """dsa_indexer_projections_splitk at the edges of its forms (16 / 17 tokens, 32-token tiles)
+    on order-sensitive inputs: F.linear's bits, with RoPE in both roundings and without."""
+    from ascendc_kernel_amd import task2_indexer as t2
+    if not t2._measured_build(gpu):
+        pytest.skip("hipBLASLt's summation order was measured on one build only")
+    g = torch.Generator(device=gpu).manual_seed(b * s)
+    m = b * s
+    qr, wq = _planted(m, 1024, 256, g, gpu)
+    x, wp = _planted(m, 16, 1024, g, gpu)
+    qr, x = qr.view(b, s, 256), x.view(b, s, 1024)
+    fr = oix.precompute_freqs_cis(32, s, device=gpu)
+    _say("splitk", b, s)
+    ref = torch.nn.functional.linear(qr, wq).unflatten(-1, (16, 64))
+    q, wl = _native.indexer_projections(qr, wq, None, x, wp, 64, 32, splitk=True)
+    assert _ne(q, ref) == 0 and _ne(wl, torch.nn.functional.linear(x, wp)) == 0
+    qc, wl = _native.indexer_projections(qr, wq, fr, x, wp, 64, 32, _native.DSA_ROPE_CPU, splitk=True)
+    f = torch.view_as_real(fr).reshape(s, 16, 2).cpu().numpy()
+    assert int((bits_of(qc) != rules.rope_bf16(bits_of(ref), f, 32, "cpu")).sum()) == 0
+    oix.apply_rotary_emb(ref[..., -32:], fr)
+    q, wl = _native.indexer_projections(qr, wq, fr, x, wp, 64, 32, splitk=True)
+    assert _ne(q, ref) == 0 and _ne(wl, torch.nn.functional.linear(x, wp)) == 0
+
+
+@pytest.mark.parametrize("b,s,start", [(8, 1, 2599), (2, 3, 640), (1, 50, 0), (3, 101, 0)])
+def test_model_splitk_route(gpu, b, s, start):
+    """Model.forward on the split-k launch gives the F.linear path's picks: with every input
+    aligned, with x and qr at addresses that F.linear takes and the launch does not, and captured
+    in a graph whose replays mix with eager calls."""
+    from ascendc_kernel_amd import task2_indexer as t2
+    if not t2._measured_build(gpu):
+        pytest.skip("hipBLASLt's summation order was measured on one build only")
+    g = torch.Generator().manual_seed(31 + s)
+    args = t2._make_args()
+    kv = torch.randn(8, 650, 64, generator=g).to(torch.bfloat16).to(gpu)
+    model = t2.Model(args, t2.precompute_freqs_cis(32, 2600, device=gpu), kv, 4).to(gpu).requires_grad_(False)
+    buf = torch.randn(2 * b * s * 1024, generator=g).to(torch.bfloat16).to(gpu)
+    x, xu = buf[: b * s * 1024].view(b, s, 1024), buf[1: 1 + b * s * 1024].view(b, s, 1024)
+    qr, qru = buf[: b * s * 256].view(b, s, 256), buf[3: 3 + b * s * 256].view(b, s, 256)
+    assert model.route(x, qr) == "splitk" and model.route(xu, qru) != "splitk"
+    _say("splitk model", b, s, start)
+
+    def want(xx, qq):
+        q = torch.nn.functional.linear(qq, model.wq_b.weight).unflatten(-1, (16, 64))
+        wl = torch.nn.functional.linear(xx, model.weights_proj.weight)
+        n = (start + s) // 4
+        return _native.indexer_score_topk(q, kv, wl, 64 ** -0.5 * 16 ** -0.5, model.freqs_cis[start:start + s], 32, n,
+                                          min(128, n), 4, start == 0, 0)
+
+    ref = want(x, qr)
+    assert torch.equal(model(x, qr, start, 0), ref)
+    if b * s < t2.Q_PROJ_MIN_TOKENS:  # (from there on the query kernel refused unaligned qr before, too)
+        assert torch.equal(model(xu, qru, start, 0), want(xu, qru))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = model(x, qr, start, 0)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, ref) and torch.equal(model(x, qr, start, 0), ref)
+        got.zero_()

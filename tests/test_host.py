@@ -158,6 +158,25 @@ def test_projection_tables_match_measurement():
             assert not t2._within(a - 1, table) and not t2._within(b + 1, table)
 
 
+def test_splitk_route_matches_measurement():
+    """The split-k launch serves exactly the token counts 1 .. 16,384 where both of its outputs
+    were measured equal to F.linear (projection_ranges.json), the 16-head shapes only."""
+    import json
+    import os
+    from conftest import GOLDEN
+    with open(os.path.join(GOLDEN, "projection_ranges.json")) as f:
+        r = json.load(f)
+    c3 = dict(q_lora_rank=256, rope_head_dim=32, head_dim=64, n_q=1024, dim=1024, n_w=16, bf16=True,
+              on_gpu=True, build_ok=True)
+    equal = [tuple(v) for v in r["splitk_equal"]]
+    assert r["splitk_mmax"] == t2.SPLITK_MAX_TOKENS
+    for m in range(0, t2.SPLITK_MAX_TOKENS + 2):
+        assert t2.splitk_route(m, **c3) == t2._within(m, equal), m
+    for other in (dict(q_lora_rank=1536), dict(rope_head_dim=64), dict(head_dim=128), dict(n_q=2048), dict(dim=2048),
+                  dict(n_w=32), dict(bf16=False), dict(on_gpu=False), dict(build_ok=False)):
+        assert not t2.splitk_route(8, **{**c3, **other})
+
+
 # ---------------------------------------------------------------- steady-state launch plans
 class _FakePrepared:
     """Stands in for _native.Prepared, which holds its inputs (`keep`) so that their memory
