@@ -24,7 +24,8 @@
 // finds the k-th key, ties are taken in index order with ballots, and the k
 // winners are bitonic-sorted on a (key, ~index) composite before the int64
 // indices are written. Waves take token pairs from the end of the sequence
-// first, so the longest causal rows start first.
+// first, so the longest causal rows start first. With few token pairs several waves share
+// one pair's candidates instead (ix_score_topk_few_kernel, chosen by few_waves).
 #include "dsa_common.h"
 
 #include <atomic>
@@ -122,12 +123,16 @@ __device__ __forceinline__ int find_bin(const uint32_t* hist, int lane, uint32_t
   uint32_t local = 0;
 #pragma unroll
   for (int i = 0; i < 8; ++i) local += bins[i];
+  // Suffix sum over the half: DPP row shifts within each row of 16 lanes (lanes past the
+  // row add 0), then the upper row's total for the lower row (no LDS round trips).
   uint32_t incl = local;
-#pragma unroll
-  for (int off = 1; off < 32; off <<= 1) {
-    const uint32_t o = __shfl(incl, (lane + off) & 63, 64);
-    if (hl + off < 32) incl += o;
-  }
+  incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x101, 0xf, 0xf, false);  // row_shl:1
+  incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x102, 0xf, 0xf, false);
+  incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x104, 0xf, 0xf, false);
+  incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x108, 0xf, 0xf, false);
+  const uint32_t up0 = (uint32_t)__builtin_amdgcn_readlane((int)incl, 16);
+  const uint32_t up1 = (uint32_t)__builtin_amdgcn_readlane((int)incl, 48);
+  if (hl < 16) incl += half ? up1 : up0;
   uint32_t cum = incl - local;
   int fb = -1;
   uint32_t fgt = 0;
@@ -140,11 +145,206 @@ __device__ __forceinline__ int find_bin(const uint32_t* hist, int lane, uint32_t
     }
     cum = nc;
   }
-  const uint32_t hm = (uint32_t)(__ballot(fb >= 0) >> (32 * half));
-  const int src = hm ? (int)(__builtin_ctz(hm)) + 32 * half : lane;
-  const int b = __shfl(fb, src, 64);
-  gt = __shfl(fgt, src, 64);
-  return hm ? b : -1;
+  // At most one lane of each half holds the bin; without one the half's answer is -1.
+  const uint64_t found = __ballot(fb >= 0);
+  const int src0 = __builtin_ctz((uint32_t)found | 0x80000000u);
+  const int src1 = 32 + __builtin_ctz((uint32_t)(found >> 32) | 0x80000000u);
+  const int bin0 = __builtin_amdgcn_readlane(fb, src0), bin1 = __builtin_amdgcn_readlane(fb, src1);
+  const uint32_t gt0 = (uint32_t)__builtin_amdgcn_readlane((int)fgt, src0);
+  const uint32_t gt1 = (uint32_t)__builtin_amdgcn_readlane((int)fgt, src1);
+  gt = half ? gt1 : gt0;
+  return half ? bin1 : bin0;
+}
+
+// Head weights of token t, bf16(fp32(wl) * w_scale), as fp32 values (0 for t >= S).
+__device__ __forceinline__ void load_head_weights(const IxParams& p, int b, int t, float (&w)[kH]) {
+  if (t < p.S) {
+    const u32x4* wp = reinterpret_cast<const u32x4*>(p.wl + ((int64_t)b * p.S + t) * kH);
+    const u32x4 w0 = wp[0], w1 = wp[1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      w[2 * i] = bf2f(f2bf(bf_lo(w0[i]) * p.wscale));
+      w[2 * i + 1] = bf2f(f2bf(bf_hi(w0[i]) * p.wscale));
+      w[8 + 2 * i] = bf2f(f2bf(bf_lo(w1[i]) * p.wscale));
+      w[8 + 2 * i + 1] = bf2f(f2bf(bf_hi(w1[i]) * p.wscale));
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < kH; ++i) w[i] = 0.f;
+  }
+}
+
+// A operand: row i = lane % 32 is token t0 + (i/4)%2, head i%4 + 4(i/8); lane
+// holds channels 16ks + 8(lane/32) .. +7 of that row, RoPE applied when asked.
+// The 32x32 product leaves rows 8(r/4) + 4(lane/32) + r%4 in accumulator r of a
+// lane, so with this row order accumulator r of lanes 0..31 is head r of token t0
+// and of lanes 32..63 head r of token t0 + 1, for candidate lane % 32: every lane
+// holds all 16 heads of one (token, candidate) without an exchange of halves.
+__device__ __forceinline__ void load_q_rows(const IxParams& p, int b, int t0, int lane, bf16x8 (&qa)[4]) {
+  const int tq = t0 + ((lane >> 2) & 1);
+  const int hq = (lane & 3) | (((lane & 31) >> 3) << 2);
+  const int hsel = lane >> 5;
+  if (tq < p.S) {
+    const int64_t row = ((int64_t)b * p.S + tq) * kH + hq;
+    const uint16_t* src = p.q + row * kD;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      u32x4 v = *reinterpret_cast<const u32x4*>(src + 16 * ks + 8 * hsel);
+      if (p.freqs != nullptr) {
+        const int half_rd = p.rd >> 1;
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const int dch = 16 * ks + 8 * hsel + 2 * jj;
+          const int pj = (dch - (kD - p.rd)) >> 1;
+          if (dch >= kD - p.rd) {
+            const float c = p.freqs[((int64_t)tq * half_rd + pj) * 2];
+            const float d = p.freqs[((int64_t)tq * half_rd + pj) * 2 + 1];
+            const int64_t n = row * half_rd + pj;
+            float re, im;
+            rope_pair(bf_lo(v[jj]), bf_hi(v[jj]), c, d, p.rope_mode, n, re, im);
+            v[jj] = pack_bf2(re, im);
+          }
+        }
+      }
+      qa[ks] = __builtin_bit_cast(bf16x8, v);
+    }
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qa[ks] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+  }
+}
+
+// The rounding chain of one (token, candidate) over its 16 raw head scores (acc) and head
+// weights: the fp32 head sum that the score is rounded from.
+__device__ __forceinline__ float head_total(const f32x16& acc, const float (&w)[kH]) {
+  // The einsum's bf16 rounding, then relu on the bf16 bit patterns (both heads
+  // of a word at once): word k holds heads 2k, 2k+1.
+  uint32_t pk[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    s16v2 h = __builtin_bit_cast(s16v2, pack_bf2(acc[2 * k], acc[2 * k + 1]));
+    pk[k] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(h, (s16v2){0, 0}));
+  }
+  // * w -> bf16 (the products are exact in fp32), as fp32 values: one
+  // v_cvt_pk_bf16_f32 with a zero low operand leaves bf16(x) in the high half and
+  // zeros below it, which is bf16(x) as an fp32 value.
+  float v[16];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    v[2 * k] = bf16_as_f32(bf_lo(pk[k]) * w[2 * k]);
+    v[2 * k + 1] = bf16_as_f32(bf_hi(pk[k]) * w[2 * k + 1]);
+  }
+  // IEEE fp32 adds in torch's order (accumulator j sums heads j, j+4, j+8, j+12).
+  // torch's four accumulators start at +0; adding the +0 once to the total instead
+  // gives the same value (x + 0 == x except for the sign of a zero, and a -0 can
+  // only reach the total when every term is -0).
+  float a4[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) a4[j] = ((v[j] + v[j + 4]) + v[j + 8]) + v[j + 12];
+  return (((a4[0] + a4[1]) + a4[2]) + a4[3]) + 0.0f;
+}
+
+// The score of a head sum (sc, bf16 bits) and its 16-bit order key.
+__device__ __forceinline__ uint16_t order_key(float tot, uint16_t& sc) {
+  // The reference adds the 0/-inf mask, bf16(x + 0), which only turns -0 into +0.
+  // Here sc is never -0: tot is +0 (the + 0 above) or a sum of bf16 values, all
+  // multiples of 2^-133, so |tot| >= 2^-133 rounds to a nonzero bf16 (the conversion
+  // keeps fp32 denormals: it matches IEEE round-to-nearest-even on them).
+  sc = f2bf(tot);
+  // Order key: sign set -> all bits flipped, else the sign bit flipped; the sign of
+  // the bf16 is that of tot (NaN aside), taken from tot's bits with one shift.
+  const uint32_t neg = (uint32_t)((int32_t)__builtin_bit_cast(uint32_t, tot) >> 31);
+  uint16_t u = (uint16_t)(sc ^ (neg | 0x8000u));
+  if (__builtin_isnan(tot)) u = 0xffffu;  // NaN ranks above everything
+  return u;
+}
+
+// The order of the K gathered picks (32 E per half-wave, entry hl * E + i in sv[i]).
+template <int E>
+__device__ __forceinline__ void sort_picks(uint32_t (&sv)[E], int hl) {
+  constexpr int KP = 32 * E;
+  if (E > 1) {
+    // k > 32: torch sorts the gathered picks stably by value, i.e. value
+    // descending then index ascending = descending order of the entries (all
+    // distinct but for the zero fill, so any correct sort gives the same order).
+    // Bitonic sort (descending) of KP entries, E per lane, element e = hl*E + i.
+    // A compare-exchange is one med3 against a per-lane bound (all ones keeps the
+    // larger entry, zero the smaller); lanes exchange through DPP or ds_swizzle.
+#pragma unroll
+    for (int k = 2; k <= KP; k <<= 1) {
+#pragma unroll
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        if (j >= E) {
+          // (e & j) and (e & k) only depend on hl here (j, k >= E and E a power of 2).
+          const int lj = j / E;
+          const bool lower = (hl & lj) == 0;
+          const bool desc = (hl & (k / E)) == 0;
+          const uint32_t bound = (lower == desc) ? 0xffffffffu : 0u;
+#pragma unroll
+          for (int i = 0; i < E; ++i) sv[i] = med3_u32(sv[i], xor_lanes(sv[i], lj), bound);
+        } else {
+#pragma unroll
+          for (int i = 0; i < E; ++i) {
+            if ((i & j) == 0) {
+              const uint32_t x = sv[i], y = sv[i + j];
+              if (k < E) {  // direction fixed by i
+                const bool desc = (i & k) == 0;
+                sv[i] = desc ? max(x, y) : min(x, y);
+                sv[i + j] = desc ? min(x, y) : max(x, y);
+              } else {
+                const uint32_t bound = (hl & (k / E)) == 0 ? 0xffffffffu : 0u;
+                sv[i] = med3_u32(x, y, bound);
+                sv[i + j] = med3_u32(x, y, ~bound);
+              }
+            }
+          }
+        }
+      }
+    }
+  } else {
+    // k <= 32: torch's 32-slot bitonic network on the gathered list. A slot pair
+    // (lower A, upper B) at stride st belongs to comparator thread
+    // tid = lower slot with bit st removed; stages of size 2..16 use the direction
+    // flag (tid & size/2) != 0, the final merge uses false. The pair exchanges when
+    // ((A > B and A valid) or B invalid) == flag, which also moves equal values.
+    uint32_t x = sv[0];
+    auto stage = [&](int size, int st, bool final_merge) {
+      const uint32_t o = (uint32_t)__shfl_xor((int)x, st, 64);
+      const bool lower = (hl & st) == 0;
+      const uint32_t A = lower ? x : o, B = lower ? o : x;
+      const int lo = lower ? hl : (hl ^ st);
+      const int tid = ((lo >> 1) & ~(st - 1)) | (lo & (st - 1));
+      const bool flag = final_merge ? false : ((tid & (size >> 1)) != 0);
+      const bool va = (A >> 15) & 1u, vb = (B >> 15) & 1u;
+      const bool sw = (((A >> 16) > (B >> 16)) && va) || !vb;
+      if (sw == flag) x = lower ? B : A;
+    };
+#pragma unroll
+    for (int size = 2; size < 32; size <<= 1)
+#pragma unroll
+      for (int st = size >> 1; st > 0; st >>= 1) stage(size, st, false);
+#pragma unroll
+    for (int st = 16; st > 0; st >>= 1) stage(32, st, true);
+    sv[0] = x;
+  }
+}
+
+// The pick of a sorted (E > 1) or networked (E = 1) entry: its candidate index.
+template <int E>
+__device__ __forceinline__ uint32_t pick_of(uint32_t v) {
+  return (E == 1) ? (v & 0x7fffu) : (0xffffu - (v & 0xffffu));
+}
+
+// The entry of candidate c with order key u:
+// E > 1: (key << 16) | ~index, later sorted as a whole (stable order).
+// E = 1: (float-order key << 16) | valid << 15 | index, in gather order.
+template <int E>
+__device__ __forceinline__ uint32_t entry_of(uint32_t u, uint32_t c) {
+  if (E == 1) {
+    const uint32_t fk = (u == 0x7fffu) ? 0x8000u : u;  // -0 == +0 for the comparator
+    return (fk << 16) | 0x8000u | c;
+  }
+  return (u << 16) | (0xffffu - c);
 }
 
 // kDump: the bf16 scores are written to p.scores (the score-stage entry point);
@@ -181,63 +381,10 @@ __global__ __launch_bounds__(256) void ix_score_topk_kernel(IxParams p) {
   // Candidate tiles (32 rows x 128 B) in a 3-slot LDS ring after the wave areas.
   uint8_t* ring = smem + 4 * (size_t)p.wave_bytes;
 
-  // Head weights of this half's token, bf16(fp32(wl) * w_scale), fp32 copies.
   float w[kH];
-  if (t < p.S) {
-    const u32x4* wp = reinterpret_cast<const u32x4*>(p.wl + ((int64_t)b * p.S + t) * kH);
-    const u32x4 w0 = wp[0], w1 = wp[1];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      w[2 * i] = bf2f(f2bf(bf_lo(w0[i]) * p.wscale));
-      w[2 * i + 1] = bf2f(f2bf(bf_hi(w0[i]) * p.wscale));
-      w[8 + 2 * i] = bf2f(f2bf(bf_lo(w1[i]) * p.wscale));
-      w[8 + 2 * i + 1] = bf2f(f2bf(bf_hi(w1[i]) * p.wscale));
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < kH; ++i) w[i] = 0.f;
-  }
-
-  // A operand: row i = lane % 32 is token t0 + (i/4)%2, head i%4 + 4(i/8); lane
-  // holds channels 16ks + 8(lane/32) .. +7 of that row, RoPE applied when asked.
-  // The 32x32 product leaves rows 8(r/4) + 4(lane/32) + r%4 in accumulator r of a
-  // lane, so with this row order accumulator r of lanes 0..31 is head r of token t0
-  // and of lanes 32..63 head r of token t0 + 1, for candidate lane % 32: every lane
-  // holds all 16 heads of one (token, candidate) without an exchange of halves.
+  load_head_weights(p, b, t, w);
   bf16x8 qa[4];
-  {
-    const int tq = t0 + ((lane >> 2) & 1);
-    const int hq = (lane & 3) | (((lane & 31) >> 3) << 2);
-    const int hsel = lane >> 5;
-    if (tq < p.S) {
-      const int64_t row = ((int64_t)b * p.S + tq) * kH + hq;
-      const uint16_t* src = p.q + row * kD;
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        u32x4 v = *reinterpret_cast<const u32x4*>(src + 16 * ks + 8 * hsel);
-        if (p.freqs != nullptr) {
-          const int half_rd = p.rd >> 1;
-#pragma unroll
-          for (int jj = 0; jj < 4; ++jj) {
-            const int dch = 16 * ks + 8 * hsel + 2 * jj;
-            const int pj = (dch - (kD - p.rd)) >> 1;
-            if (dch >= kD - p.rd) {
-              const float c = p.freqs[((int64_t)tq * half_rd + pj) * 2];
-              const float d = p.freqs[((int64_t)tq * half_rd + pj) * 2 + 1];
-              const int64_t n = row * half_rd + pj;
-              float re, im;
-              rope_pair(bf_lo(v[jj]), bf_hi(v[jj]), c, d, p.rope_mode, n, re, im);
-              v[jj] = pack_bf2(re, im);
-            }
-          }
-        }
-        qa[ks] = __builtin_bit_cast(bf16x8, v);
-      }
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) qa[ks] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
-    }
-  }
+  load_q_rows(p, b, t0, lane, qa);
 
   // Zero this half's histogram (8 bins per lane).
   *reinterpret_cast<u32x4*>(myhist + 8 * hl) = u32x4{0u, 0u, 0u, 0u};
@@ -289,43 +436,11 @@ __global__ __launch_bounds__(256) void ix_score_topk_kernel(IxParams p) {
       acc = mfma32x32x16(qa[ks], __builtin_bit_cast(bf16x8, *src), acc);
     }
 
-    // The einsum's bf16 rounding, then relu on the bf16 bit patterns (both heads
-    // of a word at once): word k holds heads 2k, 2k+1.
-    uint32_t pk[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      s16v2 h = __builtin_bit_cast(s16v2, pack_bf2(acc[2 * k], acc[2 * k + 1]));
-      pk[k] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(h, (s16v2){0, 0}));
-    }
-    // * w -> bf16 (the products are exact in fp32), as fp32 values: one
-    // v_cvt_pk_bf16_f32 with a zero low operand leaves bf16(x) in the high half and
-    // zeros below it, which is bf16(x) as an fp32 value.
-    float v[16];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      v[2 * k] = bf16_as_f32(bf_lo(pk[k]) * w[2 * k]);
-      v[2 * k + 1] = bf16_as_f32(bf_hi(pk[k]) * w[2 * k + 1]);
-    }
-    // IEEE fp32 adds in torch's order (accumulator j sums heads j, j+4, j+8, j+12).
-    // torch's four accumulators start at +0; adding the +0 once to the total instead
-    // gives the same value (x + 0 == x except for the sign of a zero, and a -0 can
-    // only reach the total when every term is -0).
-    float a4[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) a4[j] = ((v[j] + v[j + 4]) + v[j + 8]) + v[j + 12];
-    const float tot = (((a4[0] + a4[1]) + a4[2]) + a4[3]) + 0.0f;
-    // The reference adds the 0/-inf mask, bf16(x + 0), which only turns -0 into +0.
-    // Here sc is never -0: tot is +0 (the + 0 above) or a sum of bf16 values, all
-    // multiples of 2^-133, so |tot| >= 2^-133 rounds to a nonzero bf16 (the conversion
-    // keeps fp32 denormals: it matches IEEE round-to-nearest-even on them).
-    const uint16_t sc = f2bf(tot);
+    const float tot = head_total(acc, w);
+    uint16_t sc;
+    const uint16_t u = order_key(tot, sc);
     const int c = 32 * tile + hl;
     const bool valid = c < nv;
-    // Order key: sign set -> all bits flipped, else the sign bit flipped; the sign of
-    // the bf16 is that of tot (NaN aside), taken from tot's bits with one shift.
-    const uint32_t neg = (uint32_t)((int32_t)__builtin_bit_cast(uint32_t, tot) >> 31);
-    uint16_t u = (uint16_t)(sc ^ (neg | 0x8000u));
-    if (__builtin_isnan(tot)) u = 0xffffu;  // NaN ranks above everything
     if constexpr (kDump) {
       if (t < p.S && c < p.T)
         p.scores[((int64_t)b * p.S + t) * p.T + c] = valid ? sc : (uint16_t)0xff80u;
@@ -397,15 +512,6 @@ __global__ __launch_bounds__(256) void ix_score_topk_kernel(IxParams p) {
 
   // Gather the K picks in torch's order: [keys > V in index order] then
   // [keys == V in index order], masked -inf candidates counting as index >= nv.
-  // E > 1: entry = (key << 16) | ~index, later sorted as a whole (stable order).
-  // E = 1: entry = (float-order key << 16) | valid << 15 | index, in gather order.
-  auto entry = [&](uint32_t u, uint32_t c) -> uint32_t {
-    if (E == 1) {
-      const uint32_t fk = (u == 0x7fffu) ? 0x8000u : u;  // -0 == +0 for the comparator
-      return (fk << 16) | 0x8000u | c;
-    }
-    return (u << 16) | (0xffffu - c);
-  };
   // One token at a time over all 64 lanes (64 candidates a step), so the ranks come
   // straight from the 64-bit ballots: mbcnt gives the lanes below, and the running
   // counts stay wave-uniform.
@@ -430,7 +536,7 @@ __global__ __launch_bounds__(256) void ix_score_topk_kernel(IxParams p) {
       const uint64_t gb = __builtin_amdgcn_uicmp(u, Vh, 34) & vb;       // u > Vh
       if (gt) {
         const uint32_t pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(gb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)gb, gt_run));
-        if (pos < (uint32_t)KP) sb[pos] = entry(u, (uint32_t)c);
+        if (pos < (uint32_t)KP) sb[pos] = entry_of<E>(u, (uint32_t)c);
       }
       gt_run += (uint32_t)__builtin_popcountll(gb);
       const bool eq = valid && u == Vh;
@@ -439,7 +545,7 @@ __global__ __launch_bounds__(256) void ix_score_topk_kernel(IxParams p) {
         if (eq) {
           const uint32_t er = __builtin_amdgcn_mbcnt_hi((uint32_t)(eb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)eb, eq_run));
           const uint32_t pos = ngt + er;
-          if (er < need && pos < (uint32_t)KP) sb[pos] = entry(u, (uint32_t)c);
+          if (er < need && pos < (uint32_t)KP) sb[pos] = entry_of<E>(u, (uint32_t)c);
         }
         eq_run += (uint32_t)__builtin_popcountll(eb);
       }
@@ -449,7 +555,7 @@ __global__ __launch_bounds__(256) void ix_score_topk_kernel(IxParams p) {
       // the remaining ties are masked candidates nv, nv+1, ...
       for (uint32_t j = (uint32_t)lane; j < need - eq_taken; j += 64) {
         const uint32_t pos = ngt + eq_taken + j;
-        if (pos < (uint32_t)KP) sb[pos] = entry(kNegInfKey, (uint32_t)nvh + j);
+        if (pos < (uint32_t)KP) sb[pos] = entry_of<E>(kNegInfKey, (uint32_t)nvh + j);
       }
     }
   }
@@ -465,70 +571,7 @@ __global__ __launch_bounds__(256) void ix_score_topk_kernel(IxParams p) {
 #pragma unroll
   for (int i = 0; i < E; ++i) sv[i] = mysbuf[hl * E + i];
 
-  if (E > 1) {
-    // k > 32: torch sorts the gathered picks stably by value, i.e. value
-    // descending then index ascending = descending order of the entries (all
-    // distinct but for the zero fill, so any correct sort gives the same order).
-    // Bitonic sort (descending) of KP entries, E per lane, element e = hl*E + i.
-    // A compare-exchange is one med3 against a per-lane bound (all ones keeps the
-    // larger entry, zero the smaller); lanes exchange through DPP or ds_swizzle.
-#pragma unroll
-    for (int k = 2; k <= KP; k <<= 1) {
-#pragma unroll
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        if (j >= E) {
-          // (e & j) and (e & k) only depend on hl here (j, k >= E and E a power of 2).
-          const int lj = j / E;
-          const bool lower = (hl & lj) == 0;
-          const bool desc = (hl & (k / E)) == 0;
-          const uint32_t bound = (lower == desc) ? 0xffffffffu : 0u;
-#pragma unroll
-          for (int i = 0; i < E; ++i) sv[i] = med3_u32(sv[i], xor_lanes(sv[i], lj), bound);
-        } else {
-#pragma unroll
-          for (int i = 0; i < E; ++i) {
-            if ((i & j) == 0) {
-              const uint32_t x = sv[i], y = sv[i + j];
-              if (k < E) {  // direction fixed by i
-                const bool desc = (i & k) == 0;
-                sv[i] = desc ? max(x, y) : min(x, y);
-                sv[i + j] = desc ? min(x, y) : max(x, y);
-              } else {
-                const uint32_t bound = (hl & (k / E)) == 0 ? 0xffffffffu : 0u;
-                sv[i] = med3_u32(x, y, bound);
-                sv[i + j] = med3_u32(x, y, ~bound);
-              }
-            }
-          }
-        }
-      }
-    }
-  } else {
-    // k <= 32: torch's 32-slot bitonic network on the gathered list. A slot pair
-    // (lower A, upper B) at stride st belongs to comparator thread
-    // tid = lower slot with bit st removed; stages of size 2..16 use the direction
-    // flag (tid & size/2) != 0, the final merge uses false. The pair exchanges when
-    // ((A > B and A valid) or B invalid) == flag, which also moves equal values.
-    uint32_t x = sv[0];
-    auto stage = [&](int size, int st, bool final_merge) {
-      const uint32_t o = (uint32_t)__shfl_xor((int)x, st, 64);
-      const bool lower = (hl & st) == 0;
-      const uint32_t A = lower ? x : o, B = lower ? o : x;
-      const int lo = lower ? hl : (hl ^ st);
-      const int tid = ((lo >> 1) & ~(st - 1)) | (lo & (st - 1));
-      const bool flag = final_merge ? false : ((tid & (size >> 1)) != 0);
-      const bool va = (A >> 15) & 1u, vb = (B >> 15) & 1u;
-      const bool sw = (((A >> 16) > (B >> 16)) && va) || !vb;
-      if (sw == flag) x = lower ? B : A;
-    };
-#pragma unroll
-    for (int size = 2; size < 32; size <<= 1)
-#pragma unroll
-      for (int st = size >> 1; st > 0; st >>= 1) stage(size, st, false);
-#pragma unroll
-    for (int st = 16; st > 0; st >>= 1) stage(32, st, true);
-    sv[0] = x;
-  }
+  sort_picks<E>(sv, hl);
 
   if (t < p.S) {
     int64_t* dst = p.out + ((int64_t)b * p.S + t) * p.K;
@@ -536,7 +579,199 @@ __global__ __launch_bounds__(256) void ix_score_topk_kernel(IxParams p) {
     for (int i = 0; i < E; ++i) {
       const uint32_t e = (uint32_t)(hl * E + i);
       if (e < K) {
-        const uint32_t c = (E == 1) ? (sv[i] & 0x7fffu) : (0xffffu - (sv[i] & 0xffffu));
+        const uint32_t c = pick_of<E>(sv[i]);
+        dst[e] = (p.causal && c >= (uint32_t)nv) ? (int64_t)-1 : (int64_t)c + p.offset;
+      }
+    }
+  }
+}
+
+// Few tokens: one workgroup of W waves per token pair, its candidate tiles divided among
+// the waves (wave wi takes tiles wi, wi + W, ...). Each wave copies its tiles into its own
+// two ring slots, so the tile loop has no barrier; keys and histograms of the pair are
+// shared in LDS. The selection is
+// divided too: candidate tiles for the second histogram, and W / 2 contiguous candidate
+// segments per token for the gather (counted, then placed after the lower segments' picks,
+// which keeps index order). Wave 0 sorts both tokens' picks on its two halves.
+//
+// With few pairs ix_score_topk_kernel is bound by one wave's chain of tiles and its select
+// (650 candidates: 21 tiles, ~15 us; 2048: ~38 us, whatever the number of tokens up to
+// ~2000). Divided over 8 waves: 7.2 and 11.9 us for 8 decode tokens. The copies are whole
+// 1 KB runs into LDS: fragment loads straight from memory touch 32 rows each and were
+// bound by that (2048 candidates: 14.6 us, and 15.5 us with three tiles in flight).
+template <int E, int W>
+__global__ __launch_bounds__(64 * W) void ix_score_topk_few_kernel(IxParams p) {
+  static_assert(W == 2 || W == 4 || W == 8, "waves per token pair");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  constexpr int KP = 32 * E;
+  constexpr int kSeg = W / 2;                         // gather segments per token
+  uint32_t* hist1 = reinterpret_cast<uint32_t*>(smem + 8192 * W);  // [2][256] high bytes (after the W tile rings)
+  uint32_t* hist2 = hist1 + 512;                        // [2][256] low bytes of the k-th key's bin
+  uint32_t* cnt = hist2 + 512;                          // [2][kSeg] gt, then [2][kSeg] eq
+  uint32_t* sbuf = cnt + 4 * kSeg;                      // [2][KP] picks
+  uint16_t* keys = reinterpret_cast<uint16_t*>(sbuf + 2 * KP);  // [2][tiles * 32]
+  const int lane = threadIdx.x & 63;
+  const int wi = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int half = lane >> 5, hl = lane & 31;
+  const int b = (int)(blockIdx.x % (unsigned)p.B);
+  const int pr = p.npairs - 1 - (int)(blockIdx.x / (unsigned)p.B);
+  const int t0 = 2 * pr;
+  const int t = t0 + half;
+  const int nv = n_valid(p, t);
+  const int ntile = (n_valid(p, min(t0 + 1, p.S - 1)) + 31) >> 5;
+  const int krow = 32 * (p.keys_bytes / 128);  // key row length: whole tiles
+
+  // Tile copies into the wave's two ring slots, as in ix_score_topk_kernel (rows >= T read
+  // as zero): unit i moves rows 8i .. 8i+7.
+  const i32x4 krs = make_rsrc(p.kv + (int64_t)b * p.kvbs, (uint32_t)p.T * (uint32_t)(kD * 2));
+  const uint32_t ring_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + 8192u * (uint32_t)wi;
+  const uint32_t koff = (uint32_t)((lane >> 3) * kD + 8 * ((lane & 7) ^ (lane >> 3))) * 2u;
+  auto issue = [&](int tile, int slot) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      lds_dma16(krs, (uint32_t)((32 * tile + 8 * i) * kD * 2) + koff, ring_lds + 4096u * (uint32_t)slot + 1024u * (uint32_t)i);
+  };
+  if (wi < ntile) issue(wi, 0);
+  if (wi + W < ntile) issue(wi + W, 1);
+  float w[kH];
+  load_head_weights(p, b, t, w);
+  bf16x8 qa[4];
+  load_q_rows(p, b, t0, lane, qa);
+  for (int i = (int)threadIdx.x; i < 1024; i += 64 * W) hist1[i] = 0u;
+  // Consume the compiler-tracked loads here, so that its vmcnt(0) for them stays out of the loop.
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) asm volatile("" ::"v"(qa[ks]));
+#pragma unroll
+  for (int i = 0; i < kH; ++i) asm volatile("" ::"v"(w[i]));
+  __syncthreads();
+  uint32_t* myhist = hist1 + 256 * half;
+  uint32_t boff[4];  // the lane's B fragments inside a ring slot
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) boff[ks] = ring_lds + 16u * (uint32_t)(8 * hl + ((2 * ks + half) ^ (hl & 7)));
+  auto step = [&](auto slot_c, const int tile) {
+    constexpr int kSlot = decltype(slot_c)::value;
+    if (tile + W < ntile) wait_vmcnt<4>();  // only the next tile's copies may be outstanding
+    else wait_vmcnt<0>();
+    asm volatile("" ::: "memory");
+    f32x16 acc = {};
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const auto* src = (__attribute__((address_space(3))) const u32x4*)(uintptr_t)(boff[ks] + 4096u * kSlot);
+      acc = mfma32x32x16(qa[ks], __builtin_bit_cast(bf16x8, *src), acc);
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the slot's reads have returned
+    if (tile + 2 * W < ntile) issue(tile + 2 * W, kSlot);
+    uint16_t sc;
+    const uint16_t u = order_key(head_total(acc, w), sc);
+    const int c = 32 * tile + hl;
+    keys[half * krow + c] = u;
+    if (c < nv) atomicAdd(&myhist[u >> 8], 1u);
+  };
+  for (int tile = wi; tile < ntile; tile += 2 * W) {
+    step(std::integral_constant<int, 0>{}, tile);
+    if (tile + W < ntile) step(std::integral_constant<int, 1>{}, tile + W);
+  }
+  constexpr uint32_t kNegInfKey = 0x007fu;  // masked candidates enter the histograms analytically
+  const uint32_t K = (uint32_t)p.K;
+  const uint32_t nmask = (t < p.S) ? (uint32_t)(p.T - nv) : 0u;
+  if (wi == 0 && hl == 0 && nmask > 0) atomicAdd(&myhist[kNegInfKey >> 8], nmask);
+  __syncthreads();
+
+  // Every wave finds the bins for itself.
+  uint32_t gt1 = 0, gt2 = 0;
+  const int b1 = find_bin(myhist, lane, K, gt1);
+  uint32_t* myhist2 = hist2 + 256 * half;
+  for (int tile = wi; tile < ntile; tile += W) {
+    const uint32_t u = keys[half * krow + 32 * tile + hl];
+    if (32 * tile + hl < nv && (int)(u >> 8) == b1) atomicAdd(&myhist2[u & 255u], 1u);
+  }
+  if (wi == 0 && hl == 0 && nmask > 0 && b1 == (int)(kNegInfKey >> 8)) atomicAdd(&myhist2[kNegInfKey & 255u], nmask);
+  __syncthreads();
+  const int b0 = find_bin(myhist2, lane, K - gt1, gt2);
+  const bool real = (t < p.S) && b1 >= 0 && b0 >= 0;
+  const uint32_t V = real ? (((uint32_t)b1 << 8) | (uint32_t)b0) : 0x10000u;  // 0x10000: nothing matches
+  const uint32_t n_gt = real ? gt1 + gt2 : 0u;
+  const uint32_t need_eq = real ? K - n_gt : 0u;
+
+  // Gather: this wave's segment of token h, in steps of 64 candidates.
+  const int h = wi & 1, seg = wi >> 1;
+  const uint32_t Vh = (uint32_t)__builtin_amdgcn_readlane((int)V, 32 * h);
+  const uint32_t ngt = (uint32_t)__builtin_amdgcn_readlane((int)n_gt, 32 * h);
+  const uint32_t need = (uint32_t)__builtin_amdgcn_readlane((int)need_eq, 32 * h);
+  const int nvh = __builtin_amdgcn_readlane(nv, 32 * h);
+  const int seglen = ((nvh + 64 * kSeg - 1) / (64 * kSeg)) * 64;
+  const int s_beg = min(nvh, seg * seglen), s_end = min(nvh, s_beg + seglen);
+  const uint16_t* kh = keys + h * krow;
+  uint32_t ng = 0, ne = 0;
+#pragma unroll 2
+  for (int c0 = s_beg; c0 < s_end; c0 += 64) {
+    // order keys are >= 0x007f: the 0 past the segment never matches
+    const uint32_t u = c0 + lane < s_end ? (uint32_t)kh[c0 + lane] : 0u;
+    ng += (uint32_t)__builtin_popcountll(__builtin_amdgcn_uicmp(u, Vh, 34));  // u > Vh
+    ne += (uint32_t)__builtin_popcountll(__builtin_amdgcn_uicmp(u, Vh, 32));  // u == Vh
+  }
+  if (lane == 0) {
+    cnt[h * kSeg + seg] = ng;
+    cnt[(2 + h) * kSeg + seg] = ne;
+  }
+  __syncthreads();
+  uint32_t gt_run = 0, eq_run = 0, eq_all = 0;
+#pragma unroll
+  for (int i = 0; i < kSeg; ++i) {
+    const uint32_t e = cnt[(2 + h) * kSeg + i];
+    if (i < seg) {
+      gt_run += cnt[h * kSeg + i];
+      eq_run += e;
+    }
+    eq_all += e;
+  }
+  uint32_t* sb = sbuf + KP * h;
+#pragma unroll 2
+  for (int c0 = s_beg; c0 < s_end; c0 += 64) {
+    const uint32_t c = (uint32_t)(c0 + lane);
+    const uint32_t u = (int)c < s_end ? (uint32_t)kh[c] : 0u;
+    const uint64_t gb = __builtin_amdgcn_uicmp(u, Vh, 34);
+    if (u > Vh) {
+      const uint32_t pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(gb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)gb, gt_run));
+      if (pos < (uint32_t)KP) sb[pos] = entry_of<E>(u, c);
+    }
+    gt_run += (uint32_t)__builtin_popcountll(gb);
+    const uint64_t eb = __builtin_amdgcn_uicmp(u, Vh, 32);
+    if (eb != 0) {
+      if (u == Vh) {
+        const uint32_t er = __builtin_amdgcn_mbcnt_hi((uint32_t)(eb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)eb, eq_run));
+        const uint32_t pos = ngt + er;
+        if (er < need && pos < (uint32_t)KP) sb[pos] = entry_of<E>(u, c);
+      }
+      eq_run += (uint32_t)__builtin_popcountll(eb);
+    }
+  }
+  if (seg == 0) {
+    const uint32_t eq_taken = eq_all < need ? eq_all : need;
+    if (Vh == kNegInfKey) {  // the remaining ties are masked candidates nv, nv+1, ...
+      for (uint32_t j = (uint32_t)lane; j < need - eq_taken; j += 64) {
+        const uint32_t pos = ngt + eq_taken + j;
+        if (pos < (uint32_t)KP) sb[pos] = entry_of<E>(kNegInfKey, (uint32_t)nvh + j);
+      }
+    }
+  }
+  __syncthreads();
+  if (wi != 0) return;
+  const uint32_t nsel = real ? K : 0u;
+  uint32_t sv[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const uint32_t e = (uint32_t)(hl * E + i);
+    sv[i] = e < nsel ? sbuf[KP * half + e] : 0u;  // E > 1: sorts last; E = 1: invalid slot
+  }
+  sort_picks<E>(sv, hl);
+  if (t < p.S) {
+    int64_t* dst = p.out + ((int64_t)b * p.S + t) * p.K;
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      const uint32_t e = (uint32_t)(hl * E + i);
+      if (e < K) {
+        const uint32_t c = pick_of<E>(sv[i]);
         dst[e] = (p.causal && c >= (uint32_t)nv) ? (int64_t)-1 : (int64_t)c + p.offset;
       }
     }
@@ -578,6 +813,49 @@ int dsa_indexer_wide_launch(const void* q, const void* kv_cache, int64_t kv_batc
                             int64_t workspace_bytes, hipStream_t stream);
 
 namespace {
+
+// Waves per token pair of ix_score_topk_few_kernel, or 0 for ix_score_topk_kernel, for
+// `pairs` workgroups whose longest row has nt candidate tiles on cu CUs. Measured at 32 ..
+// 2048 candidates and 8 .. 3072 pairs (256 CUs; us, ix_score_topk_kernel -> this):
+//  one pair per CU: 8 waves above 8 tiles (650: 17.4 -> 8.3, four waves 9.3), 4 from 4 tiles
+//    (128: 7.0 -> 5.6, eight 6.1), else 2 (64: 5.6 -> 4.7);
+//  two per CU: 4 waves (650: 17.3 -> 10.7; 2048: 42.1 -> 20.8), 2 below 4 tiles (5.6 -> 5.3);
+//  up to three per CU 4 waves from 8 tiles (256: 9.5 -> 8.4), up to four 2 (256: 9.7 -> 8.8;
+//    2048: 42.7 -> 32.8); below 8 tiles the shared steps cost as much as they save;
+//  beyond that only causal rows, half of which are short, gain, with 2 waves: up to six per
+//    CU from 8 tiles (256: 10.3 -> 9.1), up to eight from 20 (650: 19.4 -> 18.4; 1300:
+//    31.9 -> 25.1). At 12 per CU the tile loop's throughput decides (650: 20.5 -> 24.4).
+int few_waves(int64_t pairs, int nt, bool causal, int cu) {
+  if (pairs <= cu) return nt > 8 ? 8 : nt >= 4 ? 4 : 2;
+  if (pairs <= 2 * (int64_t)cu) return nt >= 4 ? 4 : 2;
+  if (pairs <= 3 * (int64_t)cu) return nt >= 8 ? 4 : 0;
+  if (pairs <= 4 * (int64_t)cu) return nt >= 8 ? 2 : 0;
+  if (causal && pairs <= 6 * (int64_t)cu) return nt >= 8 ? 2 : 0;
+  if (causal && pairs <= 8 * (int64_t)cu) return nt >= 20 ? 2 : 0;
+  return 0;
+}
+
+template <int E, int W>
+int launch_few(const IxParams& p, unsigned pairs, hipStream_t st) {
+  // Tile rings, histograms, segment counts, picks, keys.
+  const size_t smem = 8192 * W + 4096 + 16 * (W / 2) + 2 * 32 * E * 4 + (size_t)p.keys_bytes;
+  if (smem > 64 * 1024 &&
+      dsa_host::ensure_dyn_lds((const void*)ix_score_topk_few_kernel<E, W>, (int)smem) != DSA_OK)
+    return DSA_ERR_LAUNCH;
+  hipLaunchKernelGGL((ix_score_topk_few_kernel<E, W>), dim3(pairs), dim3(64 * W), smem, st, p);
+  return hipGetLastError() == hipSuccess ? DSA_OK : DSA_ERR_LAUNCH;
+}
+
+template <int W>
+int launch_few_w(const IxParams& p, int e, unsigned pairs, hipStream_t st) {
+  switch (e) {
+    case 1: return launch_few<1, W>(p, pairs, st);
+    case 2: return launch_few<2, W>(p, pairs, st);
+    case 4: return launch_few<4, W>(p, pairs, st);
+    case 8: return launch_few<8, W>(p, pairs, st);
+    default: return DSA_ERR_UNSUPPORTED;
+  }
+}
 
 int launch_ix(const void* q, const void* kv_cache, int64_t kv_batch_stride, const void* wl,
               float w_scale, const void* freqs_cis, int32_t rope_mode, int64_t* out,
@@ -645,6 +923,17 @@ int launch_ix(const void* q, const void* kv_cache, int64_t kv_batch_stride, cons
     if (out != nullptr || E != 1) return DSA_ERR_UNSUPPORTED;
     hipLaunchKernelGGL((ix_score_topk_kernel<1, true>), dim3((unsigned)blocks), dim3(256), smem, st, p);
     return hipGetLastError() == hipSuccess ? DSA_OK : DSA_ERR_LAUNCH;
+  }
+  int cu = 0;
+  if (dsa_host::device_cu_count(&cu) != DSA_OK) return DSA_ERR_DEVICE;
+  const int64_t pairs = b * (int64_t)p.npairs;
+  const int64_t longest = p.causal ? s / ratio : n_cand;
+  const int nt = (int)(((longest < n_cand ? longest : n_cand) + 31) / 32);
+  switch (few_waves(pairs, nt, p.causal != 0, cu)) {
+    case 2: return launch_few_w<2>(p, E, (unsigned)pairs, st);
+    case 4: return launch_few_w<4>(p, E, (unsigned)pairs, st);
+    case 8: return launch_few_w<8>(p, E, (unsigned)pairs, st);
+    default: break;
   }
   switch (E) {
     case 1: hipLaunchKernelGGL((ix_score_topk_kernel<1, false>), dim3((unsigned)blocks), dim3(256), smem, st, p); break;

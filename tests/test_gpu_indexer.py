@@ -456,3 +456,41 @@ def test_model_launch_plan_reuse(gpu):
     r.weights_proj.weight.data.copy_(m.weights_proj.weight.data)
     _check_equal(m(x2, qr2, sp, off), r(x2, qr2, sp, off), "plan new weights")
     _check_equal(m(x2, qr2, 0, 3), r(x2, qr2, 0, 3), "plan new offset")
+
+
+# Few token pairs: several waves share a pair's candidates. The edges (256 CUs) of the number
+# of pairs and of candidate tiles (2 / 3, 3 / 4, 7 / 8 / 9, 20, 64 tiles), a last tile of one
+# candidate, odd token counts (a pair's second token missing), k at 1, 32, 33 and 256, causal
+# rows with fewer candidates than k.
+FEW = [
+    # b, s, T, k, ratio, causal
+    (1, 1, 1, 1, 1, False), (8, 1, 650, 128, 4, False), (3, 1, 2048, 256, 1, False), (1, 2, 97, 33, 1, False),
+    (2, 5, 289, 32, 1, False), (128, 4, 257, 64, 1, False), (1, 513, 2048, 256, 1, False), (257, 2, 96, 96, 1, False),
+    (2, 511, 65, 40, 1, False), (3, 512, 256, 128, 1, False), (2, 1025, 225, 128, 1, False), (4, 512, 641, 200, 1, False),
+    (1, 63, 63, 16, 1, True), (1, 515, 257, 130, 2, True), (4, 255, 63, 32, 4, True), (1, 2047, 2047, 256, 1, True),
+    (3, 1003, 250, 128, 4, True), (1, 3071, 255, 128, 12, True), (2, 2047, 682, 128, 3, True),
+]
+
+
+@pytest.mark.parametrize("case", FEW)
+@pytest.mark.parametrize("ties", [False, True])
+def test_few_pairs_edges(gpu, case, ties):
+    """The picks against torch's topk of the score stage's bf16 scores (the kernel that the
+    score-stage tests hold to the reference), with N(0, 1) inputs and with inputs of a few
+    small values, whose scores tie by the hundreds (also at the k-th pick)."""
+    b, s, T, k, ratio, causal = case
+    _say("few pairs", case, "ties" if ties else "")
+    g = torch.Generator(device=gpu).manual_seed(s + T)
+    draw = lambda *n: (torch.randint(-1, 2, n, generator=g, device=gpu).float() if ties
+                       else torch.randn(n, generator=g, device=gpu)).to(torch.bfloat16)
+    q, kv, wl = draw(b, s, 16, 64), draw(b, T, 64), draw(b, s, 16)
+    scale = 64 ** -0.5 * 16 ** -0.5
+    got = _native.indexer_score_topk(q, kv, wl, scale, None, 32, T, k, ratio, causal, 5)
+    scores = _native.indexer_scores(q, kv, wl, scale, None, 32, T, ratio, causal)
+    idx = scores.topk(k, dim=-1)[1]
+    if causal:
+        lim = torch.arange(1, s + 1, device=gpu).unsqueeze(1) // ratio
+        want = torch.where(idx >= lim, -1, idx + 5)
+    else:
+        want = idx + 5
+    _check_equal(got, want, f"few{case}")
