@@ -8,8 +8,8 @@
 // one workgroup per token, one wave per 32 heads (ceil(h/32) waves). The slots are
 // processed in blocks of 32. The selected kv rows (256 B each) of a block are
 // copied straight from global memory into LDS by global_load_lds_dwordx4 (no
-// register staging), into a ring of kRing block buffers: kRing - 1 blocks are in
-// flight while one is computed. Every wave then runs
+// register staging), into a ring of kRing block buffers: one block is in flight while
+// the scores of the next and the products of the current one are computed. Every wave then runs
 //   S^T[32 keys x 32 heads]  = K[32 x 128] . Q^T[128 x 32]   (8 x mfma 32x32x16)
 //   online softmax with the sink as the initial maximum (log2 domain)
 //   O^T[128 x 32 heads]     += V^T[128 x 32] . (P_hi + P_lo)^T (16 x mfma 32x32x16)
@@ -29,7 +29,7 @@ namespace {
 
 constexpr int kD = 128;
 constexpr int kKB = 32;          // slots per block
-constexpr int kRing = 4;         // LDS block buffers (kRing - 1 blocks in flight)
+constexpr int kRing = 3;         // LDS block buffers (one block in flight beside the two in use)
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kRaise = 8.0f;   // log2 headroom before the running max is raised
 // bf16 pairs (-1, 0) and (0, -1) as bit patterns: dot2(h, neg_lo, p0) = p0 - h.lo,
@@ -63,11 +63,22 @@ __device__ __forceinline__ int out_ch(int dt, int i) {
 // LDS row r (256 B = 16 chunks of 16 B): chunk c lives at r*16 + (c ^ (r & 15)).
 __device__ __forceinline__ int swz(int r, int c) { return r * 16 + (c ^ (r & 15)); }
 
+// Bound by the matrix cores and the VALU (per block and wave 24 products, ~770 cycles, and
+// ~700 cycles of softmax), which overlap only across the waves of a SIMD, so the kernel
+// keeps three there: at most 168 VGPRs (fragment addresses come from one register each by
+// xor, mask bits and copy offsets are formed at their use) and a ring of three. Against two
+// waves at 214 VGPRs and a ring of four: configs[3] 397-412 -> 383-388 us (1.0 PFLOP/s of
+// issued products), 3 x 421 tokens x 48 heads, 333 slots 31.0 -> 26.6, 4096 tokens x 96
+// heads, 256 slots 103 -> 83-85, 4000 x 128 heads, 2048 slots 650 -> 650. The same registers
+// at two waves per SIMD: no change. No s_setprio, or the raised priority on the products
+// instead: 1-3 % slower.
 template <int NW, typename IdxT>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void sa_gather_kernel(GatherParams p) {
   const IdxT* const idx = static_cast<const IdxT*>(p.idx);
-  __shared__ u32x4 ring[kRing][kKB * 16];  // kRing blocks of 32 gathered rows (8 KB each)
+  // kRing blocks of 32 gathered rows (8 KB each); at the end one 8 KB area per wave. 1 KB
+  // alignment: fragment addresses inside a block are formed by xor.
+  __shared__ __align__(1024) u32x4 ring[kRing > NW ? kRing : NW][kKB * 16];
   __shared__ int32_t nblk_w[NW];  // per wave: blocks up to its last valid slot
   extern __shared__ int32_t slot[];         // the token's slot indices (masked -> -1)
   const int tid = threadIdx.x;
@@ -149,27 +160,37 @@ void sa_gather_kernel(GatherParams p) {
   const int wis = __builtin_amdgcn_readfirstlane(wi);
   const i32x4 rsrc = make_rsrc(kvb, (uint32_t)p.NKV * (uint32_t)(kD * 2));
   const uint32_t ring_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) u32x4*)&ring[0][0];
-  int urow[kUnits];
-  uint32_t uoff[kUnits], ulds[kUnits];
-#pragma unroll
-  for (int i = 0; i < kUnits; ++i) {
-    int u = wis + NW * i;
-    if (u >= 8) u -= 8;
-    urow[i] = 4 * u + (lane >> 4);
-    uoff[i] = 16u * (uint32_t)((lane & 15) ^ (urow[i] & 15));  // bytes within the row
-    ulds[i] = ring_lds + 1024u * (uint32_t)u;
-  }
+  // Per lane and unit u: tile row 4u + lane/16 and byte offset 16 ((lane%16) ^ (row%16)) in
+  // the row, the unit entering as a scalar. They are recomputed from the lane id at each
+  // use: held across the block loop they would spill.
+  const uint32_t slot_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int32_t*)slot;
+  auto lane_id = [] {
+    int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(ln));
+    return ln;
+  };
+  auto unit = [&](int i) {
+    const int u = wis + NW * i;
+    return u >= 8 ? u - 8 : u;
+  };
   // Slot values (kv rows) of this lane's units of block blk.
   auto rows_of = [&](int blk, int (&rv)[kUnits]) {
+    const uint32_t srow = slot_lds + 4u * (uint32_t)(lane_id() >> 4);
 #pragma unroll
-    for (int i = 0; i < kUnits; ++i) rv[i] = slot[blk * kKB + urow[i]];
+    for (int i = 0; i < kUnits; ++i)
+      rv[i] = *(__attribute__((address_space(3))) const int32_t*)(uintptr_t)(srow + (uint32_t)(blk * kKB + 4 * unit(i)) * 4u);
   };
   // Copy block blk (rows rv) into ring buffer rs. A masked row (-1) gives an
   // offset beyond the resource, which reads zeros.
   auto issue = [&](int rs, const int (&rv)[kUnits]) {
+    const int ln = lane_id();
+    const uint32_t ubase = 16u * (uint32_t)((ln & 15) ^ (ln >> 4));
 #pragma unroll
-    for (int i = 0; i < kUnits; ++i)
-      lds_dma16(rsrc, (uint32_t)rv[i] * (uint32_t)(kD * 2) + uoff[i], ulds[i] + 8192u * (uint32_t)rs);
+    for (int i = 0; i < kUnits; ++i) {
+      const int u = unit(i);
+      lds_dma16(rsrc, ((uint32_t)rv[i] * (uint32_t)(kD * 2)) + (ubase ^ (64u * (uint32_t)(u & 3))),
+                ring_lds + 1024u * (uint32_t)u + 8192u * (uint32_t)rs);
+    }
   };
   f32x16 o[4];
 #pragma unroll
@@ -181,17 +202,29 @@ void sa_gather_kernel(GatherParams p) {
   float m_run = fmaxf(sink_l2, -FLT_MAX);
   float l_run = 0.f;       // this lane's partial sum of exp2(s - m_run)
 
-  // S^T = K . Q^T for the block in LDS buffer kvl: A = K rows (key = lane%32,
+  // S^T = K . Q^T for the block in LDS buffer j: A = K rows (key = lane%32,
   // channels 16ks + 8hf ..). Lane holds keys 8(r/4) + 4hf + (r%4) of head col.
-  auto qk = [&](const u32x4* kvl) {
+  // Chunk 2ks + hf of the row sits at (2ks + hf) ^ (row%16) = 2ks ^ (hf ^ row%16), so the
+  // eight addresses are kbase with a constant xored in.
+  typedef __attribute__((address_space(3))) const u32x4* lds_cu32x4_ptr;
+  const uint32_t kbase = ring_lds + 16u * (uint32_t)swz(lane & 31, hf);
+  auto qk = [&](const int j) {
     f32x16 acc = {};
+    uint32_t kb_ = kbase;
+    asm volatile("" : "+v"(kb_));
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      const bf16x8 a = __builtin_bit_cast(bf16x8, kvl[swz(lane & 31, 2 * ks + hf)]);
+      const bf16x8 a = __builtin_bit_cast(bf16x8, *(lds_cu32x4_ptr)(uintptr_t)((kb_ ^ (32u * ks)) + 8192u * j));
       acc = mfma32x32x16(a, qf[ks], acc);
     }
     return acc;
   };
+  // V^T reads: supplier lane u of a 16-lane group reads 4 channels of one key row, key =
+  // base + (u >> 2), channels out_ch(dt, 16*g16 + 4*(u & 3)) .. +3. The chunk's bits are
+  // dt (2..1) and the lane's (3, 0), so dt is a xor, and 8 rows on flip the swizzle's bit 3.
+  const int u = lane & 15, g16 = (lane >> 4) & 1;
+  const int vch = out_ch(0, 16 * g16 + 4 * (u & 3));
+  const uint32_t vbase = ring_lds + 16u * (uint32_t)swz(4 * hf + (u >> 2), vch >> 3) + 2u * (uint32_t)(vch & 7);
 
   int rv[kUnits];
 #pragma unroll
@@ -215,9 +248,8 @@ void sa_gather_kernel(GatherParams p) {
   // Two-stage pipeline: iteration kb computes S of block kb+1 on the matrix
   // cores while the VALU runs the softmax of block kb, then O += P(kb) V(kb).
   // Block kb+1 must be in LDS at the start of iteration kb, block kb is read
-  // until its end; the copy issued in iteration kb (block kb+3) goes to the
-  // buffer of block kb-1, released by the barrier. So 2 copies are in flight.
-  static_assert(kRing == 4, "the waits assume a ring of 4 buffers");
+  // until its end; the copy issued in iteration kb (block kb+2) goes to the
+  // buffer of block kb-1, released by the barrier.
   // One iteration for block kb, which sits in ring buffer j = kb % kRing (the
   // loop is unrolled by kRing so that j, and with it every LDS offset below,
   // is a compile-time constant).
@@ -233,22 +265,19 @@ void sa_gather_kernel(GatherParams p) {
   auto step = [&](const int kb, const int j) {
     uint32_t vm_next = 0u;
     if (kb + 1 < nb) {
-      // Block kb+1 has landed once at most one younger block is outstanding.
-      if (kb + 2 < nb) wait_vmcnt<kUnits>();
-      else wait_vmcnt<0>();
+      wait_vmcnt<0>();  // block kb+1 has landed (kb+2 is issued below)
       __syncthreads();  // block kb+1 is in LDS for every wave; block kb-1 is consumed
       if (kb + kRing - 1 < nb) issue((j + kRing - 1) % kRing, rv);
       vm_next = (uint32_t)__ballot(vslot >= 0);
       rows_of(min(kb + kRing, nb - 1), rv);
-      vslot = slot[min(kb + 2, nb - 1) * kKB + (lane & 31)];
+      vslot = slot[min(kb + 2, nb - 1) * kKB + (lane_id() & 31)];
     }
     // Masked slots of block kb -> -inf (uniform branch; full blocks skip it).
     if (vm_cur != 0xffffffffu) {
+      const uint32_t vmh = vm_cur >> (4 * hf);  // bit 8(r/4) + r%4: the lane's key of register r
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = 8 * (r >> 2) + 4 * hf + (r & 3);
-        if (!((vm_cur >> key) & 1u)) s_cur[r] = -INFINITY;
-      }
+      for (int r = 0; r < 16; ++r)
+        if ((vmh & (1u << (8 * (r >> 2) + (r & 3)))) == 0u) s_cur[r] = -INFINITY;
     }
     // max(s) * c2 == max(s * c2) for c2 > 0; the other lane half holds the
     // other 16 keys of the same head.
@@ -280,7 +309,7 @@ void sa_gather_kernel(GatherParams p) {
     // shared with another workgroup's wave, the softmax (VALU) of one wave then
     // tends to issue while the other's products occupy the matrix cores (~4 %).
     __builtin_amdgcn_s_setprio(1);
-    const f32x16 s_next = qk(ring[(j + 1) % kRing]);
+    const f32x16 s_next = qk((j + 1) % kRing);
 
     float pe[16];
 #pragma unroll
@@ -308,40 +337,46 @@ void sa_gather_kernel(GatherParams p) {
     }
     // O^T += V^T . P^T. A operand rows: channel out_ch(dt, lane%32); the two
     // transposed reads give keys 16st + 4hf + (0..3) and 16st + 8 + 4hf + (0..3).
-    // Supplier lane u of a 16-lane group reads 4 channels of one key row:
-    // key = base + (u >> 2), channels out_ch(dt, 16*g16 + 4*(u & 3)) .. +3.
+    // One fragment is read ahead of its two products (the order is pinned below).
     __builtin_amdgcn_s_setprio(0);
-    const int u = lane & 15, g16 = (lane >> 4) & 1;
-    const uint16_t* kvh = reinterpret_cast<const uint16_t*>(ring[j]);
+    uint32_t vb_ = vbase;
+    asm volatile("" : "+v"(vb_));
+    auto rdv = [&](int i) {
+      const int st = i >> 2, dt = i & 3;
+      const uint32_t at = 8192u * j + 4096u * st;
+      const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_s16x4_ptr)(uintptr_t)((vb_ ^ (32u * dt)) + at));
+      const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_s16x4_ptr)(uintptr_t)((vb_ ^ (32u * dt + 128u)) + at + 2048u));
+      return __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    bf16x8 va = rdv(0);
 #pragma unroll
-    for (int st = 0; st < 2; ++st) {
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        const int ch = out_ch(dt, 16 * g16 + 4 * (u & 3));
-        const int r0 = 16 * st + 4 * hf + (u >> 2);
-        const int r1 = r0 + 8;
-        const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_s16x4_ptr)(kvh + swz(r0, ch >> 3) * 8 + (ch & 7)));
-        const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_s16x4_ptr)(kvh + swz(r1, ch >> 3) * 8 + (ch & 7)));
-        const s16x8 v01 = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-        const bf16x8 a = __builtin_bit_cast(bf16x8, v01);
-        o[dt] = mfma32x32x16(a, plo[st], o[dt]);
-        o[dt] = mfma32x32x16(a, phi[st], o[dt]);
-      }
+    for (int i = 0; i < 8; ++i) {
+      bf16x8 vn = va;
+      if (i + 1 < 8) vn = rdv(i + 1);
+      o[i & 3] = mfma32x32x16(va, plo[i >> 2], o[i & 3]);
+      o[i & 3] = mfma32x32x16(va, phi[i >> 2], o[i & 3]);
+      va = vn;
     }
+    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+    for (int i = 0; i < 7; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
     s_cur = s_next;
     vm_cur = vm_next;
   };
 
   if (nb > 0) {
-    if (nb >= 3) wait_vmcnt<2 * kUnits>();
-    else if (nb == 2) wait_vmcnt<kUnits>();
+    if (nb >= 2) wait_vmcnt<kUnits>();
     else wait_vmcnt<0>();
     __syncthreads();
     vm_cur = (uint32_t)__ballot(vslot >= 0);
     vslot = slot[min(1, nb - 1) * kKB + (lane & 31)];
-    s_cur = qk(ring[0]);
+    s_cur = qk(0);
     for (int kb0 = 0; kb0 < nb; kb0 += kRing) {
 #pragma unroll
       for (int j = 0; j < kRing; ++j) {
