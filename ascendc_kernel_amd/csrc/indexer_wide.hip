@@ -100,6 +100,20 @@ __device__ __forceinline__ int n_valid_w(const WideParams& p, int t) {
 }
 
 
+// Inclusive prefix sum over the 64 lanes by DPP: row shifts within each row of 16 lanes,
+// then the row totals (lane 15 of rows 0, 2 to rows 1, 3; lane 31 to rows 2, 3). No LDS
+// round trips, which a chain of lane permutes would take six of.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t x) {
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);  // row_shr:1
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return x;
+}
+__device__ __forceinline__ uint32_t last_lane(uint32_t x) { return (uint32_t)__builtin_amdgcn_readlane((int)x, 63); }
+
 // Full wave over a 256-bin histogram (bins ascending in key) kept as NC copies
 // kCopyStride words apart and summed here: the bin b with count(bins > b) < need <=
 // count(bins >= b); gt = count(bins > b).
@@ -116,13 +130,8 @@ __device__ __forceinline__ int find_bin64(const uint32_t* hist, int lane, uint32
     v[3] += w[3];
   }
   const uint32_t local = v[0] + v[1] + v[2] + v[3];
-  uint32_t incl = local;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t o = __shfl(incl, (lane + off) & 63, 64);
-    if (lane + off < 64) incl += o;
-  }
-  uint32_t cum = incl - local;
+  const uint32_t below = wave_scan(local);
+  uint32_t cum = last_lane(below) - below;  // entries in the bins of higher lanes
   int fb = -1;
   uint32_t fgt = 0;
 #pragma unroll
@@ -136,8 +145,8 @@ __device__ __forceinline__ int find_bin64(const uint32_t* hist, int lane, uint32
   }
   const uint64_t m = __ballot(fb >= 0);
   const int src = m ? (int)__builtin_ctzll(m) : 0;
-  gt = __shfl(fgt, src, 64);
-  return __shfl(fb, src, 64);
+  gt = (uint32_t)__builtin_amdgcn_readlane((int)fgt, src);
+  return __builtin_amdgcn_readlane(fb, src);
 }
 
 // The occupied bins (non-zero total over NC copies) at or above lo_bin of a 256-bin
@@ -159,14 +168,9 @@ __device__ __forceinline__ int rank_map64(const uint32_t* hist, int lane, int lo
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     if (v[i] != 0u && 4 * lane + i >= lo_bin) occ |= 1u << i;
-  const uint32_t local = (uint32_t)__builtin_popcount(occ);
-  uint32_t incl = local;  // occupied bins in lanes >= lane
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t o = __shfl(incl, (lane + off) & 63, 64);
-    if (lane + off < 64) incl += o;
-  }
-  uint32_t above = incl - local;
+  const uint32_t below = wave_scan((uint32_t)__builtin_popcount(occ));
+  const uint32_t total = last_lane(below);
+  uint32_t above = total - below;  // occupied bins in higher lanes
   uint32_t word = 0u;
 #pragma unroll
   for (int i = 3; i >= 0; --i)
@@ -175,7 +179,7 @@ __device__ __forceinline__ int rank_map64(const uint32_t* hist, int lane, int lo
       ++above;
     }
   map[lane] = word;
-  return __shfl((int)incl, 0, 64);
+  return (int)total;
 }
 
 // hist[bin] += 1 for the active lanes of a wave, one LDS atomic per distinct bin
@@ -283,12 +287,7 @@ __device__ __forceinline__ void radix_pass_desc(const uint32_t* src, uint32_t* d
       cnt[i][w] = scans ? wr[w * 256 + kQ * tt + i] : 0u;
       loc += cnt[i][w];
     }
-  uint32_t incl = loc;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t o = (uint32_t)__shfl_up((int)incl, off, 64);
-    if (lane >= off) incl += o;
-  }
+  const uint32_t incl = wave_scan(loc);
   if (lane == 63 && scans) wt[wv] = incl;
   __syncthreads();
   if (scans) {
@@ -469,32 +468,61 @@ __global__ __launch_bounds__(512) void ix_wide_kernel(WideParams p) {
   const int64_t row_bt = (int64_t)b * p.S + (tok_ok ? t : 0);
   uint16_t* mykeys = keys + tl * p.tpad;
 
-  // Q fragments (A operand): row col -> head hq; channels 16ks + 8hf .. +7, RoPE'd on the fly.
+  // Tile copies: wave wi moves unit wi (rows 4wi .. 4wi+3 of the tile).
+  const i32x4 rsrc = make_rsrc(p.kv + (int64_t)b * p.kvbs, (uint32_t)p.T * (uint32_t)(kWD * 2));
+  const uint32_t ring_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) u32x4*)ring;
+  const int wis = __builtin_amdgcn_readfirstlane(wi);
+  const int urow = 4 * wis + (lane >> 4);
+  const uint32_t uoff = 16u * (uint32_t)((lane & 15) ^ (urow & 15));
+  const uint32_t ulds = ring_lds + 1024u * (uint32_t)wis;
+  auto issue = [&](int n) {
+    lds_dma16(rsrc, (uint32_t)(kTileC * (nbase + n) + urow) * (uint32_t)(kWD * 2) + uoff,
+              ulds + 8192u * (uint32_t)(n % kRingW));
+  };
+#pragma unroll
+  for (int j = 0; j < kRingW - 1; ++j)
+    if (j < ntiles) issue(j);
+
+  // Q fragments (A operand): row col -> head hq; channels 16ks + 8hf .. +7, RoPE'd on the
+  // fly. The rows' loads are in flight while the 4 tokens' table rows (rd / 2 complex each)
+  // go to LDS, one load per thread, so the rotation waits for one memory latency in all (read
+  // pair by pair from memory it took 2.5 us of a decode step).
   const int hq = head_of_row<KY>(col, y);
   bf16x8 qa[8];
   {
     const uint16_t* qrow = p.q + (row_bt * kWH + hq) * kWD + 8 * hf;
     const int half_rd = p.rd >> 1;
     const int rbase = kWD - p.rd;
+    u32x4 v[8];
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-      u32x4 v = tok_ok ? *reinterpret_cast<const u32x4*>(qrow + 16 * ks) : u32x4{0u, 0u, 0u, 0u};
-      if (p.freqs != nullptr && tok_ok) {
+    for (int ks = 0; ks < 8; ++ks) v[ks] = *reinterpret_cast<const u32x4*>(qrow + 16 * ks);
+    if (p.freqs != nullptr) {
+      float2* tab = reinterpret_cast<float2*>(hist);  // [kTok][rd / 2], at most 2 KB of the 8 KB
+      const int rows = min(kTok, p.S - t0);
+      const float2* src = reinterpret_cast<const float2*>(p.freqs) + (int64_t)t0 * half_rd;
+      for (int i = tid; i < rows * half_rd; i += 512) tab[i] = src[i];
+      __syncthreads();
+      const float2* mytab = tab + (tok_ok ? tl : 0) * half_rd;
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks) {
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
           const int d0 = 16 * ks + 8 * hf + 2 * w;
           if (d0 >= rbase) {
             const int pj = (d0 - rbase) >> 1;
             const int64_t n = (row_bt * kWH + hq) * half_rd + pj;
-            const float c = p.freqs[((int64_t)t * half_rd + pj) * 2];
-            const float d = p.freqs[((int64_t)t * half_rd + pj) * 2 + 1];
+            const float2 cd = mytab[pj];
             float re, im;
-            rope_pair(bf_lo(v[w]), bf_hi(v[w]), c, d, p.rope_mode, n, re, im);
-            v[w] = pack_bf2(re, im);
+            rope_pair(bf_lo(v[ks][w]), bf_hi(v[ks][w]), cd.x, cd.y, p.rope_mode, n, re, im);
+            v[ks][w] = pack_bf2(re, im);
           }
         }
       }
-      qa[ks] = __builtin_bit_cast(bf16x8, v);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      if (!tok_ok) v[ks] = u32x4{0u, 0u, 0u, 0u};
+      qa[ks] = __builtin_bit_cast(bf16x8, v[ks]);
     }
   }
   // Head weights of the lane's 16 heads (bf16 bits): wlo[m] = w of register 2m's head
@@ -511,20 +539,6 @@ __global__ __launch_bounds__(512) void ix_wide_kernel(WideParams p) {
     whi[m] = w1 << 16;
   }
 
-  // Tile copies: wave wi moves unit wi (rows 4wi .. 4wi+3 of the tile).
-  const i32x4 rsrc = make_rsrc(p.kv + (int64_t)b * p.kvbs, (uint32_t)p.T * (uint32_t)(kWD * 2));
-  const uint32_t ring_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) u32x4*)ring;
-  const int wis = __builtin_amdgcn_readfirstlane(wi);
-  const int urow = 4 * wis + (lane >> 4);
-  const uint32_t uoff = 16u * (uint32_t)((lane & 15) ^ (urow & 15));
-  const uint32_t ulds = ring_lds + 1024u * (uint32_t)wis;
-  auto issue = [&](int n) {
-    lds_dma16(rsrc, (uint32_t)(kTileC * (nbase + n) + urow) * (uint32_t)(kWD * 2) + uoff,
-              ulds + 8192u * (uint32_t)(n % kRingW));
-  };
-#pragma unroll
-  for (int j = 0; j < kRingW - 1; ++j)
-    if (j < ntiles) issue(j);
   // Consume the compiler-tracked loads here (their vmcnt(0) also covers the copies).
 #pragma unroll
   for (int ks = 0; ks < 8; ++ks) asm volatile("" ::"v"(qa[ks]));
@@ -804,17 +818,12 @@ __global__ __launch_bounds__(NT) void ix_select_kernel(SelParams p) {
       const uint32_t u = key_of(e);
       cnt += (u > kth ? 1u : 0u) + (u == kth_e ? 0x10000u : 0u);
     }
-    incl = cnt;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t o = (uint32_t)__shfl_up((int)incl, off, 64);
-      if (lane >= off) incl += o;
-    }
+    incl = wave_scan(cnt);
   }
   if (lane == 63) wt[wv] = incl;
   __syncthreads();
-  uint32_t base = incl - cnt;
-  for (int w = 0; w < wv; ++w) base += wt[w];
+  // The lower waves' total: one read and a scan (NW <= 16 lanes hold a wave's total each).
+  uint32_t base = incl - cnt + last_lane(wave_scan(lane < wv ? wt[lane] : 0u));
   uint32_t og = base & 0xffffu, oe = n_gt + (base >> 16);  // next slots of each kind
   const uint32_t oe_end = n_gt + need_eq;
   const uint32_t ibase = 0xffffu - (uint32_t)c0;
