@@ -44,6 +44,7 @@ EXPORTS = (
     "dsa_indexer_projections",
     "dsa_indexer_projections_splitk",
     "dsa_indexer_decode_projections",
+    "dsa_indexer_decode_projections_rope",
 )
 
 _c_i64 = ctypes.c_int64
@@ -140,6 +141,10 @@ def load() -> ctypes.CDLL:
     lib.dsa_indexer_decode_projections.restype = ctypes.c_int
     lib.dsa_indexer_decode_projections.argtypes = [
         _c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp]
+    lib.dsa_indexer_decode_projections_rope.restype = ctypes.c_int
+    lib.dsa_indexer_decode_projections_rope.argtypes = [
+        _c_vp, _c_vp, _c_vp, ctypes.c_int32, _c_vp, _c_vp, _c_vp, _c_vp,
+        _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp]
     v = lib.dsa_abi_version()
     if v != ABI_VERSION:
         raise RuntimeError(f"{path}: ABI version {v}, expected {ABI_VERSION}")
@@ -547,16 +552,19 @@ def indexer_projections(qr: torch.Tensor, wq_packed: torch.Tensor, freqs_cis: Op
     return q, wl
 
 
-#: argument slots of the two outputs of dsa_indexer_decode_projections
-DECODE_SLOT_Q = 4
-DECODE_SLOT_WL = 5
+#: argument slots of the two outputs of dsa_indexer_decode_projections_rope
+DECODE_SLOT_Q = 6
+DECODE_SLOT_WL = 7
 
 
-def prepare_indexer_decode_projections(qr: torch.Tensor, wq: torch.Tensor, x: torch.Tensor, wproj: torch.Tensor):
-    """Checks and marshals dsa_indexer_decode_projections; returns (Launch, q_shape,
+def prepare_indexer_decode_projections(qr: torch.Tensor, wq: torch.Tensor, x: torch.Tensor, wproj: torch.Tensor,
+                                       freqs_cis: Optional[torch.Tensor] = None, head_dim: int = 0,
+                                       rope_head_dim: int = 0, rope_mode: int = DSA_ROPE_TORCH_ROCM):
+    """Checks and marshals dsa_indexer_decode_projections_rope; returns (Launch, q_shape,
     wl_shape, keep) with the outputs in the argument slots DECODE_SLOT_Q / DECODE_SLOT_WL.
     qr: bf16 [b, s, 1536], x: bf16 [b, s, 7168] with b * s <= 16; wq [n_q, 1536] and
-    wproj [n_w, 7168] the Linear weights as they are."""
+    wproj [n_w, 7168] the Linear weights as they are; freqs_cis: rows for the s positions
+    (None: q without RoPE)."""
     load()
     if qr.dim() != 3 or x.dim() != 3 or qr.shape[:2] != x.shape[:2]:
         raise ValueError(f"qr {tuple(qr.shape)} and x {tuple(x.shape)} do not match")
@@ -567,18 +575,24 @@ def prepare_indexer_decode_projections(qr: torch.Tensor, wq: torch.Tensor, x: to
             raise TypeError("qr, x and both weights must be bfloat16")
     b, s, k_q = qr.shape
     k_w = x.shape[2]
+    fr = _freqs_view(freqs_cis, s, rope_head_dim) if freqs_cis is not None else None
     qr, x, wq, wproj = qr.contiguous(), x.contiguous(), wq.contiguous(), wproj.contiguous()
-    dev = _require_gpu(qr, x, wq, wproj)
-    args = [qr.data_ptr(), wq.data_ptr(), x.data_ptr(), wproj.data_ptr(), None, None,
-            b * s, wq.shape[0], k_q, wproj.shape[0], k_w, stream_handle(dev)]
-    return (Launch("dsa_indexer_decode_projections", args), (b, s, wq.shape[0]), (b, s, wproj.shape[0]),
-            (qr, x, wq, wproj))
+    dev = _require_gpu(qr, x, wq, wproj, *([fr] if fr is not None else []))
+    args = [qr.data_ptr(), wq.data_ptr(), fr.data_ptr() if fr is not None else None, int(rope_mode),
+            x.data_ptr(), wproj.data_ptr(), None, None,
+            b * s, wq.shape[0], k_q, wproj.shape[0], k_w, head_dim, rope_head_dim, max(s, 1), stream_handle(dev)]
+    return (Launch("dsa_indexer_decode_projections_rope", args), (b, s, wq.shape[0]), (b, s, wproj.shape[0]),
+            (qr, x, wq, wproj, fr))
 
 
-def indexer_decode_projections(qr: torch.Tensor, wq: torch.Tensor, x: torch.Tensor, wproj: torch.Tensor):
+def indexer_decode_projections(qr: torch.Tensor, wq: torch.Tensor, x: torch.Tensor, wproj: torch.Tensor,
+                               freqs_cis: Optional[torch.Tensor] = None, head_dim: int = 0, rope_head_dim: int = 0,
+                               rope_mode: int = DSA_ROPE_TORCH_ROCM):
     """q = qr . wq^T as bf16 [b, s, n_q] and wl = x . wproj^T as bf16 [b, s, n_w] for
-    b * s <= 16 tokens, in hipBLASLt's local-split rounding (no RoPE)."""
-    launch, q_shape, wl_shape, _keep = prepare_indexer_decode_projections(qr, wq, x, wproj)
+    b * s <= 16 tokens, in hipBLASLt's local-split rounding; with freqs_cis, RoPE on the last
+    rope_head_dim channels of every head_dim of q."""
+    launch, q_shape, wl_shape, _keep = prepare_indexer_decode_projections(qr, wq, x, wproj, freqs_cis, head_dim,
+                                                                          rope_head_dim, rope_mode)
     q = torch.empty(q_shape, dtype=torch.bfloat16, device=qr.device)
     wl = torch.empty(wl_shape, dtype=torch.bfloat16, device=qr.device)
     launch.set(DECODE_SLOT_Q, q.data_ptr())

@@ -2,7 +2,7 @@
 // tokens (1..16) in one launch, at the DeepSeek-V3.2 indexer shapes (q_lora_rank
 // 1536, dim 7168). These are the two F.linear calls of the indexer's forward,
 // reference/task2_v0_ref.py:129 (q) and :132 (weights), through Linear.forward
-// :81-83; RoPE stays with the score kernel as on the F.linear route.
+// :81-83, with apply_rotary_emb (:131) on the rounded q where the caller gives the table.
 //
 // Rounding reproduced: torch-ROCm runs both products through hipBLASLt, which
 // for 1..16 tokens at these shapes picks a kernel with a local split of the
@@ -25,7 +25,10 @@
 //    them, with the tokens' x rows, through LDS in 4 phases of 2048 k; waves
 //    0..3 run the 4 chains from LDS.
 //
-// The wl workgroups come first in the grid, so they start before the q ones.
+// The wl workgroups come first in the grid, so they start before the q ones. The weights
+// are read with plain loads: non-temporal ones bypass what the MALL holds of them (16
+// tokens 13.8 -> 9.7 us with one layer's weights, 14.2 -> 10.0 with four layers' in turn).
+// Up to 4 tokens take a finer work split (ix_decode_proj_few_kernel).
 #include "dsa_common.h"
 
 using namespace dsa;
@@ -56,23 +59,63 @@ struct DecodeProjParams {
   const uint16_t* wp;   // [n_w, 7168]
   uint16_t* q;          // [m, n_q]
   uint16_t* wl;         // [m, n_w]
+  const float* freqs;   // [S, rd/2, 2] RoPE table rows, or nullptr: no RoPE
   int32_t m, n_q, n_w, wl_blocks;
+  int32_t D, rd, S, mode;  // head dim, rotated channels, tokens per sequence, rounding
 };
 
 __device__ __forceinline__ float add_rn(float a, float b) { return __fadd_rn(a, b); }
 
 // Element t (0..255) of a 16-channel x 16-token tile whose four chains are f32x4
 // lanes of red[w0 .. w0+3][64]: lane t/4, register t%4 -> token lane%16, channel
-// 4*(lane/16) + t%4. Sums the chains in order and stores bf16 for tokens < m.
-__device__ __forceinline__ void reduce_store(const f32x4* red, int w0, int t, int m, uint16_t* out,
-                                             int n, int n0) {
+// 4*(lane/16) + t%4.
+__device__ __forceinline__ int elem_tok(int t) { return (t >> 2) & 15; }
+__device__ __forceinline__ int elem_row(int t) { return 4 * (t >> 6) + (t & 3); }
+
+// Sums the chains of element t in order and rounds once to bf16.
+__device__ __forceinline__ uint16_t chain_sum(const f32x4* red, int w0, int t) {
   const int lane = t >> 2, r = t & 3;
   const float* f = reinterpret_cast<const float*>(red);
-  const float s = add_rn(add_rn(add_rn(f[(w0 * 64 + lane) * 4 + r], f[((w0 + 1) * 64 + lane) * 4 + r]),
-                                f[((w0 + 2) * 64 + lane) * 4 + r]),
-                         f[((w0 + 3) * 64 + lane) * 4 + r]);
-  const int col = lane & 15, row = 4 * (lane >> 4) + r;
-  if (col < m) out[(int64_t)col * n + n0 + row] = f2bf(s);
+  return f2bf(add_rn(add_rn(add_rn(f[(w0 * 64 + lane) * 4 + r], f[((w0 + 1) * 64 + lane) * 4 + r]),
+                            f[((w0 + 2) * 64 + lane) * 4 + r]),
+                     f[((w0 + 3) * 64 + lane) * 4 + r]));
+}
+
+// q's element t of the tile at channel n0: its RoPE table entry (read early, beside the
+// weights), and the store, rotated with the neighbour thread's channel of the pair. Doing it
+// here takes one element per thread; the score kernel's prologue, 16 pairs per lane, made a
+// decode step 1.9 us longer.
+struct RopeElem {
+  float2 cs;
+  int pj;  // complex index within the head, or -1: not rotated
+};
+__device__ __forceinline__ RopeElem rope_elem(const DecodeProjParams& p, int t, int n0) {
+  RopeElem e = {float2{1.f, 0.f}, -1};
+  if (p.freqs != nullptr) {
+    const int d = (n0 + elem_row(t)) % p.D - (p.D - p.rd);
+    if (d >= 0) {
+      e.pj = d >> 1;
+      const int tok = min(elem_tok(t), p.m - 1);
+      e.cs = reinterpret_cast<const float2*>(p.freqs)[(int64_t)(tok % p.S) * (p.rd >> 1) + e.pj];
+    }
+  }
+  return e;
+}
+__device__ __forceinline__ void store_q(const DecodeProjParams& p, const f32x4* red, int w0, int t, int n0,
+                                        const RopeElem& e) {
+  uint16_t h = chain_sum(red, w0, t);
+  const int tok = elem_tok(t), ch = n0 + elem_row(t);
+  if (p.freqs != nullptr) {
+    const uint16_t o = (uint16_t)__builtin_amdgcn_mov_dpp((int)h, 0xB1, 0xF, 0xF, false);  // the pair's other channel
+    if (e.pj >= 0) {
+      const bool im_ch = (t & 1) != 0;
+      float re, im;
+      rope_pair(bf2f(im_ch ? o : h), bf2f(im_ch ? h : o), e.cs.x, e.cs.y, p.mode,
+                ((int64_t)tok * (p.n_q / p.D) + ch / p.D) * (p.rd >> 1) + e.pj, re, im);
+      h = f2bf(im_ch ? im : re);
+    }
+  }
+  if (tok < p.m) p.q[(int64_t)tok * p.n_q + ch] = h;
 }
 
 __device__ void q_role(const DecodeProjParams& p, int blk, uint8_t* smem) {
@@ -85,12 +128,15 @@ __device__ void q_role(const DecodeProjParams& p, int blk, uint8_t* smem) {
   const u32x4* wa0 = reinterpret_cast<const u32x4*>(p.wq + (int64_t)(nb + r16) * kQK + koff);
   const u32x4* wa1 = reinterpret_cast<const u32x4*>(p.wq + (int64_t)(nb + 16 + r16) * kQK + koff);
   const u32x4* xb = reinterpret_cast<const u32x4*>(p.qr + (int64_t)tok * kQK + koff);
+  RopeElem re[2];  // of the two elements this thread stores
+#pragma unroll
+  for (int i = 0; i < 2; ++i) re[i] = rope_elem(p, tid & 255, blk * kQRows + ((tid + i * kThreads) >> 8) * 16);
   u32x4 a0[kQSteps], a1[kQSteps], b[kQSteps];
 #pragma unroll
   for (int s = 0; s < kQSteps; ++s) {
     b[s] = xb[s * (kQDepth / 8)];
-    a0[s] = ld_nt(wa0 + s * (kQDepth / 8));
-    a1[s] = ld_nt(wa1 + s * (kQDepth / 8));
+    a0[s] = wa0[s * (kQDepth / 8)];
+    a1[s] = wa1[s * (kQDepth / 8)];
   }
   // All 36 loads in flight before the first product (the scheduler would otherwise
   // interleave them with the chains and keep fewer outstanding).
@@ -110,7 +156,7 @@ __device__ void q_role(const DecodeProjParams& p, int blk, uint8_t* smem) {
   for (int i = 0; i < 2; ++i) {
     const int e = tid + i * kThreads;  // 4 row groups x 256 elements
     const int rgp = e >> 8;
-    reduce_store(red, rgp * 4, e & 255, p.m, p.q, p.n_q, blk * kQRows + rgp * 16);
+    store_q(p, red, rgp * 4, e & 255, blk * kQRows + rgp * 16, re[i]);
   }
 }
 
@@ -124,7 +170,7 @@ __device__ __forceinline__ void load_w(u32x4 (&r)[2 * NB], const uint16_t* wp, i
 #pragma unroll
   for (int i = 0; i < 2 * NB; ++i) {
     const int j = tid + i * kThreads;
-    r[i] = ld_nt(reinterpret_cast<const u32x4*>(wp + (int64_t)(n0 + j / kRow) * kWK + ph * 2048 + (j % kRow) * 8));
+    r[i] = *reinterpret_cast<const u32x4*>(wp + (int64_t)(n0 + j / kRow) * kWK + ph * 2048 + (j % kRow) * 8);
   }
 }
 template <int NB>
@@ -208,7 +254,123 @@ __device__ void wl_role(const DecodeProjParams& p, int blk, uint8_t* smem) {
   f32x4* red = reinterpret_cast<f32x4*>(smem);
   if (wave < kSplit) red[wave * 64 + lane] = acc;
   __syncthreads();
-  if (tid < 256) reduce_store(red, 0, tid, p.m, p.wl, p.n_w, n0);
+  if (tid < 256 && elem_tok(tid) < p.m)
+    p.wl[(int64_t)elem_tok(tid) * p.n_w + n0 + elem_row(tid)] = chain_sum(red, 0, tid);
+}
+
+// Up to 4 tokens: the same chains and sums with the bytes spread evenly over the CUs. A q
+// workgroup covers 32 channels (wave w: chain w % 4 of row group w / 4, 12 weight and 12 qr
+// fragments in flight), and a wl workgroup 4 channels (57 KB of weight rows and the tokens'
+// x rows, all in flight at once, staged through LDS in 2 phases of 7 depth blocks; its matrix
+// rows 4..15 repeat rows 0..3 and are not stored). Every workgroup then waits for about 100
+// KB instead of 196-229 KB, and with 57 KB of LDS and 128 VGPRs two fit on a CU, so the 272
+// workgroups run at once. More than 4 tokens would put 16 x 14 KB per token of x beside
+// that, which the 16-channel workgroups above read once. 1 token: 10.9 us with the split
+// above, 8.0 with this one, 5.8 with plain loads (7.0 with four layers' weights in turn:
+// 26 MB at 5.8 TB/s with the launch); hipBLASLt's two kernels 8.7 + 8.5.
+constexpr int kFewTok = 4;
+constexpr int kFewQRows = 32;                          // q channels per workgroup
+constexpr int kFewWRows = 4;                           // wl channels per workgroup
+constexpr int kFewBlocks = 7;                          // depth blocks per phase
+constexpr int kFewChunks = kFewBlocks * kWDepth * 2 / 16;  // 448 chunks of 16 B per row and phase
+constexpr int kFewPitch = kFewChunks * 16 + 16;
+constexpr int kFewLoads = (4 * kFewChunks + kThreads - 1) / kThreads;  // 4 per lane (the last one partly)
+static_assert(kWK == 2 * kFewBlocks * kWDepth, "wl phases");
+
+__device__ void few_q_role(const DecodeProjParams& p, int blk, uint8_t* smem) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int c = wave & 3, rg = wave >> 2;  // chain, row group
+  const int r16 = lane & 15, g = lane >> 4;
+  const int tok = min(r16, p.m - 1);  // columns >= m compute on a valid row and are not stored
+  const int koff = c * (kQDepth / 4) + g * 8;
+  const u32x4* wa = reinterpret_cast<const u32x4*>(p.wq + (int64_t)(blk * kFewQRows + rg * 16 + r16) * kQK + koff);
+  const u32x4* xb = reinterpret_cast<const u32x4*>(p.qr + (int64_t)tok * kQK + koff);
+  const RopeElem re = rope_elem(p, tid & 255, blk * kFewQRows + 16 * (tid >> 8));
+  u32x4 a[kQSteps], b[kQSteps];
+#pragma unroll
+  for (int s = 0; s < kQSteps; ++s) {
+    a[s] = wa[s * (kQDepth / 8)];
+    b[s] = xb[s * (kQDepth / 8)];
+  }
+  __builtin_amdgcn_sched_barrier(0);  // every load in flight before the first product
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < kQSteps; ++s)
+    acc = mfma16x16x32(__builtin_bit_cast(bf16x8, a[s]), __builtin_bit_cast(bf16x8, b[s]), acc);
+  f32x4* red = reinterpret_cast<f32x4*>(smem);
+  red[wave * 64 + lane] = acc;  // [row group][chain][lane]
+  __syncthreads();
+  store_q(p, red, 4 * (tid >> 8), tid & 255, blk * kFewQRows + 16 * (tid >> 8), re);
+}
+
+__device__ void few_wl_role(const DecodeProjParams& p, int blk, uint8_t* smem) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n0 = blk * kFewWRows;
+  u32x4 w[2][kFewLoads], x[2][kFewLoads];
+#pragma unroll
+  for (int ph = 0; ph < 2; ++ph)
+#pragma unroll
+    for (int i = 0; i < kFewLoads; ++i) {
+      const int j = tid + i * kThreads, row = j / kFewChunks, ch = j % kFewChunks;
+      const int64_t at = ph * (kFewChunks * 8) + ch * 8;
+      if (row < kFewWRows) w[ph][i] = *reinterpret_cast<const u32x4*>(p.wp + (int64_t)(n0 + row) * kWK + at);
+      if (row < p.m) x[ph][i] = *reinterpret_cast<const u32x4*>(p.x + (int64_t)row * kWK + at);
+    }
+  uint8_t* wt = smem;
+  uint8_t* xt = smem + kFewWRows * kFewPitch;
+  const int r4 = lane & 3, g = lane >> 4;  // W row; token (rows >= m hold stale data, their columns are not stored)
+  const uint8_t* wa = wt + r4 * kFewPitch + (wave * (kWDepth / kSplit) + g * 8) * 2;
+  const uint8_t* xa = xt + r4 * kFewPitch + (wave * (kWDepth / kSplit) + g * 8) * 2;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ph = 0; ph < 2; ++ph) {
+#pragma unroll
+    for (int i = 0; i < kFewLoads; ++i) {
+      const int j = tid + i * kThreads, row = j / kFewChunks, ch = j % kFewChunks;
+      if (row < kFewWRows) *reinterpret_cast<u32x4*>(wt + row * kFewPitch + ch * 16) = w[ph][i];
+      if (row < p.m) *reinterpret_cast<u32x4*>(xt + row * kFewPitch + ch * 16) = x[ph][i];
+    }
+    __syncthreads();
+    if (wave < kSplit) {
+      // Chain c = wave: step t (= 4 d + s) is k = d * 512 + c * 128 + s * 32 of the phase;
+      // the fragments of step t + 3 are read while step t's product runs.
+      constexpr int kSteps = 4 * kFewBlocks;
+      auto at = [](int t) { return (t >> 2) * kWDepth * 2 + (t & 3) * 64; };
+      u32x4 fa[4], fb[4];
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        fa[t] = *reinterpret_cast<const u32x4*>(wa + at(t));
+        fb[t] = *reinterpret_cast<const u32x4*>(xa + at(t));
+      }
+#pragma unroll
+      for (int t = 0; t < kSteps; ++t) {
+        if (t + 3 < kSteps) {
+          fa[(t + 3) % 4] = *reinterpret_cast<const u32x4*>(wa + at(t + 3));
+          fb[(t + 3) % 4] = *reinterpret_cast<const u32x4*>(xa + at(t + 3));
+        }
+        __builtin_amdgcn_sched_barrier(0);  // keep the read-ahead ahead of the product
+        acc = mfma16x16x32(__builtin_bit_cast(bf16x8, fa[t % 4]), __builtin_bit_cast(bf16x8, fb[t % 4]), acc);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();
+  }
+  // Rows 0..3 of the product sit in lanes 0..15 (token lane, channel n0 + register).
+  f32x4* red = reinterpret_cast<f32x4*>(smem);
+  if (wave < kSplit) red[wave * 64 + lane] = acc;
+  __syncthreads();
+  const int col = tid >> 2, r = tid & 3;
+  if (col < p.m) {
+    const float s = add_rn(add_rn(add_rn(red[col][r], red[64 + col][r]), red[128 + col][r]), red[192 + col][r]);
+    p.wl[(int64_t)col * p.n_w + n0 + r] = f2bf(s);
+  }
+}
+
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void ix_decode_proj_few_kernel(
+    DecodeProjParams p) {
+  __shared__ __align__(16) uint8_t smem[2 * kFewWRows * kFewPitch];
+  if ((int)blockIdx.x < p.wl_blocks) few_wl_role(p, blockIdx.x, smem);
+  else few_q_role(p, blockIdx.x - p.wl_blocks, smem);
 }
 
 __global__ __launch_bounds__(kThreads) void ix_decode_proj_kernel(DecodeProjParams p) {
@@ -219,17 +381,27 @@ __global__ __launch_bounds__(kThreads) void ix_decode_proj_kernel(DecodeProjPara
 
 }  // namespace
 
-extern "C" int dsa_indexer_decode_projections(const void* qr, const void* wq, const void* x, const void* wproj,
-                                              void* q, void* wl, int64_t m, int64_t n_q, int64_t k_q,
-                                              int64_t n_w, int64_t k_w, void* stream) {
+namespace {
+
+// Both decode entry points (freqs_cis nullptr: without RoPE).
+int decode_projections(const void* qr, const void* wq, const void* freqs_cis, int32_t rope_mode, const void* x,
+                       const void* wproj, void* q, void* wl, int64_t m, int64_t n_q, int64_t k_q, int64_t n_w,
+                       int64_t k_w, int64_t head_dim, int64_t rd, int64_t s_len, void* stream) {
   if (m < 0 || n_q <= 0 || k_q <= 0 || n_w <= 0 || k_w <= 0) return DSA_ERR_SHAPE;
   if (m > 16 || k_q != kQK || k_w != kWK || n_q % kQRows != 0 || n_w % 16 != 0 || n_q > (1 << 20) ||
       n_w > (1 << 16))
     return DSA_ERR_UNSUPPORTED;
+  if (freqs_cis != nullptr) {
+    if (head_dim <= 0 || n_q % head_dim != 0 || rd <= 0 || rd > head_dim || (rd & 1) || (head_dim & 1) ||
+        s_len <= 0 || m % s_len != 0)
+      return DSA_ERR_SHAPE;
+    if (rope_mode != DSA_ROPE_CPU && rope_mode != DSA_ROPE_TORCH_ROCM) return DSA_ERR_UNSUPPORTED;
+  }
   if (m == 0) return DSA_OK;
   if (!qr || !wq || !x || !wproj || !q || !wl) return DSA_ERR_NULL;
   if (!dsa_host::aligned16(qr) || !dsa_host::aligned16(wq) || !dsa_host::aligned16(x) ||
-      !dsa_host::aligned16(wproj) || ((uintptr_t)q & 1u) || ((uintptr_t)wl & 1u))
+      !dsa_host::aligned16(wproj) || ((uintptr_t)q & 1u) || ((uintptr_t)wl & 1u) ||
+      ((uintptr_t)freqs_cis & 7u))
     return DSA_ERR_ALIGN;
   DecodeProjParams p;
   p.qr = (const uint16_t*)qr;
@@ -238,11 +410,39 @@ extern "C" int dsa_indexer_decode_projections(const void* qr, const void* wq, co
   p.wp = (const uint16_t*)wproj;
   p.q = (uint16_t*)q;
   p.wl = (uint16_t*)wl;
+  p.freqs = (const float*)freqs_cis;
+  p.D = (int32_t)head_dim;
+  p.rd = (int32_t)rd;
+  p.S = (int32_t)s_len;
+  p.mode = rope_mode;
   p.m = (int32_t)m;
   p.n_q = (int32_t)n_q;
   p.n_w = (int32_t)n_w;
+  if (m <= kFewTok) {
+    p.wl_blocks = (int32_t)(n_w / kFewWRows);
+    const unsigned grid = (unsigned)(p.wl_blocks + n_q / kFewQRows);
+    hipLaunchKernelGGL(ix_decode_proj_few_kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, p);
+    return hipGetLastError() == hipSuccess ? DSA_OK : DSA_ERR_LAUNCH;
+  }
   p.wl_blocks = (int32_t)(n_w / 16);
   const unsigned grid = (unsigned)(p.wl_blocks + n_q / kQRows);
   hipLaunchKernelGGL(ix_decode_proj_kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, p);
   return hipGetLastError() == hipSuccess ? DSA_OK : DSA_ERR_LAUNCH;
+}
+
+}  // namespace
+
+extern "C" int dsa_indexer_decode_projections(const void* qr, const void* wq, const void* x, const void* wproj,
+                                              void* q, void* wl, int64_t m, int64_t n_q, int64_t k_q,
+                                              int64_t n_w, int64_t k_w, void* stream) {
+  return decode_projections(qr, wq, nullptr, 0, x, wproj, q, wl, m, n_q, k_q, n_w, k_w, 0, 0, 0, stream);
+}
+
+extern "C" int dsa_indexer_decode_projections_rope(const void* qr, const void* wq, const void* freqs_cis,
+                                                   int32_t rope_mode, const void* x, const void* wproj, void* q,
+                                                   void* wl, int64_t m, int64_t n_q, int64_t k_q, int64_t n_w,
+                                                   int64_t k_w, int64_t head_dim, int64_t rd, int64_t s_len,
+                                                   void* stream) {
+  return decode_projections(qr, wq, freqs_cis, rope_mode, x, wproj, q, wl, m, n_q, k_q, n_w, k_w, head_dim, rd,
+                            s_len, stream);
 }

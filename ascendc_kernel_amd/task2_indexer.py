@@ -13,8 +13,8 @@ relu-weighted head sum, the causal mask and the top-k (``dsa_indexer_score_topk`
 The projections run as one kernel launch (``dsa_indexer_projections`` or, in the order
 of hipBLASLt's split k, ``dsa_indexer_projections_splitk``: q with RoPE, and the head
 weights), as the query-projection kernel beside ``F.linear``, as one decode launch for
-1..16 tokens (``dsa_indexer_decode_projections``, both products in hipBLASLt's split-k
-order; the score kernel applies RoPE), or as two ``F.linear`` (the reference's own op; the
+1..16 tokens (``dsa_indexer_decode_projections_rope``, both products in hipBLASLt's
+split-k order), or as two ``F.linear`` (the reference's own op; the
 score kernel then applies RoPE), whichever ``splitk_route`` and ``projection_route`` pick:
 a kernel only where its rounding was measured equal to ``F.linear`` on this torch-ROCm
 build. Inputs must be on the HIP device;
@@ -185,8 +185,7 @@ def projection_route(m: int, q_lora_rank: int, rope_head_dim: int, head_dim: int
     """Which path computes the two projections of Model.forward for m = b * s tokens:
     'both'  one launch of dsa_indexer_projections (q with RoPE, and weights_proj);
     'q'     dsa_indexer_q_proj for q with RoPE, F.linear for weights_proj;
-    'decode' one launch of dsa_indexer_decode_projections for both (no RoPE: the score
-            kernel applies it);
+    'decode' one launch of dsa_indexer_decode_projections_rope for both (q with RoPE);
     'torch' F.linear for both (the score kernel then applies RoPE).
     A kernel is used only where its rounding was measured equal to F.linear."""
     if not (bf16 and on_gpu and build_ok):
@@ -337,15 +336,15 @@ class _IndexerPlan:
                 self.proj.set(_native.PROJ_SLOT_Q, q.data_ptr())
                 self.proj.set(_native.PROJ_SLOT_WL, wl.data_ptr())
         elif self.route == "decode":
-            # q = qr . wq_b^T and wl = x . weights_proj^T in one launch, in hipBLASLt's
-            # rounding at decode sizes (task2_v0_ref.py:129,132); RoPE in the score kernel.
+            # q = RoPE(qr . wq_b^T) and wl = x . weights_proj^T in one launch, in hipBLASLt's
+            # rounding at decode sizes (task2_v0_ref.py:129-132).
             self.proj, _q_shape, wl_shape, self.proj_keep = _native.prepare_indexer_decode_projections(
-                qr, self.wq, x, self.wp)
+                qr, self.wq, x, self.wp, freqs, hd, rd, mode)
             self.q = torch.empty(bsz, seqlen, model.n_local_heads, hd, dtype=torch.bfloat16, device=x.device)
             self.wl = torch.empty(wl_shape, dtype=torch.bfloat16, device=x.device)
             self.proj.set(_native.DECODE_SLOT_Q, self.q.data_ptr())
             self.proj.set(_native.DECODE_SLOT_WL, self.wl.data_ptr())
-            self.score = _native.prepare_indexer_score_topk(self.q, kv, self.wl, w_scale, freqs, **score_kw)
+            self.score = _native.prepare_indexer_score_topk(self.q, kv, self.wl, w_scale, None, **score_kw)
         elif self.route == "q":
             # q = RoPE(qr . wq_b^T) by dsa_indexer_q_proj; weights_proj stays F.linear.
             prep = _native.prepare_indexer_q_proj(qr, self.wq, freqs, hd, rd, mode)

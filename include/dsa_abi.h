@@ -368,6 +368,19 @@ int dsa_indexer_decode_projections(const void* qr, const void* wq, const void* x
                                    void* q, void* wl, int64_t m, int64_t n_q, int64_t k_q, int64_t n_w,
                                    int64_t k_w, void* stream);
 
+/*
+ * dsa_indexer_decode_projections with apply_rotary_emb (reference/task2_v0_ref.py:131) on the
+ * last rd channels of every head of the rounded q (then pass a NULL table to the score call).
+ *   freqs_cis  complex64 [s_len, rd/2] rows of positions start_pos .. (8-byte aligned), or NULL
+ *   rope_mode  DSA_ROPE_TORCH_ROCM or DSA_ROPE_CPU
+ * n_q % head_dim == 0, rd even, 0 < rd <= head_dim, m % s_len == 0.
+ */
+int dsa_indexer_decode_projections_rope(const void* qr, const void* wq, const void* freqs_cis,
+                                        int32_t rope_mode, const void* x, const void* wproj, void* q,
+                                        void* wl, int64_t m, int64_t n_q, int64_t k_q, int64_t n_w,
+                                        int64_t k_w, int64_t head_dim, int64_t rd, int64_t s_len,
+                                        void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -324,3 +324,11 @@ def test_decode_projections_host_checks():
     for name in ("qr", "wq", "x", "wp", "q", "wl"):
         assert _dproj(lib, **{name: None}) == -1, name
     assert _dproj(lib, qr=8) == -6 and _dproj(lib, wp=24) == -6 and _dproj(lib, q=17) == -6
+
+
+def test_decode_projections_rope_host_checks():
+    lib = _native.load()
+    f = lambda m=4, d=128, rd=64, s=2, mode=1, fr=16, qr=16: lib.dsa_indexer_decode_projections_rope(
+        qr, 16, fr, mode, 16, 16, 16, 16, m, 8192, 1536, 64, 7168, d, rd, s, None)
+    assert f(m=5) == f(d=100) == f(rd=130) == f(rd=7) == f(s=0) == -2 and f(mode=3) == f(m=17) == -3
+    assert f(m=0) == 0 and f(qr=None) == -1 and f(fr=4) == f(qr=8) == -6

@@ -117,3 +117,22 @@ def test_model_decode_route(gpu):
         x = torch.zeros(1, s, KW, dtype=torch.bfloat16, device=gpu)
         qr = torch.zeros(1, s, KQ, dtype=torch.bfloat16, device=gpu)
         assert m.route(x, qr) == want, s
+
+
+@pytest.mark.parametrize("b,s", [(1, 1), (1, 4), (2, 2), (1, 5), (3, 5), (2, 8)])
+@pytest.mark.parametrize("mode", [_native.DSA_ROPE_TORCH_ROCM, _native.DSA_ROPE_CPU])
+def test_decode_projections_rope(gpu, b, s, mode):
+    """With the RoPE table the launch gives F.linear's q rotated by the standalone RoPE kernel
+    (which the rule tests hold to torch), on both sides of the 4-token work split, and the same
+    head weights."""
+    _require_measured_build(gpu)
+    g = torch.Generator(device=gpu).manual_seed(b * 10 + s)
+    wq, wp = _wide((NQ, KQ), g, gpu), _wide((NW, KW), g, gpu)
+    qr, x = _wide((b, s, KQ), g, gpu), _wide((b, s, KW), g, gpu)
+    fr = t2.precompute_freqs_cis(64, 100 + s, device=gpu)[100:]
+    _say("case rope", b, s, mode)
+    q, wl = _native.indexer_decode_projections(qr, wq, x, wp, fr, 128, 64, mode)
+    want = torch.nn.functional.linear(qr, wq).view(b, s, 64, 128)
+    _native.indexer_rope_(want, fr, 64, mode)
+    assert torch.equal(q.view(torch.int16), want.view(b, s, NQ).view(torch.int16))
+    assert torch.equal(wl.view(torch.int16), torch.nn.functional.linear(x, wp).view(torch.int16))
