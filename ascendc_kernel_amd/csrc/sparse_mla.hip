@@ -7,9 +7,9 @@
 // One workgroup per token, one wave per 16 heads (8 waves for 128 heads). Per
 // wave, Q^T (576 x 16 heads, 72 VGPRs) and O^T (512 x 16, fp32, 128 registers)
 // stay in registers. Slots go in blocks of 32: the 32 selected rows (1152 B each)
-// are copied by buffer_load ... lds into a ring of 4 LDS buffers, each row padded
-// to 73 chunks of 16 B so that one chunk read across 16 rows, and the transposed
-// reads of V, hit distinct banks. Per block and wave (mfma 16x16x32, lane l:
+// are copied by buffer_load ... lds into a ring of 4 LDS buffers, the chunks of 16 B
+// swizzled so that one chunk read across 16 rows, and the transposed reads of V, hit
+// distinct banks. Per block and wave (mfma 16x16x32, lane l:
 // head l%16, key / channel group g = l/16):
 //   S^T[2 x 16 keys x 16 heads] = K . Q^T                  (2 x 18 mfma)
 //   online softmax over the 32 keys of a head (held by the 4 lane groups, reduced
@@ -18,9 +18,16 @@
 // with the contraction over keys ordered so that each lane's 8 P values are the B
 // operand as they stand (keys 4g..4g+3 and 16+4g..16+4g+3 for lane group g).
 // The two waves of a SIMD overlap one's softmax with the other's products.
+//
+// Bound by the matrix cores (100 products per wave and block, 3,200 cycles of a SIMD's two
+// waves) and what the waves do between them. Copying whole rows with scalar addresses
+// instead of 64-chunk runs of padded rows with per-lane ones: 8192 tokens x 128 heads, top-
+// 2048 5086 -> 4750-4830 us (1.25 PFLOP/s of issued products), 300 tokens 338 -> 303 us, 1286
+// tokens x 64 heads 442 -> 390 us, the same bits.
 #include "dsa_common.h"
 
 #include <float.h>
+#include <type_traits>
 
 using namespace dsa;
 
@@ -31,10 +38,12 @@ constexpr int kDV = 512;                        // value channels
 constexpr int kKS = kDQK / 32;                  // 18 k-steps of the score product
 constexpr int kCT = kDV / 16;                   // 32 output tiles of 16 channels
 constexpr int kKB = 32;                         // slots per block
-constexpr int kRowC = kDQK / 8 + 1;             // LDS row: 72 chunks + 1 pad chunk
-constexpr int kBlkPos = kKB * kRowC;            // 2336 chunk positions per block
-constexpr int kUnitsBlk = (kBlkPos + 63) / 64;  // 37 copy units of 64 chunks
-constexpr int kBlkBytes = kUnitsBlk * 1024;     // 37888 B per buffer (copy tail included)
+// A block in LDS: 32 rows of their first 64 chunks (1 KB each, chunk c of row r at position
+// c ^ swz(r)), then the rows' last 8 chunks (128 B each, chunk 64 + c at c ^ (r/2 % 8)): 32
+// copy units of one row and 4 of eight rows' tails.
+constexpr int kTailOff = kKB * 1024;
+constexpr int kTails = 4;
+constexpr int kBlkBytes = kTailOff + kTails * 1024;  // 36864 B per buffer
 constexpr int kRingM = 4;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kRaise = 8.0f;
@@ -63,6 +72,13 @@ struct S2 {
   f32x4 t0, t1;
 };
 
+// Swizzle of row r's chunks: 16 distinct values over 16 rows (one chunk of 16 rows, a K
+// fragment, hits all banks), whose pairs are distinct over 8 rows (two chunks of 8 rows, half a
+// transposed V read).
+__device__ __forceinline__ int swz(int r) { return ((r & 7) << 1) | ((r >> 3) & 1); }
+
+typedef __attribute__((address_space(3))) const u32x4* lds_cu32x4_ptr;
+
 // kSplit: the token's slot blocks are divided among p.nsplit workgroups, each
 // writing its unnormalised partial state to p.part / p.ml (a separate
 // instantiation, so the one-pass kernel's code is unchanged by it).
@@ -70,7 +86,7 @@ template <int NW, typename IdxT, bool kSplit>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void sa_mla_kernel(MlaParams p) {
   const IdxT* const idx = static_cast<const IdxT*>(p.idx);
-  extern __shared__ __align__(16) uint8_t smem[];
+  extern __shared__ __align__(1024) uint8_t smem[];  // (fragment addresses are formed by xor inside 1 KB)
   uint8_t* ring = smem;                                                   // [kRingM][kBlkBytes]
   int32_t* slot = reinterpret_cast<int32_t*>(smem + kRingM * kBlkBytes);  // [nblk * 32]
   const int nblk = (p.TOPK + kKB - 1) / kKB;
@@ -137,42 +153,57 @@ void sa_mla_kernel(MlaParams p) {
   int nb = nblk_sh[0];
   for (int w = 1; w < NW; ++w) nb = max(nb, nblk_sh[w]);
 
-  // Copies: unit u covers chunk positions 64u .. 64u+63 of a block buffer
-  // (position P = row * 73 + chunk). Wave wi moves units wi, wi + NW, ...; every
-  // wave issues kUnitsW copies (surplus ones repeat the last unit: same bytes).
-  constexpr int kUnitsW = (kUnitsBlk + NW - 1) / NW;
+  // Copies: wave wi moves row units wi, wi + NW, ... (surplus ones repeat row 31: same bytes)
+  // and tail units wi, wi + NW, ...; with more than 4 waves, waves 0..3 one tail unit each.
+  // The slots of a block are one LDS read; a unit's row is then wave-uniform, so its address
+  // is scalar but for the lane's chunk. (One unit per 64 consecutive chunks of padded rows
+  // needed a division and a slot read per lane and unit: ~1000 cycles of a wave's ~5500 per
+  // block.)
+  constexpr int kMainW = (kKB + NW - 1) / NW;
+  constexpr int kTailW = NW > kTails ? 1 : (kTails + NW - 1) / NW;
   const int wis = __builtin_amdgcn_readfirstlane(wi);
+  const bool has_tail = NW <= kTails || wis < kTails;
   const i32x4 rsrc = make_rsrc(p.kv + (int64_t)b * p.NKV * p.kv_dim,
                                (uint32_t)p.NKV * (uint32_t)p.kv_dim * 2u);
   const uint32_t ring_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ring;
   const uint32_t row_bytes = (uint32_t)p.kv_dim * 2u;
-  // Copy offsets of block blk for this wave's units. They are recomputed from the
-  // lane id at every use: an opaque copy of the id keeps the compiler from holding
-  // ten per-lane values in registers across the block loop (which spilled them and
-  // put a scratch reload, with its vmcnt(0) wait on the copies in flight, into the
-  // loop).
-  auto rows_of = [&](int blk, uint32_t (&rv)[kUnitsW]) {
-    int ln = lane;
+  // (the lane id is taken anew at each use, so that nothing per lane is held for this)
+  auto lane_id = [] {
+    int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     asm volatile("" : "+v"(ln));
+    return ln;
+  };
+  auto issue = [&](int blk) {
+    const int ln = lane_id();
+    const uint32_t base = ring_lds + (uint32_t)(blk % kRingM) * (uint32_t)kBlkBytes;
+    const int sv = slot[blk * kKB + (ln & 31)];
+    int tv[kTailW];
 #pragma unroll
-    for (int i = 0; i < kUnitsW; ++i) {
-      int u = wis + NW * i;
-      if (u >= kUnitsBlk) u = kUnitsBlk - 1;
-      const int pos = 64 * u + ln;
-      const int r = pos / kRowC;
-      const int c = pos - r * kRowC;
-      const int w = slot[blk * kKB + min(r, kKB - 1)];
-      rv[i] = (r < kKB && w >= 0 && c < kRowC - 1) ? (uint32_t)w * row_bytes + 16u * (uint32_t)c : kOob;
+    for (int i = 0; i < kTailW; ++i) tv[i] = slot[blk * kKB + 8 * min(wis + NW * i, kTails - 1) + (ln >> 3)];
+#pragma unroll
+    for (int i = 0; i < kMainW; ++i) {
+      const int u = min(wis + NW * i, kKB - 1);
+      const int w = __builtin_amdgcn_readlane(sv, u);
+      // a masked slot (-1): an offset beyond the resource, which reads zeros
+      const uint32_t soff = w >= 0 ? (uint32_t)w * row_bytes : kOob;
+      const uint32_t keep = w >= 0 ? 0x3ffu : 0u;
+      lds_dma16(rsrc, ((16u * (uint32_t)(ln ^ swz(u))) & keep) + soff, base + 1024u * (uint32_t)u);
+    }
+    if (has_tail) {
+#pragma unroll
+      for (int i = 0; i < kTailW; ++i) {
+        const int t = min(wis + NW * i, kTails - 1);
+        const int c = 64 + ((ln & 7) ^ ((4 * t + (ln >> 4)) & 7));
+        lds_dma16(rsrc, tv[i] >= 0 ? (uint32_t)tv[i] * row_bytes + 16u * (uint32_t)c : kOob,
+                  base + (uint32_t)kTailOff + 1024u * (uint32_t)t);
+      }
     }
   };
-  auto issue = [&](int blk, const uint32_t (&rv)[kUnitsW]) {
-    const uint32_t base = ring_lds + (uint32_t)(blk % kRingM) * (uint32_t)kBlkBytes;
-#pragma unroll
-    for (int i = 0; i < kUnitsW; ++i) {
-      int u = wis + NW * i;
-      if (u >= kUnitsBlk) u = kUnitsBlk - 1;
-      lds_dma16(rsrc, rv[i], base + 1024u * (uint32_t)u);
-    }
+  // Waits until at most `n` blocks' copies of this wave are outstanding.
+  auto wait_blocks = [&](auto n) {
+    constexpr int kN = decltype(n)::value;
+    if (has_tail) wait_vmcnt<kN * (kMainW + kTailW)>();
+    else wait_vmcnt<kN * kMainW>();
   };
 
   f32x4 o[kCT];
@@ -190,11 +221,18 @@ void sa_mla_kernel(MlaParams p) {
   // channels 32ks + 8g; the lane's results are keys 16kt + 4g + r of head n.
   // Key tile 0 then key tile 1, one K fragment read ahead of its product (order
   // pinned below), so the LDS latency overlaps the matrix work.
-  auto qk = [&](const uint8_t* kvl) {
+  // Chunk 4ks + g of row n sits at (4ks ^ (g ^ swz(n))): bits 6, 7 of its address take ks % 4
+  // by xor, bits 8, 9 take ks / 4 as an offset.
+  const uint32_t kbase = ring_lds + 1024u * (uint32_t)n + 16u * (uint32_t)(g ^ swz(n));
+  const uint32_t tbase = ring_lds + (uint32_t)kTailOff + 128u * (uint32_t)n + 16u * (uint32_t)(g ^ (n >> 1));
+  auto qk = [&](const uint32_t bufoff) {
     S2 acc = {f32x4{}, f32x4{}};
-    const u32x4* r0 = reinterpret_cast<const u32x4*>(kvl) + n * kRowC + g;
+    const uint32_t kb_ = kbase + bufoff, tb_ = tbase + bufoff;
     auto frag = [&](int i) {  // i = 18 kt + ks
-      return __builtin_bit_cast(bf16x8, r0[(i >= kKS ? 16 * kRowC : 0) + 4 * (i % kKS)]);
+      const int kt = i >= kKS ? 1 : 0, ks = i - kt * kKS;
+      const uint32_t at = ks < 16 ? (kb_ ^ (64u * (ks & 3))) + 256u * (ks >> 2) + 16384u * kt
+                                  : (tb_ ^ (64u * (ks - 16))) + 2048u * kt;
+      return __builtin_bit_cast(bf16x8, *(lds_cu32x4_ptr)(uintptr_t)at);
     };
     bf16x8 a_cur = frag(0);
 #pragma unroll
@@ -217,12 +255,10 @@ void sa_mla_kernel(MlaParams p) {
 
 #pragma unroll
   for (int j = 0; j < kRingM - 1; ++j) {
-    if (j < nb) {
-      uint32_t rv[kUnitsW];
-      rows_of(j, rv);
-      issue(j, rv);
-    }
+    if (j < nb) issue(j);
   }
+  const uint32_t vbase = ring_lds + 1024u * (uint32_t)(4 * g + (n >> 2)) +
+                         16u * (uint32_t)(((n >> 1) & 1) ^ swz(4 * g + (n >> 2))) + 8u * (uint32_t)(n & 1);
   int vslot = slot[lane & 31];
 #pragma unroll
   for (int ks = 0; ks < kKS; ++ks) asm volatile("" ::"v"(qf[ks]));
@@ -245,14 +281,10 @@ void sa_mla_kernel(MlaParams p) {
   const bool late_sync = wis >= (NW + 1) / 2;
   auto sync_issue = [&](const int kb, uint32_t& vm_next) {
     if (kb + 1 < nb) {
-      if (kb + 2 < nb) wait_vmcnt<kUnitsW>();
+      if (kb + 2 < nb) wait_blocks(std::integral_constant<int, 1>{});
       else wait_vmcnt<0>();
       __syncthreads();  // block kb+1 is in LDS; block kb-1's buffer is free
-      if (kb + kRingM - 1 < nb) {
-        uint32_t rv[kUnitsW];
-        rows_of(kb + kRingM - 1, rv);
-        issue(kb + kRingM - 1, rv);
-      }
+      if (kb + kRingM - 1 < nb) issue(kb + kRingM - 1);
       vm_next = (uint32_t)__ballot(vslot >= 0);
       vslot = slot[min(kb + 2, nb - 1) * kKB + (lane & 31)];
     }
@@ -260,7 +292,8 @@ void sa_mla_kernel(MlaParams p) {
   auto step = [&](const int kb) {
     uint32_t vm_next = 0u;
     if (!late_sync) sync_issue(kb, vm_next);
-    const S2 sc = qk(ring + (kb % kRingM) * kBlkBytes);
+    const uint32_t bufoff = (uint32_t)(kb % kRingM) * (uint32_t)kBlkBytes;
+    const S2 sc = qk(bufoff);
     if (late_sync) sync_issue(kb, vm_next);
     float sv[8];  // keys 4g + r (r < 4) and 16 + 4g + (r - 4)
 #pragma unroll
@@ -328,22 +361,25 @@ void sa_mla_kernel(MlaParams p) {
     // 16ct + 4(s%4) .. +3 of key row 4g + s/4 (first read) and 16 + 4g + s/4
     // (second); the transposed reads hand channel 16ct + (lane%16) keys
     // 4g + 0..3 and 16 + 4g + 0..3 to each lane, matching the P operand.
-    const uint16_t* kvh = reinterpret_cast<const uint16_t*>(ring + (kb % kRingM) * kBlkBytes);
-    const uint16_t* row0 = kvh + (4 * g + (n >> 2)) * (kRowC * 8) + 4 * (n & 3);
-    const uint16_t* row1 = row0 + 16 * (kRowC * 8);
+    // Chunk 2ct + (s%4)/2 of the row: bits 5..7 of the address take ct % 8 by xor, bits 8, 9
+    // ct / 8 as an offset; the tiles go in groups of one xor.
+    const uint32_t vb_ = vbase + bufoff;
     // One V^T fragment is read ahead: the two reads of fragment ct+1 are issued
     // before the two products of fragment ct (the order is pinned below), so the
     // LDS latency overlaps the matrix work.
     auto read_v = [&](int ct) {
-      const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(row0 + 16 * ct));
-      const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(row1 + 16 * ct));
+      const uint32_t at = (vb_ ^ (32u * (ct & 7))) + 256u * (ct >> 3);
+      const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(uintptr_t)at);
+      const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(uintptr_t)(at + 16384u));
       return __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
     };
-    bf16x8 a_cur = read_v(0);
+    auto tile = [](int i) { return 8 * (i & 3) + (i >> 2); };
+    bf16x8 a_cur = read_v(tile(0));
 #pragma unroll
-    for (int ct = 0; ct < kCT; ++ct) {
+    for (int i = 0; i < kCT; ++i) {
+      const int ct = tile(i);
       bf16x8 a_nxt = a_cur;
-      if (ct + 1 < kCT) a_nxt = read_v(ct + 1);
+      if (i + 1 < kCT) a_nxt = read_v(tile(i + 1));
       if constexpr (kSplit) o[ct] = mfma16x16x32(a_cur, plo2, o[ct]);
       o[ct] = mfma16x16x32(a_cur, plo, o[ct]);
       o[ct] = mfma16x16x32(a_cur, phi, o[ct]);
@@ -361,8 +397,8 @@ void sa_mla_kernel(MlaParams p) {
   };
 
   if (nb > 0) {
-    if (nb >= 3) wait_vmcnt<2 * kUnitsW>();
-    else if (nb == 2) wait_vmcnt<kUnitsW>();
+    if (nb >= 3) wait_blocks(std::integral_constant<int, 2>{});
+    else if (nb == 2) wait_blocks(std::integral_constant<int, 1>{});
     else wait_vmcnt<0>();
     __syncthreads();
     vm_cur = (uint32_t)__ballot(vslot >= 0);
