@@ -170,6 +170,17 @@ def test_mla_split_decode(gpu, case):
     _compare(out, one, f"split-vs-one-pass{case}")
 
 
+@pytest.mark.parametrize("b, h, topk", [(1, 128, 1024), (1, 128, 1025), (4, 64, 512), (9, 80, 320), (9, 112, 320)])
+def test_mla_split_partial_stores(gpu, b, h, topk):
+    """Partials of 4 MB (the most that is written back) and around it (17 splits of 32 rows
+    and one; 9 tokens x 5 splits x 80 or 112 heads), with a used workspace."""
+    q, kv, idx, sink = _case(b, 1, h, 3000, topk, 50 + h, 0.1, 0.5)
+    prep = _native.prepare_sparse_mla(q, kv, idx, sink, SCALE, DV)
+    prep.keep[4].fill_(255)                  # NaN patterns: every partial has to be written
+    out = prep.run()
+    _compare(out, osa.sparse_attn_ref(q, kv, sink, idx, SCALE, v_dim=DV), f"stores{(b, h, topk)}")
+
+
 @pytest.mark.parametrize("split", [False, True])
 def test_mla_neg_inf_sink_masked_leading_block(gpu, split):
     """A -inf sink (no sink mass) with the first slot blocks fully masked: the running
