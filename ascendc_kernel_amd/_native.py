@@ -252,6 +252,42 @@ class Prepared:
         return out
 
 
+# Native serving of further calls with a prepared call's layouts (csrc/fastcall.cpp): what a
+# pointer argument is filled with besides the index of one of the call's tensors.
+FAST_OUT, FAST_TEMP, FAST_STREAM = -1, -2, -3
+#: entry point (without _i64) -> signature kind and the position of its float argument
+_FAST_KIND = {"dsa_sparse_attn_fwd": (0, 11), "dsa_sparse_mla_fwd": (1, 13), "dsa_sparse_mla_fwd_ws": (2, 13),
+              "dsa_indexer_score_topk": (3, 4), "dsa_indexer_score_topk_ws": (4, 4),
+              "dsa_indexer_projections_splitk": (5, None), "dsa_indexer_decode_projections_rope": (5, None)}
+_fastcall = None
+
+
+def fast_run(plan, *args):
+    """The output of a call that `plan` (of fast_plan) serves, else None."""
+    return _fastcall.run(plan, *args)
+
+
+def fast_plan(tensors, scalars, launches, patches, out_shape, out_like: int, temp_bytes: int, positions=None):
+    """A native plan for calls whose tensors have these layouts and whose scalars are these, from
+    the marshalled `launches`: patches = [(launch, slot, tensor index or FAST_*, byte offset)]
+    fill every pointer per call; the output has out_shape and the dtype of tensor out_like (-1:
+    int64); temp_bytes of scratch are allocated per call. positions: an indexer's, whose calls
+    then end in start_pos and offset (struct Positions). None where a tensor cannot be served."""
+    global _fastcall, fast_run
+    if _fastcall is None:
+        from . import _fastcall as mod
+        _fastcall, fast_run = mod, mod.run
+    calls = []
+    for launch in launches:
+        kind, at = _FAST_KIND[launch.name.replace("_i64", "")]
+        values = [a.value or 0 for a in launch.args]
+        calls.append((kind, ctypes.cast(launch.fn, _c_vp).value, [int(v) for v in values],
+                      float(values[at]) if at is not None else 0.0))
+    ws_fn = ctypes.cast(load().dsa_indexer_workspace_bytes, _c_vp).value
+    return _fastcall.make(tuple(tensors), tuple(scalars), calls, list(patches), list(out_shape), out_like,
+                          temp_bytes, positions, ws_fn)
+
+
 def prepare_sparse_attn(q: torch.Tensor, kv: torch.Tensor, topk_idxs: torch.Tensor,
                         attn_sink: torch.Tensor, softmax_scale: float,
                         variant: int = DSA_SA_AUTO) -> Prepared:

@@ -18,6 +18,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 REPO = os.path.dirname(PKG_DIR)
 LIB_NAME = "libdsa_mi355x.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
+FASTCALL_PATH = os.path.join(PKG_DIR, "_fastcall.so")
 ARCH = "gfx950"
 
 # -ffp-contract=off: every fused multiply-add in the kernels is written out
@@ -58,14 +59,36 @@ def _compile(src: str, obj: str) -> None:
         raise RuntimeError(f"hipcc failed for {os.path.basename(src)}:\n{err}")
 
 
+def _build_fastcall() -> None:
+    """``_fastcall.so``, the host-only extension of the modules' repeated calls (torch's headers)."""
+    import sysconfig
+
+    import torch
+    base = os.path.dirname(torch.__file__)
+    tmp = FASTCALL_PATH + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           *(f"-I{d}" for d in (f"{base}/include", f"{base}/include/torch/csrc/api/include",
+                                sysconfig.get_paths()["include"], "/opt/rocm/include")),
+           "-o", tmp, os.path.join(CSRC, "fastcall.cpp"), f"-L{base}/lib",
+           "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for fastcall.cpp:\n{r.stderr}")
+    os.replace(tmp, FASTCALL_PATH)
+
+
 def build(verbose: bool = False) -> str:
-    """Compile all kernels for gfx950 and link ``libdsa_mi355x.so``; returns its path."""
+    """Compile all kernels for gfx950 and link ``libdsa_mi355x.so`` (its path is returned), and
+    compile the ``_fastcall`` extension."""
     objdir = os.path.join(REPO, "_build", "dsa")
     os.makedirs(objdir, exist_ok=True)
     srcs = sources()
     objs = [os.path.join(objdir, os.path.basename(s)[:-4] + ".o") for s in srcs]
     with _cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+        fast = ex.submit(_build_fastcall)
         list(ex.map(_compile, srcs, objs))
+        fast.result()
     tmp = LIB_PATH + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)

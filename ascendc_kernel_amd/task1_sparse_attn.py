@@ -37,8 +37,21 @@ class Model(nn.Module):
         # their memory cannot be reused for other tensors (which could repeat a pointer)
         # while the key that names them is cached.
         self._plan = None
+        # The native plan that serves further calls with the last calls' layouts, and the
+        # layout seen last on the way to building one.
+        self._fast = None
+        self._fast_scratch = False
+        self._seen = None
 
     def forward(self, q: torch.Tensor, kv: torch.Tensor, topk_idxs: torch.Tensor) -> torch.Tensor:
+        # Calls with the layouts of the calls before them, whatever their tensors. (A split MLA
+        # launch takes scratch memory: there the last call's own plan is looked at first.
+        # Scratch of its own per module, rather than the allocator's block that the call before
+        # has just used too, is 1.5-2.3 us faster at one token of 128 heads.)
+        if self._fast is not None and not self._fast_scratch:
+            out = self._run_fast(q, kv, topk_idxs)
+            if out is not None:
+                return out
         # Steady state (the Ascend ModelNew's fast path binds its launch after the third call
         # with the same input pointers, src/task1_sparse_attn.py:751-755,789-801): the same
         # pointers, shapes, dtypes, sink and stream as the last call reuse its checked and
@@ -52,9 +65,40 @@ class Model(nn.Module):
                    _native.stream_handle(dev), self.variant, self.v_dim)
             plan = self._plan
             if plan is None or plan[0] != key:
+                if self._fast is not None and self._fast_scratch:
+                    out = self._run_fast(q, kv, topk_idxs)
+                    if out is not None:
+                        return out
                 plan = self._plan = (key, self._prepare(q, kv, topk_idxs))
-            return plan[1].run()
+            out = plan[1].run()
+            if dev.type == "cuda":
+                self._learn(plan[1], q, kv, topk_idxs)
+            return out
         return self._prepare(q, kv, topk_idxs).run()
+
+    def _run_fast(self, q: torch.Tensor, kv: torch.Tensor, topk_idxs: torch.Tensor):
+        return _native.fast_run(self._fast, q, kv, topk_idxs, self.attn_sink, self.n_heads, self.head_dim,
+                                self.v_dim, self.variant, self.softmax_scale)
+
+    def _learn(self, prepared: "_native.Prepared", q, kv, topk_idxs) -> None:
+        """Builds the native plan when two calls in a row had the same layouts."""
+        seen = (q.shape, kv.shape, topk_idxs.shape, topk_idxs.dtype, self.v_dim, self.variant)
+        if self._seen != seen:
+            self._seen = seen
+            return
+        self._seen = None
+        sink, launch, ws = self.attn_sink, prepared.launch, prepared.keep[4:]
+        if prepared.keep[3].data_ptr() != sink.data_ptr():
+            return  # converted: the launch reads a copy
+        stream = len(launch.args) - 1
+        patches = [(0, i, i, 0) for i in range(4)]
+        patches += [(0, prepared.out_slot, _native.FAST_OUT, 0), (0, stream, _native.FAST_STREAM, 0)]
+        if ws:
+            patches.append((0, stream - 2, _native.FAST_TEMP, 0))
+        self._fast_scratch = bool(ws)
+        self._fast = _native.fast_plan(
+            (q, kv, topk_idxs, sink), (self.n_heads, self.head_dim, self.v_dim, self.variant, self.softmax_scale),
+            (launch,), patches, prepared.out_shape, 0, ws[0].numel() if ws else 0)
 
     def _prepare(self, q: torch.Tensor, kv: torch.Tensor, topk_idxs: torch.Tensor) -> "_native.Prepared":
         if q.dim() != 4 or q.shape[2] != self.n_heads or q.shape[3] != self.head_dim:

@@ -238,6 +238,10 @@ class Model(nn.Module):
         # key that names them is cached.
         self._plan = None
         self._packed = None
+        # The native plan that serves further calls with the last calls' layouts, and the
+        # layout seen last on the way to building one.
+        self._fast = None
+        self._seen = None
 
     def route(self, x: torch.Tensor, qr: torch.Tensor) -> str:
         """The projections' path for these inputs: 'splitk' (splitk_route), else what
@@ -257,8 +261,15 @@ class Model(nn.Module):
         # after the third call with the same pointers, src/task2_indexer.py:1069-1072,
         # 1340-1348): the same inputs, positions, weights (pointer and version), cache, table
         # and stream as the last call reuse its plan; only the fresh output is allocated.
-        dev = x.device
         wq, wp, kv, fc = self.wq_b.weight, self.weights_proj.weight, self.kv_cache, self.freqs_cis
+        # Calls with the layouts of the calls before them, whatever their tensors and positions.
+        if self._fast is not None:
+            out = _native.fast_run(self._fast, x, qr, wq, wp, kv, fc, self.rope_mode, self.compress_ratio,
+                                   self.index_topk, self.n_heads, self.n_local_heads, self.head_dim,
+                                   self.rope_head_dim, self.softmax_scale, start_pos, offset)
+            if out is not None:
+                return out
+        dev = x.device
         # (A plan reads kv_cache and freqs_cis in place, so it sees their updates; it is kept
         # only where neither needs a contiguous copy, which would not.)
         if (dev.type == _native.PLAN_DEVICE_TYPE and x.is_contiguous() and qr.is_contiguous() and kv.dim() == 3
@@ -270,7 +281,10 @@ class Model(nn.Module):
             plan = self._plan
             if plan is None or plan.key != key:
                 plan = self._plan = _IndexerPlan(self, x, qr, start_pos, offset, key)
-            return plan.run()
+            out = plan.run()
+            if dev.type == "cuda" and plan.empty is None and plan.route in ("splitk", "decode"):
+                self._learn(plan, x, qr, start_pos)
+            return out
         return _IndexerPlan(self, x, qr, start_pos, offset, None).run()
 
     def packed_weights(self):
@@ -287,6 +301,44 @@ class Model(nn.Module):
         """Drops the packed weights and the cached plan (after writes through .data)."""
         self._packed = None
         self._plan = None
+        self._fast = self._seen = None
+
+    def _learn(self, plan: "_IndexerPlan", x: torch.Tensor, qr: torch.Tensor, start_pos: int) -> None:
+        """Builds the native plan when two calls in a row had the same layouts (one launch for
+        both projections from the weights in place, then the score kernel)."""
+        kv, fc = self.kv_cache, self.freqs_cis
+        seen = (x.shape, qr.shape, kv.shape, kv.stride(), fc.shape, start_pos == 0, self.rope_mode,
+                self.compress_ratio, self.index_topk)
+        if self._seen != seen:
+            self._seen = seen
+            return
+        self._seen = None
+        tensors = x, qr, wq, wp, kv, fc = x, qr, self.wq_b.weight, self.weights_proj.weight, kv, fc
+        if not (wq.is_contiguous() and wp.is_contiguous()):
+            return  # the launch reads copies
+        temp, stream = _native.FAST_TEMP, _native.FAST_STREAM
+        splitk = plan.route == "splitk"
+        x_slot, wp_slot, q_slot, wl_slot = (5, 6, 4, 7) if splitk else (4, 5, 6, 7)
+        tokens = x.shape[0] * x.shape[1]
+        wl_off = 2 * tokens * wq.shape[0]                       # q, wl and the score workspace
+        ws_off = (wl_off + 2 * tokens * wp.shape[0] + 255) // 256 * 256
+        score = plan.score.launch
+        has_ws = score.name.endswith("_ws")
+        patches = [(0, 0, 1, 0), (0, 1, 2, 0), (0, 2, 5, 0), (0, x_slot, 0, 0), (0, wp_slot, 3, 0),
+                   (0, q_slot, temp, 0), (0, wl_slot, temp, wl_off), (0, 16, stream, 0),
+                   (1, _native.SCORE_SLOT_Q, temp, 0), (1, 1, 4, 0), (1, _native.SCORE_SLOT_WL, temp, wl_off),
+                   (1, _native.SCORE_SLOT_OUT, _native.FAST_OUT, 0), (1, len(score.args) - 1, stream, 0)]
+        if has_ws:
+            patches.append((1, 18, temp, ws_off))
+        row_bytes = 8 * (fc.numel() // fc.shape[0])
+        if row_bytes % 16:
+            return
+        positions = (start_pos == 0, x.shape[1], self.compress_ratio, self.index_topk, fc.shape[0], row_bytes,
+                     kv.shape[1], 0, 2, 1, ws_off if has_ws else -1)
+        self._fast = _native.fast_plan(
+            tensors, (self.rope_mode, self.compress_ratio, self.index_topk, self.n_heads, self.n_local_heads,
+                      self.head_dim, self.rope_head_dim, self.softmax_scale),
+            (plan.proj, score), patches, plan.score.out_shape, -1, ws_off, positions)
 
 
 class _IndexerPlan:

@@ -1,0 +1,125 @@
+"""Native serving of calls with known layouts (csrc/fastcall.cpp): what a plan takes and refuses,
+on the CPU with a recording C function as the launch, and the modules on the GPU against a fresh
+module's first call."""
+import ctypes
+
+import pytest
+import torch
+
+from ascendc_kernel_amd import _native
+from ascendc_kernel_amd import task1_sparse_attn as t1
+from ascendc_kernel_amd import task2_indexer as t2
+
+
+class _Recorder:
+    """A C function with dsa_sparse_attn_fwd's signature that records its arguments."""
+
+    def __init__(self):
+        self.calls, self.rc = [], 0
+        p, i = ctypes.c_void_p, ctypes.c_int64
+        self.fn = ctypes.CFUNCTYPE(ctypes.c_int, p, p, p, p, p, i, i, i, i, i, i, ctypes.c_float, ctypes.c_int32,
+                                   p)(self._record)
+
+    def _record(self, *args):
+        self.calls.append(args)
+        return self.rc
+
+
+def _cpu_plan(tensors, rec):
+    from ascendc_kernel_amd import _fastcall
+    call = (0, ctypes.cast(rec.fn, ctypes.c_void_p).value, [0] * 5 + [1, 2, 3, 4, 5, 6] + [0, 7, 0], 0.5)
+    patches = [(0, i, i, 0) for i in range(4)] + [(0, 4, _native.FAST_OUT, 0), (0, 13, _native.FAST_STREAM, 0)]
+    return _fastcall.run, _fastcall.make(tuple(tensors), (64, None, 0.25), [call], patches, [2, 3], 0, 0, None, 0)
+
+
+def test_plan_takes_layouts_not_tensors():
+    rec = _Recorder()
+    ts = [torch.zeros(4, 8, dtype=torch.bfloat16) for _ in range(4)]
+    run, plan = _cpu_plan(ts, rec)
+    others = [t.clone() for t in ts]
+    for inputs in (ts, others):
+        out = run(plan, *inputs, 64, None, 0.25)
+        assert out.shape == (2, 3) and out.dtype == torch.bfloat16
+        args = rec.calls[-1]
+        assert args[:5] == tuple(t.data_ptr() for t in (*inputs, out)) and args[5:13] == (1, 2, 3, 4, 5, 6, 0.5, 7)
+    with torch.inference_mode():  # other dispatch keys
+        assert run(plan, *[t.clone() for t in ts], 64, None, 0.25) is None
+
+
+def test_plan_refuses_other_layouts():
+    rec = _Recorder()
+    ts = [torch.zeros(4, 8, dtype=torch.bfloat16) for _ in range(4)]
+    run, plan = _cpu_plan(ts, rec)
+    whole = torch.zeros(5 * 8 + 8, dtype=torch.bfloat16)
+    off = (16 - whole.data_ptr() % 16) % 16 // 2 + 1         # two bytes past a 16-byte address
+    for other in (torch.zeros(4, 9, dtype=torch.bfloat16), torch.zeros(8, 4, dtype=torch.bfloat16).t(),
+                  torch.zeros(4, 8), whole[off:off + 32].view(4, 8), None,
+                  torch.zeros(4, 8, dtype=torch.bfloat16).to_sparse()):
+        assert run(plan, other, *ts[1:], 64, None, 0.25) is None
+    assert run(plan, *ts, 65, None, 0.25) is None
+    assert run(plan, *ts, 64, 0, 0.25) is None
+    assert run(plan, *ts, 64, None, 0.5) is None
+    assert run(plan, *ts, 64, None) is None
+    assert run(None, *ts, 64, None, 0.25) is None
+    assert torch.vmap(lambda t: ts[0] if run(plan, t, *ts[1:], 64, None, 0.25) is None else t,
+                      randomness="error")(ts[0].expand(2, 4, 8)).shape == (2, 4, 8)
+    with torch.device("meta"):                               # an active function mode
+        assert run(plan, *ts, 64, None, 0.25) is None
+    assert not rec.calls
+    rec.rc = -2                                              # a refused launch
+    assert run(plan, *ts, 64, None, 0.25) is None and len(rec.calls) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h, d, v, m, n_kv, topk", [(64, 128, None, 40, 32, 16), (48, 128, None, 3, 700, 333),
+                                                    (128, 576, 512, 1, 900, 300), (80, 576, 512, 67, 900, 128)])
+def test_attention_calls(h, d, v, m, n_kv, topk):
+    """New tensors of known layouts, on another stream too, give a fresh module's bits."""
+    g = torch.Generator(device="cuda").manual_seed(h + m)
+    model, side = t1.Model(h, d, v).to("cuda"), torch.cuda.Stream()
+    with torch.no_grad():
+        model.attn_sink.copy_(torch.randn(h, generator=g, device="cuda"))
+    for call in range(5):
+        q = torch.randn(2, m, h, d, generator=g, device="cuda", dtype=torch.bfloat16)
+        kv = torch.randn(2, n_kv, d, generator=g, device="cuda", dtype=torch.bfloat16)
+        idx = torch.randint(-1, n_kv, (2, m, topk), generator=g, device="cuda", dtype=torch.int32)
+        fresh = t1.Model(h, d, v).to("cuda")
+        fresh.load_state_dict(model.state_dict())
+        want = fresh(q, kv, idx)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side if call == 4 else torch.cuda.current_stream()):
+            got = model(q, kv, idx)
+        torch.cuda.synchronize()
+        assert (model._fast is not None) == (call >= 1)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    with pytest.raises((ValueError, TypeError)):
+        model(q.float(), kv, idx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["indexer", "dsa"])
+@pytest.mark.parametrize("s, starts", [(1, (300, 301, 302, 511, 16)), (2, (64, 66, 510, 100, 98)),
+                                       (11, (0, 0, 0, 0, 0))])
+def test_indexer_calls(kind, s, starts):
+    """New inputs, positions and offsets give a fresh module's picks; positions outside the
+    table or the cache are refused as before."""
+    g = torch.Generator(device="cuda").manual_seed(s)
+    ql, dim, heads, hd, rd, ratio = (256, 1024, 16, 64, 32, 4) if kind == "indexer" else (1536, 7168, 64, 128, 64, 1)
+    a = t2.ModelArgs(max_batch_size=1, max_seq_len=512, dim=dim, index_n_heads=heads, index_head_dim=hd,
+                     index_topk=40, q_lora_rank=ql, rope_head_dim=rd)
+    freqs = t2.precompute_freqs_cis(rd, 512)
+    cache = torch.randn(1, 512 // ratio, hd, generator=g, device="cuda", dtype=torch.bfloat16)
+    model = t2.Model(a, freqs, cache, ratio).to("cuda")
+    for call, start in enumerate(starts):
+        x = torch.randn(1, s, dim, generator=g, device="cuda", dtype=torch.bfloat16)
+        qr = torch.randn(1, s, ql, generator=g, device="cuda", dtype=torch.bfloat16)
+        fresh = t2.Model(a, freqs, cache, ratio).to("cuda")
+        fresh.load_state_dict(model.state_dict())
+        want = fresh(x, qr, start, call)
+        got = model(x, qr, start, call)
+        assert torch.equal(got, want)
+        if fresh.route(x, qr) in ("splitk", "decode"):
+            assert (model._fast is not None) == (call >= 1)
+    if starts[0]:
+        with pytest.raises((ValueError, RuntimeError)):
+            model(x, qr, 513 - s, 0)
