@@ -23,6 +23,11 @@ class Model(nn.Module):
 
     #: kernel choice passed to the C ABI (auto = multiplicity kernel when n_kv <= 32)
     variant: int = _native.DSA_SA_AUTO
+    # The native plan that serves further calls with the last calls' layouts (and whether it
+    # takes scratch memory), and the layout seen last on the way to building one.
+    _fast = None
+    _fast_scratch = False
+    _seen = None
 
     def __init__(self, n_heads: int, head_dim: int, v_dim: int = None):
         """`v_dim` (not in the reference, default None = head_dim): value width for sparse
@@ -37,11 +42,6 @@ class Model(nn.Module):
         # their memory cannot be reused for other tensors (which could repeat a pointer)
         # while the key that names them is cached.
         self._plan = None
-        # The native plan that serves further calls with the last calls' layouts, and the
-        # layout seen last on the way to building one.
-        self._fast = None
-        self._fast_scratch = False
-        self._seen = None
 
     def forward(self, q: torch.Tensor, kv: torch.Tensor, topk_idxs: torch.Tensor) -> torch.Tensor:
         # Calls with the layouts of the calls before them, whatever their tensors. (A split MLA

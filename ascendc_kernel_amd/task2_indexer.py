@@ -215,6 +215,10 @@ class Model(nn.Module):
 
     #: which torch rounding of the RoPE complex product to reproduce
     rope_mode: int = _native.DSA_ROPE_TORCH_ROCM
+    # The native plan that serves further calls with the last calls' layouts, and the layout
+    # seen last on the way to building one.
+    _fast = None
+    _seen = None
 
     def __init__(self, args: ModelArgs, freqs_cis: torch.Tensor, kv_cache: torch.Tensor,
                  compress_ratio: int = 4):
@@ -238,10 +242,6 @@ class Model(nn.Module):
         # key that names them is cached.
         self._plan = None
         self._packed = None
-        # The native plan that serves further calls with the last calls' layouts, and the
-        # layout seen last on the way to building one.
-        self._fast = None
-        self._seen = None
 
     def route(self, x: torch.Tensor, qr: torch.Tensor) -> str:
         """The projections' path for these inputs: 'splitk' (splitk_route), else what
