@@ -280,9 +280,9 @@ int dsa_indexer_scores(const void* q, const void* kv_cache, int64_t kv_batch_str
  *   q          bf16 [m, n] output
  * Requirements: k % 32 == 0, n % 256 == 0, head_dim in {64, 128}, (head_dim - rd) % 8 == 0,
  * m * k * 2 and n * k * 2 below 2^32, m % s_len == 0; pointers 16-byte aligned.
- * The drop-in Model uses it for q_lora_rank 256 and rd 32 from 64 tokens (configs[2]:
- * ~19 us against ~26 us for hipBLASLt's F.linear alone) and keeps F.linear + the score
- * kernel's own RoPE below 64 tokens and for other k.
+ * The drop-in Model uses it for q_lora_rank 256 and rd 32 from 64 tokens where neither
+ * dsa_indexer_projections nor dsa_indexer_projections_splitk gives F.linear's weights_proj
+ * (20,800 tokens: ~19 us against ~26 us for hipBLASLt's F.linear alone).
  */
 int dsa_indexer_q_proj(const void* qr, const void* wq, const void* freqs_cis, int32_t rope_mode,
                        void* q, int64_t m, int64_t n, int64_t k, int64_t head_dim, int64_t rd,
