@@ -92,6 +92,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, uin
                                            (int)bytes, 0x00020000);
 }
 
+// The buffer intrinsics' cache bit of a store that is written through the L2: its lines are
+// not left dirty for the kernel's end, where a dependent kernel waits for their flush.
+constexpr int kSc1 = 16;
+
 // One buffer_load_dwordx4 ... lds: lane l copies the 16 B at byte offset voff of
 // the resource to LDS byte address m0 + 16 * l (m0 is wave-uniform). It is
 // issued from inline asm so that the compiler does not track it: its own

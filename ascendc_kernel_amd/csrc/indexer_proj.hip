@@ -332,13 +332,20 @@ struct QTileCopier {
   }
 };
 
+constexpr int64_t kThroughTokens = 1024;  // see kThrough below
+
 // The q tiles of q-role block `blk`. kPacked: W comes as fragments pre-packed by
 // dsa_indexer_pack_projection_weights (wave slice r = n / 64, tile i, k-step ks, lane:
 // 16 B), loaded straight into registers with 1 KB coalesced loads after the first two
 // tiles' copies are issued; otherwise W is staged through LDS from its [N, 256] rows.
 // part: 0 = every tile of the block's token run, 1 = all but its tail, 2 = the tail only
 // (tail16 / 16 of the run's tiles).
-template <int RD, int RM, bool kPacked>
+// kThrough: over kThroughTokens the q rows (2 KB each) are written through the L2. The score
+// kernel that follows waits for what is left dirty at this kernel's end: projections + score of
+// the 16-head indexer, ratio 4, written back -> through: 1500 tokens 14.8 -> 14.6 us, 2000
+// 18.8 -> 18.1, 3009 20.0 -> 18.7, 6400 25.5 -> 24.6, 15200 44.9 -> 43.2; 1000 equal, 600 11.5
+// -> 11.65. Packed weights (from 15,361 tokens): 20,800 65.4 -> 65.6, so not there.
+template <int RD, int RM, bool kPacked, bool kThrough = false>
 __device__ __forceinline__ void q_role(const SProjParams& p, int blk, uint8_t* smem, int part) {
   using C = SCfg<RD>;
   const int tid = threadIdx.x;
@@ -505,7 +512,10 @@ __device__ __forceinline__ void q_role(const SProjParams& p, int blk, uint8_t* s
       // Rows at or past M are beyond the resource and dropped.
       const uint32_t off = mm < (uint32_t)p.M ? (mm * (uint32_t)p.N + (uint32_t)(n0 + 64 * wis + 8 * ch)) * 2u
                                               : 0xfffffff0u;
-      __builtin_amdgcn_raw_buffer_store_b128(v, qrs, (int)off, 0, 0);
+      if (kThrough && p.M > kThroughTokens)
+        __builtin_amdgcn_raw_buffer_store_b128(v, qrs, (int)off, 0, kSc1);
+      else
+        __builtin_amdgcn_raw_buffer_store_b128(v, qrs, (int)off, 0, 0);
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -642,12 +652,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   extern __shared__ __align__(16) uint8_t smem[];
   const int b = blockIdx.x;
   if (b < p.nq) {
-    q_role<RD, RM, !kSplitK>(p.q, b, smem, p.wtail ? 1 : 0);
+    q_role<RD, RM, !kSplitK, kSplitK>(p.q, b, smem, p.wtail ? 1 : 0);
   } else {
     w_role<kSplitK, !kSplitK>(p.w, b - p.nq, smem);
     if (p.wtail) {
       __syncthreads();  // the w role's LDS (W fragments) becomes the q role's ring
-      q_role<RD, RM, !kSplitK>(p.q, b - p.nq, smem, 2);
+      q_role<RD, RM, !kSplitK, kSplitK>(p.q, b - p.nq, smem, 2);
     }
   }
 }

@@ -46,7 +46,6 @@ constexpr int kTails = 4;
 constexpr int kBlkBytes = kTailOff + kTails * 1024;  // 36864 B per buffer
 constexpr int kRingM = 4;
 constexpr uint32_t kThroughBytes = 4u << 20;     // split partials over this are written through (see there)
-constexpr int kSc1 = 16;                         // the buffer intrinsics' cache bit for that
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kRaise = 8.0f;
 constexpr uint32_t kOob = 0xfffffff0u;          // a copy offset beyond any resource: reads zeros

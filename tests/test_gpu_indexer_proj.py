@@ -216,7 +216,7 @@ def _planted(m, n, k, g, dev):
     return x.to(torch.bfloat16), w.to(torch.bfloat16)
 
 
-@pytest.mark.parametrize("b,s", [(1, 1), (3, 5), (2, 8), (1, 17), (1, 31), (4, 8), (1, 33), (3, 1003), (1, 5000),
+@pytest.mark.parametrize("b,s", [(1, 1), (3, 5), (2, 8), (1, 17), (1, 31), (4, 8), (1, 33), (1, 1024), (1, 1025), (3, 1003), (1, 5000),
                                  (1, 15360), (1, 15518), (2, 8192)])
 def test_splitk_projections_equal_f_linear(gpu, b, s):
     """dsa_indexer_projections_splitk at the edges of its forms (16 / 17 tokens, 32-token tiles)
