@@ -161,7 +161,12 @@ py::object make(py::tuple tensors, py::tuple scalars, py::list calls, py::list p
     if (!same(t, e)) return py::none();  // misaligned
     plan->tensors.push_back(std::move(e));
   }
-  for (auto h : scalars) plan->scalars.push_back(py::reinterpret_borrow<py::object>(h));
+  for (auto h : scalars) {
+    PyObject* o = h.ptr();
+    // Plain values only: an object that can change in place would still be the plan's own.
+    if (o != Py_None && !PyLong_Check(o) && !PyFloat_Check(o)) return py::none();
+    plan->scalars.push_back(py::reinterpret_borrow<py::object>(h));
+  }
   plan->device = plan->tensors.at(0).device;
   for (const Layout& e : plan->tensors)
     if (e.device != plan->device) return py::none();

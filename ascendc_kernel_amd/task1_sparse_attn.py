@@ -54,15 +54,17 @@ class Model(nn.Module):
                 return out
         # Steady state (the Ascend ModelNew's fast path binds its launch after the third call
         # with the same input pointers, src/task1_sparse_attn.py:751-755,789-801): the same
-        # pointers, shapes, dtypes, sink and stream as the last call reuse its checked and
-        # marshalled launch; only the fresh output is allocated. Anything else (including an
-        # in-place update of attn_sink, which moves its version counter) prepares anew.
+        # pointers, shapes, dtypes, sink, stream and scalars of the module (the launch's arguments
+        # hold them) as the last call reuse its checked and marshalled launch; only the fresh
+        # output is allocated. Anything else (including an in-place update of attn_sink, which
+        # moves its version counter) prepares anew.
         dev = q.device
         if dev.type == _native.PLAN_DEVICE_TYPE and q.is_contiguous() and kv.is_contiguous() and topk_idxs.is_contiguous():
             sink = self.attn_sink
             key = (q.data_ptr(), kv.data_ptr(), topk_idxs.data_ptr(), q.shape, kv.shape, topk_idxs.shape,
                    q.dtype, kv.dtype, topk_idxs.dtype, sink.data_ptr(), sink._version,
-                   _native.stream_handle(dev), self.variant, self.v_dim)
+                   _native.stream_handle(dev), self.variant, self.v_dim, self.n_heads, self.head_dim,
+                   float(self.softmax_scale))
             plan = self._plan
             if plan is None or plan[0] != key:
                 if self._fast is not None and self._fast_scratch:

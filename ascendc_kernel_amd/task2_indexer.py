@@ -259,8 +259,9 @@ class Model(nn.Module):
     def forward(self, x: torch.Tensor, qr: torch.Tensor, start_pos: int, offset: int) -> torch.Tensor:
         # Steady state (the Ascend ModelNew binds a no-argument launch of the whole forward
         # after the third call with the same pointers, src/task2_indexer.py:1069-1072,
-        # 1340-1348): the same inputs, positions, weights (pointer and version), cache, table
-        # and stream as the last call reuse its plan; only the fresh output is allocated.
+        # 1340-1348): the same inputs, positions, weights (pointer and version), cache, table,
+        # stream and scalars of the module (the launches' arguments hold them) as the last call
+        # reuse its plan; only the fresh output is allocated.
         wq, wp, kv, fc = self.wq_b.weight, self.weights_proj.weight, self.kv_cache, self.freqs_cis
         # Calls with the layouts of the calls before them, whatever their tensors and positions.
         if self._fast is not None:
@@ -276,8 +277,9 @@ class Model(nn.Module):
                 and kv.stride(2) == 1 and kv.stride(1) == kv.shape[2] and fc.is_contiguous()):
             key = (x.data_ptr(), qr.data_ptr(), x.shape, qr.shape, x.dtype, qr.dtype, start_pos, offset,
                    wq.data_ptr(), wq._version, wp.data_ptr(), wp._version, kv.data_ptr(), kv.shape,
-                   kv.stride(), fc.data_ptr(), fc.shape, _native.stream_handle(dev), self.rope_mode,
-                   self.compress_ratio, self.index_topk)
+                   kv.stride(), kv.dtype, fc.data_ptr(), fc.shape, fc.dtype, _native.stream_handle(dev),
+                   self.rope_mode, self.compress_ratio, self.index_topk, self.n_heads, self.n_local_heads,
+                   self.head_dim, self.rope_head_dim, float(self.softmax_scale))
             plan = self._plan
             if plan is None or plan.key != key:
                 plan = self._plan = _IndexerPlan(self, x, qr, start_pos, offset, key)

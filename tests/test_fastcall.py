@@ -70,6 +70,16 @@ def test_plan_refuses_other_layouts():
     assert run(plan, *ts, 64, None, 0.25) is None and len(rec.calls) == 1
 
 
+def test_plan_takes_plain_scalars_only():
+    """A scalar that can change in place (a tensor) cannot be compared with the plan's value."""
+    from ascendc_kernel_amd import _fastcall
+    ts = [torch.zeros(4, 8, dtype=torch.bfloat16) for _ in range(4)]
+    call = (0, ctypes.cast(_Recorder().fn, ctypes.c_void_p).value, [0] * 14, 0.5)
+    for scalars, served in (((1, None, 0.5, True), True), ((1, torch.tensor(0.5)), False), (([1],), False)):
+        plan = _fastcall.make(tuple(ts), scalars, [call], [], [2, 3], 0, 0, None, 0)
+        assert (plan is not None) == served
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("h, d, v, m, n_kv, topk", [(64, 128, None, 40, 32, 16), (48, 128, None, 3, 700, 333),
                                                     (128, 576, 512, 1, 900, 300), (80, 576, 512, 67, 900, 128)])
@@ -123,3 +133,54 @@ def test_indexer_calls(kind, s, starts):
     if starts[0]:
         with pytest.raises((ValueError, RuntimeError)):
             model(x, qr, 513 - s, 0)
+
+
+def _attn_inputs(g, b, m, h, d, n_kv, topk):
+    return (torch.randn(b, m, h, d, generator=g, device="cuda", dtype=torch.bfloat16),
+            torch.randn(b, n_kv, d, generator=g, device="cuda", dtype=torch.bfloat16),
+            torch.randint(-1, n_kv, (b, m, topk), generator=g, device="cuda", dtype=torch.int32))
+
+
+def _ix_model(kind, g, table=512):
+    ql, dim, heads, hd, rd, ratio = (256, 1024, 16, 64, 32, 4) if kind == "indexer" else (1536, 7168, 64, 128, 64, 1)
+    a = t2.ModelArgs(max_batch_size=1, max_seq_len=table, dim=dim, index_n_heads=heads, index_head_dim=hd,
+                     index_topk=40, q_lora_rank=ql, rope_head_dim=rd)
+    cache = torch.randn(1, table // ratio, hd, generator=g, device="cuda", dtype=torch.bfloat16)
+    return lambda: t2.Model(a, t2.precompute_freqs_cis(rd, table), cache, ratio).to("cuda")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h, d, v, m, n_kv, topk", [(64, 128, None, 40, 32, 16), (128, 576, 512, 1, 900, 300)])
+def test_attention_scale_changes(h, d, v, m, n_kv, topk):
+    """A softmax_scale set between calls holds for the same and for new tensors."""
+    g = torch.Generator(device="cuda").manual_seed(h)
+    model, first = t1.Model(h, d, v).to("cuda"), _attn_inputs(g, 2, m, h, d, n_kv, topk)
+    others = _attn_inputs(g, 2, m, h, d, n_kv, topk)
+    for scale in (model.softmax_scale, 0.5, 0.01):
+        model.softmax_scale = scale
+        fresh = t1.Model(h, d, v).to("cuda")
+        fresh.softmax_scale = scale
+        for inputs in (first, first, others, first):
+            assert torch.equal(model(*inputs).view(torch.int16), fresh(*inputs).view(torch.int16)), scale
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["indexer", "dsa"])
+def test_indexer_scale_changes(kind):
+    """A softmax_scale set between calls holds for the same and for new tensors (a negative one
+    turns the order of the picks around)."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    make = _ix_model(kind, g)
+    model = make()
+    new = lambda: (torch.randn(1, 1, model.dim, generator=g, device="cuda", dtype=torch.bfloat16),
+                   torch.randn(1, 1, model.q_lora_rank, generator=g, device="cuda", dtype=torch.bfloat16), 500, 0)
+    first, others, picks = new(), new(), []
+    for scale in (model.softmax_scale, -model.softmax_scale):
+        model.softmax_scale = scale
+        fresh = make()
+        fresh.load_state_dict(model.state_dict())
+        fresh.softmax_scale = scale
+        for inputs in (first, first, others, first):
+            picks.append(model(*inputs))
+            assert torch.equal(picks[-1], fresh(*inputs)), scale
+    assert not torch.equal(picks[0], picks[4])

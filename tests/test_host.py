@@ -266,3 +266,48 @@ def test_task2_plan_cache(monkeypatch):
         m.weights_proj.weight.mul_(2)
     m(x.clone(), qr, 64, 5)
     assert len(built) == 5
+
+
+def test_plans_hold_module_scalars(monkeypatch):
+    """A scalar of the module changed between two calls with the same tensors prepares anew: the
+    launch's arguments hold its value (and a native plan is built from them)."""
+    from ascendc_kernel_amd import _native
+    log = []
+    _fake_native(monkeypatch, log)
+    monkeypatch.setattr(_native, "PLAN_DEVICE_TYPE", "cpu")
+    m = t1.Model(64, 128)
+    args = (torch.zeros(1, 40, 64, 128, dtype=torch.bfloat16), torch.zeros(1, 32, 128, dtype=torch.bfloat16),
+            torch.zeros(1, 40, 16, dtype=torch.int32))
+    for scale in (0.5, 0.25, torch.tensor(0.125), torch.tensor(0.125)):  # (the last: the same value)
+        m.softmax_scale = scale
+        m(*args)
+    assert log.count("prepare") == 3
+    m.softmax_scale.mul_(2)                            # the same object, another value
+    m(*args)
+    assert log.count("prepare") == 4
+    m.n_heads = 48
+    with pytest.raises(ValueError):                    # as a first call with this n_heads
+        m(*args)
+
+    built = []
+
+    class FakePlan:
+        def __init__(self, model, x, qr, start_pos, offset, key):
+            self.key = key
+            built.append(key)
+
+        def run(self):
+            return torch.zeros(1)
+
+    monkeypatch.setattr(t2, "_IndexerPlan", FakePlan)
+    freqs, cache = torch.ones(2600, 16, dtype=torch.complex64), torch.zeros(8, 650, 64, dtype=torch.bfloat16)
+    m = t2.Model(t2._make_args(), freqs, cache)
+    x, qr = torch.zeros(1, 64, 1024, dtype=torch.bfloat16), torch.zeros(1, 64, 256, dtype=torch.bfloat16)
+    m(x, qr, 0, 0)
+    for n, (name, value) in enumerate((("softmax_scale", 0.5), ("n_heads", 8), ("n_local_heads", 8), ("head_dim", 32),
+                                       ("rope_head_dim", 16), ("kv_cache", cache.view(torch.float16)),
+                                       ("freqs_cis", freqs.view(torch.float64)))):
+        setattr(m, name, value)
+        m(x, qr, 0, 0)
+        m(x, qr, 0, 0)
+        assert len(built) == n + 2, name
