@@ -243,7 +243,7 @@ class Model(nn.Module):
         self._plan = None
         self._packed = None
 
-    def route(self, x: torch.Tensor, qr: torch.Tensor) -> str:
+    def route(self, x: torch.Tensor, qr: torch.Tensor, start_pos: int = 0) -> str:
         """The projections' path for these inputs: 'splitk' (splitk_route), else what
         projection_route picks ('both', 'q', 'decode' or 'torch')."""
         wq, wp = self.wq_b.weight, self.weights_proj.weight
@@ -251,8 +251,11 @@ class Model(nn.Module):
                 x.shape[-1], wp.shape[0], qr.dtype == x.dtype == wq.dtype == wp.dtype == torch.bfloat16,
                 qr.is_cuda and x.is_cuda, qr.is_cuda and _measured_build(qr.device))
         if splitk_route(*args):
-            # (F.linear takes any alignment, the kernel 16 bytes; a copy made contiguous is aligned.)
-            if all(t.data_ptr() % 16 == 0 or not t.is_contiguous() for t in (x, qr, wq, wp, self.freqs_cis)):
+            # (F.linear takes any alignment, the kernel 16 bytes; a copy made contiguous is aligned.
+            # The table's rows of the call count, not its start: one row of a table with a wider row
+            # stride is contiguous as it is.)
+            rows = self.freqs_cis[start_pos:start_pos + qr.shape[1]]
+            if all(t.data_ptr() % 16 == 0 or not t.is_contiguous() for t in (x, qr, wq, wp, rows)):
                 return "splitk"
         return projection_route(*args)
 
@@ -365,7 +368,7 @@ class _IndexerPlan:
         freqs = model.freqs_cis[start_pos:end_pos]
         w_scale = model.softmax_scale * model.n_heads ** -0.5
         hd, rd, mode = model.head_dim, model.rope_head_dim, model.rope_mode
-        self.route = model.route(x, qr)
+        self.route = model.route(x, qr, start_pos)
         kv = model.kv_cache
         score_kw = dict(rope_head_dim=rd, n_cand=n_cand, k_out=k_out, ratio=ratio, causal=start_pos == 0,
                         offset=offset, rope_mode=mode)

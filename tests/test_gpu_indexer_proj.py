@@ -279,3 +279,34 @@ def test_model_splitk_route(gpu, b, s, start):
         torch.cuda.synchronize()
         assert torch.equal(got, ref) and torch.equal(model(x, qr, start, 0), ref)
         got.zero_()
+
+
+def _small_model(gpu, seed, freqs=None):
+    """A 16-head indexer for one sequence of 512 positions, and a decode step's inputs."""
+    from ascendc_kernel_amd import task2_indexer as t2
+    g = torch.Generator().manual_seed(seed)
+    a = t2.ModelArgs(max_batch_size=1, max_seq_len=512, dim=1024, index_n_heads=16, index_head_dim=64, index_topk=40,
+                     q_lora_rank=256, rope_head_dim=32)
+    kv = torch.randn(1, 128, 64, generator=g).to(torch.bfloat16).to(gpu)
+    if freqs is None:
+        freqs = t2.precompute_freqs_cis(32, 512, device=gpu)
+    model = t2.Model(a, freqs, kv, 4).to(gpu).requires_grad_(False)
+    for w in (model.wq_b.weight, model.weights_proj.weight):
+        w.copy_((torch.randn(w.shape, generator=g) * 0.02).to(gpu))
+    return model, torch.randn(1, 1, 1024, generator=g).to(torch.bfloat16).to(gpu), \
+        torch.randn(1, 1, 256, generator=g).to(torch.bfloat16).to(gpu)
+
+
+@pytest.mark.parametrize("cols", [17, 18])
+def test_model_strided_rope_table(gpu, cols):
+    """A RoPE table viewed from wider rows: one position's row is contiguous as it is, at an address
+    that F.linear's path takes and, every other position, the split-k launch does not."""
+    from ascendc_kernel_amd import task2_indexer as t2
+    plain = t2.precompute_freqs_cis(32, 512, device=gpu)
+    wide = torch.zeros(512, cols, dtype=torch.complex64, device=gpu)[:, :16].copy_(plain)
+    for start in (500, 501, 502, 503):
+        _say("strided table", cols, start)
+        model, x, qr = _small_model(gpu, start, wide)
+        want = _small_model(gpu, start, plain)[0](x, qr, start, 3)
+        for _ in range(3):
+            assert torch.equal(model(x, qr, start, 3), want)
