@@ -253,9 +253,11 @@ class Model(nn.Module):
         if splitk_route(*args):
             # (F.linear takes any alignment, the kernel 16 bytes; a copy made contiguous is aligned.
             # The table's rows of the call count, not its start: one row of a table with a wider row
-            # stride is contiguous as it is.)
+            # stride is contiguous as it is. The weights are read in place, not from a copy that a
+            # plan would keep and a write through .data would leave behind.)
             rows = self.freqs_cis[start_pos:start_pos + qr.shape[1]]
-            if all(t.data_ptr() % 16 == 0 or not t.is_contiguous() for t in (x, qr, wq, wp, rows)):
+            if (wq.is_contiguous() and wp.is_contiguous() and wq.data_ptr() % 16 == 0 and wp.data_ptr() % 16 == 0
+                    and all(t.data_ptr() % 16 == 0 or not t.is_contiguous() for t in (x, qr, rows))):
                 return "splitk"
         return projection_route(*args)
 

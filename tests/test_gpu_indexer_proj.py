@@ -310,3 +310,22 @@ def test_model_strided_rope_table(gpu, cols):
         want = _small_model(gpu, start, plain)[0](x, qr, start, 3)
         for _ in range(3):
             assert torch.equal(model(x, qr, start, 3), want)
+
+
+@pytest.mark.parametrize("which", ["wq_b", "weights_proj"])
+def test_model_strided_weights_read_live(gpu, which):
+    """Weights that are not contiguous are read as they are on each call, writes through .data
+    (which move no version counter) among them."""
+    _say("strided", which)
+    model, x, qr = _small_model(gpu, 11)
+    fresh, _, _ = _small_model(gpu, 11)
+    layer = getattr(model, which)
+    layer.weight = torch.nn.Parameter(layer.weight.t().contiguous().t(), requires_grad=False)
+    assert not layer.weight.is_contiguous()
+    first = fresh(x, qr, 500, 0)
+    assert torch.equal(model(x, qr, 500, 0), first) and torch.equal(model(x, qr, 500, 0), first)
+    for w in (layer.weight, getattr(fresh, which).weight):
+        w.data.neg_()
+    want = fresh(x, qr, 500, 0)
+    assert not torch.equal(want, first)
+    assert torch.equal(model(x, qr, 500, 0), want)
