@@ -7,7 +7,9 @@ anything another way.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
+import warnings
 from typing import Optional
 
 import torch
@@ -148,8 +150,27 @@ def load() -> ctypes.CDLL:
     v = lib.dsa_abi_version()
     if v != ABI_VERSION:
         raise RuntimeError(f"{path}: ABI version {v}, expected {ABI_VERSION}")
+    _load_fastcall()
     _lib = lib
     return lib
+
+
+def _load_fastcall() -> None:
+    """The extension behind fast_plan, with the library. It calls the library's entry points by
+    the signatures it was compiled against, so one of another ABI version is refused; without it
+    (a library given by DSA_MI355X_LIB, say) every call takes its Python path."""
+    global _fastcall, fast_run
+    try:
+        mod = importlib.import_module("ascendc_kernel_amd._fastcall")
+    except ImportError as e:
+        warnings.warn(f"_fastcall cannot be loaded ({e}): calls with layouts seen before take 4-100 us more host "
+                      "time; build it with `python -m ascendc_kernel_amd.build`", RuntimeWarning, stacklevel=3)
+        return
+    v = getattr(mod, "ABI_VERSION", None)
+    if v != ABI_VERSION:
+        raise RuntimeError(f"{_build.FASTCALL_PATH}: _fastcall has ABI version {v}, expected {ABI_VERSION}: "
+                           "build it with `python -m ascendc_kernel_amd.build`")
+    _fastcall, fast_run = mod, mod.run
 
 
 def _check(fn: str, code: int) -> None:
@@ -263,8 +284,9 @@ _fastcall = None
 
 
 def fast_run(plan, *args):
-    """The output of a call that `plan` (of fast_plan) serves, else None."""
-    return _fastcall.run(plan, *args)
+    """The output of a call that `plan` (of fast_plan) serves, else None (the extension's own
+    function once it is loaded)."""
+    return None
 
 
 def fast_plan(tensors, scalars, launches, patches, out_shape, out_like: int, temp_bytes: int, positions=None):
@@ -272,11 +294,10 @@ def fast_plan(tensors, scalars, launches, patches, out_shape, out_like: int, tem
     the marshalled `launches`: patches = [(launch, slot, tensor index or FAST_*, byte offset)]
     fill every pointer per call; the output has out_shape and the dtype of tensor out_like (-1:
     int64); temp_bytes of scratch are allocated per call. positions: an indexer's, whose calls
-    then end in start_pos and offset (struct Positions). None where a tensor cannot be served."""
-    global _fastcall, fast_run
+    then end in start_pos and offset (struct Positions). None where a tensor cannot be served, or
+    without the extension."""
     if _fastcall is None:
-        from . import _fastcall as mod
-        _fastcall, fast_run = mod, mod.run
+        return None
     calls = []
     for launch in launches:
         kind, at = _FAST_KIND[launch.name.replace("_i64", "")]

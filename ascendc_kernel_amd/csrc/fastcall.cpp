@@ -30,13 +30,17 @@
 #include <memory>
 #include <vector>
 
+#include "../../include/dsa_abi.h"
+
 namespace py = pybind11;
 
 namespace {
 
 constexpr int kMaxArgs = 24;
 
-// The C signatures of the entry points (include/dsa_abi.h), argument positions as there.
+// The entry points by their declarations in include/dsa_abi.h, argument positions as there. (The
+// _i64 ones, and dsa_indexer_decode_projections_rope of kProj, differ from the one called in what
+// pointers point to.)
 enum Kind { kAttn = 0, kMla = 1, kMlaWs = 2, kScore = 3, kScoreWs = 4, kProj = 5 };
 constexpr int kArgs[] = {14, 15, 17, 19, 21, 17};
 
@@ -49,35 +53,42 @@ struct Call {
   float f;  // the one float argument (its position in `a` is unused)
 };
 
+// A pointer argument, whatever it points to.
+struct Ptr {
+  int64_t v;
+  template <typename T>
+  operator T*() const {
+    return reinterpret_cast<T*>(static_cast<uintptr_t>(v));
+  }
+};
+
 int invoke(const Call& c) {
   const int64_t* a = c.a;
-  auto p = [a](int i) { return reinterpret_cast<void*>(static_cast<uintptr_t>(a[i])); };
-  using V = void*;
-  using I = int64_t;
+  auto p = [a](int i) { return Ptr{a[i]}; };
+  auto i32 = [a](int i) { return static_cast<int32_t>(a[i]); };
   switch (c.kind) {
     case kAttn:
-      return reinterpret_cast<int (*)(V, V, V, V, V, I, I, I, I, I, I, float, int32_t, V)>(c.fn)(
-          p(0), p(1), p(2), p(3), p(4), a[5], a[6], a[7], a[8], a[9], a[10], c.f, (int32_t)a[12], p(13));
+      return reinterpret_cast<decltype(&dsa_sparse_attn_fwd)>(c.fn)(
+          p(0), p(1), p(2), p(3), p(4), a[5], a[6], a[7], a[8], a[9], a[10], c.f, i32(12), p(13));
     case kMla:
-      return reinterpret_cast<int (*)(V, V, V, V, V, I, I, I, I, I, I, I, I, float, V)>(c.fn)(
+      return reinterpret_cast<decltype(&dsa_sparse_mla_fwd)>(c.fn)(
           p(0), p(1), p(2), p(3), p(4), a[5], a[6], a[7], a[8], a[9], a[10], a[11], a[12], c.f, p(14));
     case kMlaWs:
-      return reinterpret_cast<int (*)(V, V, V, V, V, I, I, I, I, I, I, I, I, float, V, I, V)>(c.fn)(
+      return reinterpret_cast<decltype(&dsa_sparse_mla_fwd_ws)>(c.fn)(
           p(0), p(1), p(2), p(3), p(4), a[5], a[6], a[7], a[8], a[9], a[10], a[11], a[12], c.f, p(14), a[15],
           p(16));
     case kScore:
-      return reinterpret_cast<int (*)(V, V, I, V, float, V, int32_t, V, I, I, I, I, I, I, I, I, int32_t, I, V)>(
-          c.fn)(p(0), p(1), a[2], p(3), c.f, p(5), (int32_t)a[6], p(7), a[8], a[9], a[10], a[11], a[12], a[13],
-                a[14], a[15], (int32_t)a[16], a[17], p(18));
+      return reinterpret_cast<decltype(&dsa_indexer_score_topk)>(c.fn)(
+          p(0), p(1), a[2], p(3), c.f, p(5), i32(6), p(7), a[8], a[9], a[10], a[11], a[12], a[13], a[14], a[15],
+          i32(16), a[17], p(18));
     case kScoreWs:
-      return reinterpret_cast<int (*)(V, V, I, V, float, V, int32_t, V, I, I, I, I, I, I, I, I, int32_t, I, V, I,
-                                      V)>(c.fn)(
-          p(0), p(1), a[2], p(3), c.f, p(5), (int32_t)a[6], p(7), a[8], a[9], a[10], a[11], a[12], a[13], a[14],
-          a[15], (int32_t)a[16], a[17], p(18), a[19], p(20));
+      return reinterpret_cast<decltype(&dsa_indexer_score_topk_ws)>(c.fn)(
+          p(0), p(1), a[2], p(3), c.f, p(5), i32(6), p(7), a[8], a[9], a[10], a[11], a[12], a[13], a[14], a[15],
+          i32(16), a[17], p(18), a[19], p(20));
     case kProj:
-      return reinterpret_cast<int (*)(V, V, V, int32_t, V, V, V, V, I, I, I, I, I, I, I, I, V)>(c.fn)(
-          p(0), p(1), p(2), (int32_t)a[3], p(4), p(5), p(6), p(7), a[8], a[9], a[10], a[11], a[12], a[13], a[14],
-          a[15], p(16));
+      return reinterpret_cast<decltype(&dsa_indexer_projections_splitk)>(c.fn)(
+          p(0), p(1), p(2), i32(3), p(4), p(5), p(6), p(7), a[8], a[9], a[10], a[11], a[12], a[13], a[14], a[15],
+          p(16));
   }
   return -1;
 }
@@ -309,5 +320,6 @@ PyMethodDef kRun = {"run", reinterpret_cast<PyCFunction>(reinterpret_cast<void (
 PYBIND11_MODULE(_fastcall, m) {
   m.def("make", &make);
   m.attr("MAX_TENSORS") = kMaxTensors;
+  m.attr("ABI_VERSION") = DSA_ABI_VERSION;
   m.add_object("run", py::reinterpret_steal<py::object>(PyCFunction_NewEx(&kRun, nullptr, nullptr)));
 }

@@ -2,6 +2,8 @@
 on the CPU with a recording C function as the launch, and the modules on the GPU against a fresh
 module's first call."""
 import ctypes
+import sys
+import types
 
 import pytest
 import torch
@@ -78,6 +80,33 @@ def test_plan_takes_plain_scalars_only():
     for scalars, served in (((1, None, 0.5, True), True), ((1, torch.tensor(0.5)), False), (([1],), False)):
         plan = _fastcall.make(tuple(ts), scalars, [call], [], [2, 3], 0, 0, None, 0)
         assert (plan is not None) == served
+
+
+@pytest.fixture
+def fresh_load(monkeypatch):
+    for name in ("_lib", "_fastcall"):
+        monkeypatch.setattr(_native, name, None)
+    monkeypatch.setattr(_native, "fast_run", _native.fast_run)
+
+
+def test_extension_absent(monkeypatch, fresh_load):
+    """Without the extension calls run, from the launches prepared in Python, and load() says so."""
+    monkeypatch.setitem(sys.modules, "ascendc_kernel_amd._fastcall", None)
+    with pytest.warns(RuntimeWarning, match="_fastcall"):
+        _native.load()
+    launch = _native.Launch("dsa_sparse_attn_fwd", [None] * 5 + [1] * 6 + [0.5, 0, None])
+    assert _native.fast_plan([torch.zeros(4, 8)], (), (launch,), [], [2, 3], 0, 0) is None
+
+
+def test_extension_of_another_abi(monkeypatch, fresh_load):
+    """An extension that was compiled against another version of the C ABI is refused."""
+    from ascendc_kernel_amd import _fastcall
+    assert _fastcall.ABI_VERSION == _native.ABI_VERSION
+    monkeypatch.setitem(sys.modules, "ascendc_kernel_amd._fastcall",
+                        types.SimpleNamespace(ABI_VERSION=_native.ABI_VERSION - 1))
+    for _ in range(2):
+        with pytest.raises(RuntimeError, match="_fastcall"):
+            _native.load()
 
 
 @pytest.mark.gpu
