@@ -85,16 +85,17 @@ def build(verbose: bool = False) -> str:
     os.makedirs(objdir, exist_ok=True)
     srcs = sources()
     objs = [os.path.join(objdir, os.path.basename(s)[:-4] + ".o") for s in srcs]
-    with _cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with _cf.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
         fast = ex.submit(_build_fastcall)
         list(ex.map(_compile, srcs, objs))
+        # Linked before the extension is waited for: the library is complete without it.
+        tmp = LIB_PATH + ".tmp"
+        cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"link failed:\n{r.stderr}")
+        os.replace(tmp, LIB_PATH)
         fast.result()
-    tmp = LIB_PATH + ".tmp"
-    cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError(f"link failed:\n{r.stderr}")
-    os.replace(tmp, LIB_PATH)
     if verbose:
         print(f"built {LIB_PATH} from {len(srcs)} sources", file=sys.stderr)
     return LIB_PATH

@@ -311,3 +311,22 @@ def test_plans_hold_module_scalars(monkeypatch):
         m(x, qr, 0, 0)
         m(x, qr, 0, 0)
         assert len(built) == n + 2, name
+
+
+def test_build_links_without_the_extension(monkeypatch):
+    """A failing compile of the extension is reported, with the library linked."""
+    import subprocess
+    from ascendc_kernel_amd import build
+    done = []
+
+    def broken():
+        raise RuntimeError("g++ failed")
+
+    monkeypatch.setattr(build, "_build_fastcall", broken)
+    monkeypatch.setattr(build, "_compile", lambda src, obj: None)
+    monkeypatch.setattr(build, "hipcc", lambda: "hipcc")
+    monkeypatch.setattr(build.subprocess, "run", lambda cmd, **kw: subprocess.CompletedProcess(cmd, 0, "", ""))
+    monkeypatch.setattr(build.os, "replace", lambda a, b: done.append(b))
+    with pytest.raises(RuntimeError, match="g\\+\\+ failed"):
+        build.build()
+    assert done == [build.LIB_PATH]
