@@ -289,6 +289,11 @@ def fast_run(plan, *args):
     return None
 
 
+def fast_serves(plan, *args) -> bool:
+    """Whether `plan` takes calls of these tensors and scalars."""
+    return _fastcall is not None and _fastcall.serves(plan, *args)
+
+
 def fast_plan(tensors, scalars, launches, patches, out_shape, out_like: int, temp_bytes: int, positions=None):
     """A native plan for calls whose tensors have these layouts and whose scalars are these, from
     the marshalled `launches`: patches = [(launch, slot, tensor index or FAST_*, byte offset)]

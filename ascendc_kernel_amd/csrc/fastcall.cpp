@@ -274,30 +274,38 @@ at::Tensor launch(const Plan& plan, const void* const* ptrs, int64_t start_pos, 
   return out;
 }
 
-// run(plan, tensors..., scalars..., [start_pos, offset]): the output, or None.
-PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  HANDLE_TH_ERRORS
+// The plan of args = (plan, tensors..., scalars..., ...) if the tensors' layouts (their pointers in
+// ptrs) and the scalars are its own, else null. positions: the call's two follow.
+const Plan* match(PyObject* const* args, Py_ssize_t nargs, const void** ptrs, bool positions) {
   const auto* plan = nargs > 0 ? static_cast<const Plan*>(PyCapsule_GetPointer(args[0], kCapsule)) : nullptr;
   if (plan == nullptr) {
     PyErr_Clear();
-    Py_RETURN_NONE;
+    return nullptr;
   }
-  const size_t nt = plan->tensors.size(), ns = plan->scalars.size(), np = plan->positioned ? 2 : 0;
+  const size_t nt = plan->tensors.size(), ns = plan->scalars.size(), np = positions && plan->positioned ? 2 : 0;
   if ((size_t)nargs != 1 + nt + ns + np || nt > kMaxTensors || c10::impl::dispatch_mode_enabled() ||
       at::impl::torch_function_mode_enabled())
-    Py_RETURN_NONE;
-  const void* ptrs[kMaxTensors];
+    return nullptr;
   for (size_t i = 0; i < nt; ++i) {
-    if (!THPVariable_CheckExact(args[1 + i])) Py_RETURN_NONE;
+    if (!THPVariable_CheckExact(args[1 + i])) return nullptr;
     const at::Tensor& t = THPVariable_Unpack(args[1 + i]);
-    if (!same(t, plan->tensors[i])) Py_RETURN_NONE;
+    if (!same(t, plan->tensors[i])) return nullptr;
     ptrs[i] = t.const_data_ptr();
   }
   for (size_t i = 0; i < ns; ++i)
-    if (!same(args[1 + nt + i], plan->scalars[i].ptr())) Py_RETURN_NONE;
+    if (!same(args[1 + nt + i], plan->scalars[i].ptr())) return nullptr;
+  return plan;
+}
+
+// run(plan, tensors..., scalars..., [start_pos, offset]): the output, or None.
+PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  const void* ptrs[kMaxTensors];
+  const Plan* plan = match(args, nargs, ptrs, true);
+  if (plan == nullptr) Py_RETURN_NONE;
   int64_t pos[2] = {0, 0};
-  for (size_t i = 0; i < np; ++i) {
-    PyObject* o = args[1 + nt + ns + i];
+  for (int i = 0; i < (plan->positioned ? 2 : 0); ++i) {
+    PyObject* o = args[nargs - 2 + i];
     int overflow = 0;
     if (!PyLong_CheckExact(o)) Py_RETURN_NONE;
     pos[i] = PyLong_AsLongLongAndOverflow(o, &overflow);
@@ -313,7 +321,17 @@ PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// serves(plan, tensors..., scalars...): whether run() takes these (positions aside).
+PyObject* serves(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  const void* ptrs[kMaxTensors];
+  return PyBool_FromLong(match(args, nargs, ptrs, false) != nullptr);
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef kRun = {"run", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(run)), METH_FASTCALL, nullptr};
+PyMethodDef kServes = {"serves", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(serves)),
+                       METH_FASTCALL, nullptr};
 
 }  // namespace
 
@@ -322,4 +340,5 @@ PYBIND11_MODULE(_fastcall, m) {
   m.attr("MAX_TENSORS") = kMaxTensors;
   m.attr("ABI_VERSION") = DSA_ABI_VERSION;
   m.add_object("run", py::reinterpret_steal<py::object>(PyCFunction_NewEx(&kRun, nullptr, nullptr)));
+  m.add_object("serves", py::reinterpret_steal<py::object>(PyCFunction_NewEx(&kServes, nullptr, nullptr)));
 }

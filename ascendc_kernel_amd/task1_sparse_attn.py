@@ -83,7 +83,10 @@ class Model(nn.Module):
                                 self.v_dim, self.variant, self.softmax_scale)
 
     def _learn(self, prepared: "_native.Prepared", q, kv, topk_idxs) -> None:
-        """Builds the native plan when two calls in a row had the same layouts."""
+        """Builds the native plan when two calls in a row that none served had the same layouts."""
+        if self._fast_scratch and _native.fast_serves(self._fast, q, kv, topk_idxs, self.attn_sink, self.n_heads,
+                                                      self.head_dim, self.v_dim, self.variant, self.softmax_scale):
+            return  # (not asked first for these tensors: forward)
         seen = (q.shape, kv.shape, topk_idxs.shape, topk_idxs.dtype, self.v_dim, self.variant)
         if self._seen != seen:
             self._seen = seen

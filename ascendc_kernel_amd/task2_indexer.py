@@ -311,8 +311,8 @@ class Model(nn.Module):
         self._fast = self._seen = None
 
     def _learn(self, plan: "_IndexerPlan", x: torch.Tensor, qr: torch.Tensor, start_pos: int) -> None:
-        """Builds the native plan when two calls in a row had the same layouts (one launch for
-        both projections from the weights in place, then the score kernel)."""
+        """Builds the native plan when two calls in a row that none served had the same layouts (one
+        launch for both projections from the weights in place, then the score kernel)."""
         kv, fc = self.kv_cache, self.freqs_cis
         seen = (x.shape, qr.shape, kv.shape, kv.stride(), fc.shape, start_pos == 0, self.rope_mode,
                 self.compress_ratio, self.index_topk)

@@ -213,3 +213,23 @@ def test_indexer_scale_changes(kind):
             picks.append(model(*inputs))
             assert torch.equal(picks[-1], fresh(*inputs)), scale
     assert not torch.equal(picks[0], picks[4])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h, d, v, m, n_kv, topk", [(64, 128, None, 40, 32, 16), (128, 576, 512, 1, 900, 300)])
+def test_one_plan_per_layout(monkeypatch, h, d, v, m, n_kv, topk):
+    """A layout that a native plan serves is not prepared or learned again, with the same
+    tensors, with new ones or with both in turn."""
+    g = torch.Generator(device="cuda").manual_seed(h)
+    built, fast_plan = [], _native.fast_plan
+    monkeypatch.setattr(_native, "fast_plan", lambda *a, **kw: built.append(a[4]) or fast_plan(*a, **kw))
+    model, first = t1.Model(h, d, v).to("cuda"), _attn_inputs(g, 2, m, h, d, n_kv, topk)
+    for _ in range(6):
+        model(*first)
+    for _ in range(3):
+        model(*_attn_inputs(g, 2, m, h, d, n_kv, topk))
+        model(*first)
+    assert len(built) == 1
+    for _ in range(3):                                   # another layout takes its place
+        model(*_attn_inputs(g, 1, m, h, d, n_kv, topk))
+    assert len(built) == 2
