@@ -307,8 +307,10 @@ def fast_plan(tensors, scalars, launches, patches, out_shape, out_like: int, tem
     for launch in launches:
         kind, at = _FAST_KIND[launch.name.replace("_i64", "")]
         values = [a.value or 0 for a in launch.args]
-        calls.append((kind, ctypes.cast(launch.fn, _c_vp).value, [int(v) for v in values],
-                      float(values[at]) if at is not None else 0.0))
+        scale = 0.0
+        if at is not None:  # (any float: infinities and NaN too)
+            scale, values[at] = float(values[at]), 0
+        calls.append((kind, ctypes.cast(launch.fn, _c_vp).value, values, scale))
     ws_fn = ctypes.cast(load().dsa_indexer_workspace_bytes, _c_vp).value
     return _fastcall.make(tuple(tensors), tuple(scalars), calls, list(patches), list(out_shape), out_like,
                           temp_bytes, positions, ws_fn)

@@ -109,6 +109,14 @@ def test_extension_of_another_abi(monkeypatch, fresh_load):
             _native.load()
 
 
+@pytest.mark.parametrize("scale", [float("inf"), float("nan"), -0.5])
+def test_plan_of_any_scale(scale):
+    """The float argument of a launch reaches the plan whatever its value."""
+    ts = [torch.zeros(4, 8, dtype=torch.bfloat16) for _ in range(4)]
+    launch = _native.Launch("dsa_sparse_attn_fwd", [None] * 5 + [1] * 6 + [scale, 0, None])
+    assert _native.fast_plan(ts, (), (launch,), [], [2, 3], 0, 0) is not None
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("h, d, v, m, n_kv, topk", [(64, 128, None, 40, 32, 16), (48, 128, None, 3, 700, 333),
                                                     (128, 576, 512, 1, 900, 300), (80, 576, 512, 67, 900, 128)])
