@@ -239,8 +239,8 @@ def _require_gpu(*ts: torch.Tensor) -> torch.device:
 
 class Prepared:
     """A checked, marshalled call and what it needs kept alive (inputs made contiguous,
-    workspaces, the fp32 sink copy). run() allocates the fresh output, patches its pointer
-    into the argument slot `out_slot` and launches."""
+    workspaces, the fp32 sink copy). run() allocates the fresh output, puts its pointer in the
+    argument slot `out_slot` and launches."""
     __slots__ = ("launch", "out_slot", "out_shape", "out_dtype", "device", "keep", "_like", "_proto")
 
     def __init__(self, launch: Launch, out_slot: int, out_shape, out_dtype, device, keep):
@@ -265,9 +265,11 @@ class Prepared:
             out = self._proto.new_empty(self.out_shape, dtype=self.out_dtype)
         else:
             out = torch.empty(self.out_shape, dtype=self.out_dtype, device=self.device)
+        # A list of the call's own: a launch that several threads run keeps its arguments.
         launch = self.launch
-        launch.args[self.out_slot].value = out.data_ptr()
-        rc = launch.fn(*launch.args)
+        args = launch.args.copy()
+        args[self.out_slot] = _c_vp(out.data_ptr())
+        rc = launch.fn(*args)
         if rc != 0:
             _check(launch.name, rc)
         return out

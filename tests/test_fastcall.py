@@ -3,7 +3,9 @@ on the CPU with a recording C function as the launch, and the modules on the GPU
 module's first call."""
 import ctypes
 import sys
+import threading
 import types
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 import torch
@@ -115,6 +117,48 @@ def test_plan_of_any_scale(scale):
     ts = [torch.zeros(4, 8, dtype=torch.bfloat16) for _ in range(4)]
     launch = _native.Launch("dsa_sparse_attn_fwd", [None] * 5 + [1] * 6 + [scale, 0, None])
     assert _native.fast_plan(ts, (), (launch,), [], [2, 3], 0, 0) is not None
+
+
+def test_plan_on_threads():
+    """Calls of one plan from several threads each launch with their own tensors."""
+    rec = _Recorder()
+    ts = [torch.zeros(4, 8, dtype=torch.bfloat16) for _ in range(4)]
+    run, plan = _cpu_plan(ts, rec)
+
+    def work(_):
+        for _ in range(50):
+            inputs = [t.clone() for t in ts]
+            out = run(plan, *inputs, 64, None, 0.25)
+            mine = [a for a in rec.calls if a[4] == out.data_ptr()][-1]
+            if mine[:4] != tuple(t.data_ptr() for t in inputs):
+                return False
+            kept.append((inputs, out))
+        return True
+
+    kept = []
+    with ThreadPoolExecutor(4) as pool:
+        assert all(pool.map(work, range(4)))
+    assert len({a[4] for a in rec.calls}) == 200
+
+
+def test_prepared_on_threads():
+    """A prepared launch run by two threads at once writes both outputs."""
+    barrier, seen = threading.Barrier(2), []
+
+    class FakeLaunch:
+        name = "fake"
+        args = [ctypes.c_void_p(0), ctypes.c_int64(7)]
+
+        @staticmethod
+        def fn(out, n):
+            barrier.wait(20)
+            seen.append((out.value, n.value))
+            return 0
+
+    prepared = _native.Prepared(FakeLaunch, 0, (4, 8), torch.bfloat16, torch.device("cpu"), ())
+    with ThreadPoolExecutor(2) as pool:
+        outs = list(pool.map(lambda _: prepared.run(), range(2)))
+    assert sorted(seen) == sorted((o.data_ptr(), 7) for o in outs)
 
 
 @pytest.mark.gpu
@@ -241,3 +285,29 @@ def test_one_plan_per_layout(monkeypatch, h, d, v, m, n_kv, topk):
     for _ in range(3):                                   # another layout takes its place
         model(*_attn_inputs(g, 1, m, h, d, n_kv, topk))
     assert len(built) == 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h, d, v, m, n_kv, topk", [(64, 128, None, 4, 700, 333), (128, 576, 512, 1, 900, 300)])
+def test_attention_on_threads(h, d, v, m, n_kv, topk):
+    """Calls of a known layout from four threads, each on a stream of its own, with tensors of
+    their own and with tensors they share."""
+    g = torch.Generator(device="cuda").manual_seed(h + m)
+    model = t1.Model(h, d, v).to("cuda")
+    shared = _attn_inputs(g, 2, m, h, d, n_kv, topk)
+    own = [_attn_inputs(g, 2, m, h, d, n_kv, topk) for _ in range(4)]
+    want = [t1.Model(h, d, v).to("cuda")(*i) for i in (shared, *own)]
+    for _ in range(3):
+        model(*shared)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(4)]
+
+    def work(n):
+        with torch.cuda.stream(streams[n]), torch.no_grad():
+            outs = [model(*(shared if i % 2 else own[n])) for i in range(40)]
+            streams[n].synchronize()
+        return all(torch.equal(o.view(torch.int16), want[0 if i % 2 else 1 + n].view(torch.int16))
+                   for i, o in enumerate(outs))
+
+    with ThreadPoolExecutor(4) as pool:
+        assert all(pool.map(work, range(4)))
