@@ -291,6 +291,12 @@ def fast_run(plan, *args):
     return None
 
 
+def fast_ready(dev: torch.device) -> bool:
+    """Whether plans serve calls on `dev` now (no extension, an active torch mode and another
+    current device keep every call on its Python path)."""
+    return _fastcall is not None and _fastcall.ready(dev.index)
+
+
 def fast_serves(plan, *args) -> bool:
     """Whether `plan` takes calls of these tensors and scalars."""
     return _fastcall is not None and _fastcall.serves(plan, *args)

@@ -274,6 +274,9 @@ at::Tensor launch(const Plan& plan, const void* const* ptrs, int64_t start_pos, 
   return out;
 }
 
+// An active dispatch or function mode sees every call of torch, so calls take the Python path.
+bool mode_active() { return c10::impl::dispatch_mode_enabled() || at::impl::torch_function_mode_enabled(); }
+
 // The plan of args = (plan, tensors..., scalars..., ...) if the tensors' layouts (their pointers in
 // ptrs) and the scalars are its own, else null. positions: the call's two follow.
 const Plan* match(PyObject* const* args, Py_ssize_t nargs, const void** ptrs, bool positions) {
@@ -283,9 +286,7 @@ const Plan* match(PyObject* const* args, Py_ssize_t nargs, const void** ptrs, bo
     return nullptr;
   }
   const size_t nt = plan->tensors.size(), ns = plan->scalars.size(), np = positions && plan->positioned ? 2 : 0;
-  if ((size_t)nargs != 1 + nt + ns + np || nt > kMaxTensors || c10::impl::dispatch_mode_enabled() ||
-      at::impl::torch_function_mode_enabled())
-    return nullptr;
+  if ((size_t)nargs != 1 + nt + ns + np || nt > kMaxTensors || mode_active()) return nullptr;
   for (size_t i = 0; i < nt; ++i) {
     if (!THPVariable_CheckExact(args[1 + i])) return nullptr;
     const at::Tensor& t = THPVariable_Unpack(args[1 + i]);
@@ -337,6 +338,8 @@ PyMethodDef kServes = {"serves", reinterpret_cast<PyCFunction>(reinterpret_cast<
 
 PYBIND11_MODULE(_fastcall, m) {
   m.def("make", &make);
+  // Whether calls of tensors on this device are served now, whatever their layout.
+  m.def("ready", [](int device) { return !mode_active() && c10::hip::current_device() == device; });
   m.attr("MAX_TENSORS") = kMaxTensors;
   m.attr("ABI_VERSION") = DSA_ABI_VERSION;
   m.add_object("run", py::reinterpret_steal<py::object>(PyCFunction_NewEx(&kRun, nullptr, nullptr)));

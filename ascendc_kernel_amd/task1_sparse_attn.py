@@ -73,7 +73,7 @@ class Model(nn.Module):
                         return out
                 plan = self._plan = (key, self._prepare(q, kv, topk_idxs))
             out = plan[1].run()
-            if dev.type == "cuda":
+            if dev.type == "cuda" and _native.fast_ready(dev):
                 self._learn(plan[1], q, kv, topk_idxs)
             return out
         return self._prepare(q, kv, topk_idxs).run()

@@ -289,7 +289,8 @@ class Model(nn.Module):
             if plan is None or plan.key != key:
                 plan = self._plan = _IndexerPlan(self, x, qr, start_pos, offset, key)
             out = plan.run()
-            if dev.type == "cuda" and plan.empty is None and plan.route in ("splitk", "decode"):
+            if (dev.type == "cuda" and plan.empty is None and plan.route in ("splitk", "decode")
+                    and type(start_pos) is int and type(offset) is int and _native.fast_ready(dev)):
                 self._learn(plan, x, qr, start_pos)
             return out
         return _IndexerPlan(self, x, qr, start_pos, offset, None).run()

@@ -7,6 +7,7 @@ import threading
 import types
 from concurrent.futures import ThreadPoolExecutor
 
+import numpy as np
 import pytest
 import torch
 
@@ -311,3 +312,26 @@ def test_attention_on_threads(h, d, v, m, n_kv, topk):
 
     with ThreadPoolExecutor(4) as pool:
         assert all(pool.map(work, range(4)))
+
+
+@pytest.mark.gpu
+def test_nothing_learned_for_calls_not_served(monkeypatch):
+    """Under an active torch mode, and for positions that are no plain ints, no plan serves a call
+    and none is built."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    built, fast_plan = [], _native.fast_plan
+    monkeypatch.setattr(_native, "fast_plan", lambda *a, **kw: built.append(a[4]) or fast_plan(*a, **kw))
+    attn, inputs = t1.Model(64, 128).to("cuda"), _attn_inputs(g, 2, 40, 64, 128, 32, 16)
+    ix = _ix_model("indexer", g)()
+    x = torch.randn(1, 1, 1024, generator=g, device="cuda", dtype=torch.bfloat16)
+    qr = torch.randn(1, 1, 256, generator=g, device="cuda", dtype=torch.bfloat16)
+    want, picks = attn(*inputs), ix(x, qr, 500, 0)
+    with torch.device("cuda"):
+        for _ in range(4):
+            assert torch.equal(attn(*inputs), want) and torch.equal(ix(x, qr, 500, 0), picks)
+    for _ in range(4):
+        assert torch.equal(ix(x, qr, np.int64(500), 0), picks)
+    assert not built
+    for _ in range(2):
+        attn(*inputs), ix(x, qr, 500, 0)
+    assert len(built) == 2
