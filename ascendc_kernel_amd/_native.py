@@ -258,6 +258,12 @@ class Prepared:
                                and proto.dtype == out_dtype and proto.is_contiguous()) else None
         self._proto = proto
 
+    def forget(self, *tensors: torch.Tensor) -> None:
+        """Keeps these no longer: every call sets the pointers to them anew. (Further outputs are
+        allocated from the first tensor that stays.)"""
+        self.keep = tuple(k for k in self.keep if not any(k is t for t in tensors))
+        self._like, self._proto = None, self.keep[0]
+
     def run(self) -> torch.Tensor:
         if self._like is not None:
             out = torch.empty_like(self._like)

@@ -104,6 +104,8 @@ class Model(nn.Module):
         self._fast = _native.fast_plan(
             (q, kv, topk_idxs, sink), (self.n_heads, self.head_dim, self.v_dim, self.variant, self.softmax_scale),
             (launch,), patches, prepared.out_shape, 0, ws[0].numel() if ws else 0)
+        if self._fast is not None and not ws:
+            self._plan = None  # not asked again for this layout, so the inputs need not stay
 
     def _prepare(self, q: torch.Tensor, kv: torch.Tensor, topk_idxs: torch.Tensor) -> "_native.Prepared":
         if q.dim() != 4 or q.shape[2] != self.n_heads or q.shape[3] != self.head_dim:

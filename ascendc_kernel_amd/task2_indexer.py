@@ -347,6 +347,10 @@ class Model(nn.Module):
             tensors, (self.rope_mode, self.compress_ratio, self.index_topk, self.n_heads, self.n_local_heads,
                       self.head_dim, self.rope_head_dim, self.softmax_scale),
             (plan.proj, score), patches, plan.score.out_shape, -1, ws_off, positions)
+        if self._fast is not None and splitk:
+            # Not asked again for this layout, so x and qr need not stay. (A 'decode' plan's buffers
+            # do: a graph that captured one of its calls reads them.)
+            self._plan = None
 
 
 class _IndexerPlan:
@@ -391,6 +395,7 @@ class _IndexerPlan:
             if splitk:  # q and wl of a call: one fresh buffer, wl after q (whole 2 KB rows)
                 self.q_bytes = 2 * q.numel()
                 self.qwl_words = q.numel() + wl.numel()
+                self.score.forget(q, wl)
             else:
                 self.q, self.wl = q, wl
                 self.proj.set(_native.PROJ_SLOT_Q, q.data_ptr())

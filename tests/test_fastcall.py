@@ -335,3 +335,23 @@ def test_nothing_learned_for_calls_not_served(monkeypatch):
     for _ in range(2):
         attn(*inputs), ix(x, qr, 500, 0)
     assert len(built) == 2
+
+
+@pytest.mark.gpu
+def test_indexer_keeps_no_buffers():
+    """A module on the split-k route holds no q, no head weights and no inputs between calls."""
+    g = torch.Generator(device="cuda").manual_seed(9)
+    model = _ix_model("indexer", g, 8192)()
+    new = lambda: (torch.randn(1, 8192, 1024, generator=g, device="cuda", dtype=torch.bfloat16),
+                   torch.randn(1, 8192, 256, generator=g, device="cuda", dtype=torch.bfloat16), 0, 0)
+    new()
+    before = torch.cuda.memory_allocated()
+    for call in range(3):
+        inputs = new()
+        assert model.route(*inputs[:2]) == "splitk" or call > 2
+        out = model(*inputs)
+        held = torch.cuda.memory_allocated() - before - sum(t.nbytes for t in (*inputs[:2], out))
+        assert held < 1 << 20, (call, held)
+        del out, inputs
+    torch.cuda.synchronize()
+    assert torch.cuda.memory_allocated() - before < 1 << 20
