@@ -5,7 +5,7 @@ and write tests/golden/projection_ranges.json.
 
 Run on an MI355X box (it needs torch-ROCm on a GPU and the built library):
     python tests/golden/measure_projection_ranges.py [mmax] [out.json]
-(mmax 0: only the split-k part, the rest of out.json kept.)
+(mmax 0: only the split-k part; the rest of out.json is kept, which has to be of the same build.)
 For m = 17 .. mmax (default 131072) it runs dsa_indexer_projections (q = qr . wq_b^T without
 RoPE, k = 256, n = 1024; wl = x . weights_proj^T, k = 1024, n = 16) on windows of one set
 of random inputs and compares each output tensor with F.linear. hipBLASLt chooses its
@@ -77,14 +77,24 @@ def sweep(kernel, wq, wp, qr, x, lo, hi):
     return bad.cpu()
 
 
+def kept_ranges(path, build):
+    """The file's intervals, if they were measured on this torch build and CU count."""
+    with open(path) as f:
+        res = json.load(f)
+    if any(res.get(k) != v for k, v in build.items()):
+        raise SystemExit(f"{path} holds measurements of {({k: res.get(k) for k in build})}, this is {build}: "
+                         "measure all counts")
+    return res
+
+
 def main():
     mmax = int(sys.argv[1]) if len(sys.argv) > 1 else 131072
     path = sys.argv[2] if len(sys.argv) > 2 else os.path.join(HERE, "projection_ranges.json")
     dev = torch.device("cuda:0")
-    res = {}
+    build = {"torch": torch.__version__, "hip": torch.version.hip,
+             "cus": torch.cuda.get_device_properties(dev).multi_processor_count}
     if mmax == 0:
-        with open(path) as f:
-            res = json.load(f)
+        res = kept_ranges(path, build)
     else:
         wq, wp, qr, x = inputs(mmax, dev)
         pq, pw = _native.pack_projection_weights(wq, wp)
@@ -93,9 +103,7 @@ def main():
     wq, wp, qr, x = inputs(SPLITK_MMAX, dev)
     bad = sweep(lambda a, b: _native.indexer_projections(a, wq, None, b, wp, 64, 32, splitk=True), wq, wp, qr, x,
                 1, SPLITK_MMAX)
-    res.update({"torch": torch.__version__, "hip": torch.version.hip,
-                "cus": torch.cuda.get_device_properties(dev).multi_processor_count,
-                "splitk_mmax": SPLITK_MMAX, "splitk_equal": intervals(bad.any(1), 1, SPLITK_MMAX)})
+    res.update({**build, "splitk_mmax": SPLITK_MMAX, "splitk_equal": intervals(bad.any(1), 1, SPLITK_MMAX)})
     with open(path, "w") as f:
         json.dump(res, f, indent=1)
     print(path, "q intervals", len(res["q_equal"]), "wl intervals", len(res["wl_equal"]),

@@ -330,3 +330,22 @@ def test_build_links_without_the_extension(monkeypatch):
     with pytest.raises(RuntimeError, match="g\\+\\+ failed"):
         build.build()
     assert done == [build.LIB_PATH]
+
+
+def test_projection_ranges_keep_their_build(tmp_path):
+    """A run that measures the split-k counts only keeps the other intervals of the file only
+    where they were measured on the same build and CU count."""
+    import importlib.util
+    import json
+    import os
+    from conftest import GOLDEN
+    spec = importlib.util.spec_from_file_location("measure_ranges", os.path.join(GOLDEN, "measure_projection_ranges.py"))
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    path = tmp_path / "ranges.json"
+    build = {"torch": "a", "hip": "b", "cus": 256}
+    path.write_text(json.dumps({**build, "mmax": 9, "q_equal": [[1, 2]], "wl_equal": []}))
+    assert mod.kept_ranges(str(path), build)["q_equal"] == [[1, 2]]
+    for other in ({"torch": "c"}, {"hip": "c"}, {"cus": 304}):
+        with pytest.raises(SystemExit):
+            mod.kept_ranges(str(path), {**build, **other})
