@@ -3,12 +3,12 @@
 // of sparse_attn_ref, reference/task1_v0_ref.py:5-24; duplicates and masked
 // slots handled exactly like the gather there).
 //
-// Two kernels, chosen by gather_split: this file's sa_gather_kernel (many tokens of more
-// than 32 heads) and sa_gather_split_kernel (few tokens, or at most 32 heads). The former:
+// Two kernels, chosen by gather_split: sa_gather_kernel (many tokens of more than 32
+// heads) and sa_gather_split_kernel (few tokens, or at most 32 heads). The former:
 // one workgroup per token, one wave per 32 heads (ceil(h/32) waves). The slots are
 // processed in blocks of 32. The selected kv rows (256 B each) of a block are
 // copied straight from global memory into LDS by global_load_lds_dwordx4 (no
-// register staging), into a ring of kRing block buffers: one block is in flight while
+// register staging), into a ring of kRing block buffers: one or two blocks are in flight while
 // the scores of the next and the products of the current one are computed. Every wave then runs
 //   S^T[32 keys x 32 heads]  = K[32 x 128] . Q^T[128 x 32]   (8 x mfma 32x32x16)
 //   online softmax with the sink as the initial maximum (log2 domain)
@@ -29,7 +29,6 @@ namespace {
 
 constexpr int kD = 128;
 constexpr int kKB = 32;          // slots per block
-constexpr int kRing = 3;         // LDS block buffers (one block in flight beside the two in use)
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kRaise = 8.0f;   // log2 headroom before the running max is raised
 // bf16 pairs (-1, 0) and (0, -1) as bit patterns: dot2(h, neg_lo, p0) = p0 - h.lo,
@@ -64,17 +63,22 @@ __device__ __forceinline__ int out_ch(int dt, int i) {
 __device__ __forceinline__ int swz(int r, int c) { return r * 16 + (c ^ (r & 15)); }
 
 // Bound by the matrix cores and the VALU (per block and wave 24 products, ~770 cycles, and
-// ~700 cycles of softmax), which overlap only across the waves of a SIMD, so the kernel
-// keeps three there: at most 168 VGPRs (fragment addresses come from one register each by
-// xor, mask bits and copy offsets are formed at their use) and a ring of three. Against two
-// waves at 214 VGPRs and a ring of four: configs[3] 397-412 -> 383-388 us (1.0 PFLOP/s of
-// issued products), 3 x 421 tokens x 48 heads, 333 slots 31.0 -> 26.6, 4096 tokens x 96
-// heads, 256 slots 103 -> 83-85, 4000 x 128 heads, 2048 slots 650 -> 650. The same registers
-// at two waves per SIMD: no change. No s_setprio, or the raised priority on the products
-// instead: 1-3 % slower.
-template <int NW, typename IdxT>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 3)))
+// ~700 cycles of softmax), which overlap only across the waves of a SIMD. Two forms, chosen by
+// gather_ring:
+//  kRing 3: three waves per SIMD, so at most 168 VGPRs (fragment addresses come from one
+//    register each by xor, mask bits and copy offsets are formed at their use, V fragments are
+//    read one ahead in a pinned order) and a ring of three. 4 x 4096 tokens x 64 heads, 512
+//    slots 397-412 -> 383-388 us (1.0 PFLOP/s of issued products), 3 x 421 tokens x 48 heads,
+//    333 slots 31.0 -> 26.6, 4096 tokens x 96 heads, 256 slots 103 -> 83-85;
+//  kRing 4: two waves per SIMD (196 VGPRs) with the offsets held, the order of the V reads
+//    left to the compiler and one more block in flight, for grids that leave two waves or
+//    fewer on a SIMD: 300 tokens x 64 heads, 1024 slots 35.2 -> 33.3 us.
+// The three-wave form's registers at two waves per SIMD: no change. No s_setprio, or the raised
+// priority on the products instead: 1-3 % slower.
+template <int NW, typename IdxT, int kRing>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kRing == 3 ? 3 : 2, kRing == 3 ? 3 : 2)))
 void sa_gather_kernel(GatherParams p) {
+  static_assert(kRing == 3 || kRing == 4, "one or two blocks in flight beside the two in use");
   const IdxT* const idx = static_cast<const IdxT*>(p.idx);
   // kRing blocks of 32 gathered rows (8 KB each); at the end one 8 KB area per wave. 1 KB
   // alignment: fragment addresses inside a block are formed by xor.
@@ -164,10 +168,14 @@ void sa_gather_kernel(GatherParams p) {
   // the row, the unit entering as a scalar. They are recomputed from the lane id at each
   // use: held across the block loop they would spill.
   const uint32_t slot_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int32_t*)slot;
-  auto lane_id = [] {
-    int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-    asm volatile("" : "+v"(ln));
-    return ln;
+  auto lane_id = [&] {
+    if constexpr (kRing == 4) {
+      return lane;
+    } else {
+      int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+      asm volatile("" : "+v"(ln));
+      return ln;
+    }
   };
   auto unit = [&](int i) {
     const int u = wis + NW * i;
@@ -211,7 +219,7 @@ void sa_gather_kernel(GatherParams p) {
   auto qk = [&](const int j) {
     f32x16 acc = {};
     uint32_t kb_ = kbase;
-    asm volatile("" : "+v"(kb_));
+    if constexpr (kRing == 3) asm volatile("" : "+v"(kb_));
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
       const bf16x8 a = __builtin_bit_cast(bf16x8, *(lds_cu32x4_ptr)(uintptr_t)((kb_ ^ (32u * ks)) + 8192u * j));
@@ -248,8 +256,8 @@ void sa_gather_kernel(GatherParams p) {
   // Two-stage pipeline: iteration kb computes S of block kb+1 on the matrix
   // cores while the VALU runs the softmax of block kb, then O += P(kb) V(kb).
   // Block kb+1 must be in LDS at the start of iteration kb, block kb is read
-  // until its end; the copy issued in iteration kb (block kb+2) goes to the
-  // buffer of block kb-1, released by the barrier.
+  // until its end; the copy issued in iteration kb (block kb + kRing - 1) goes to
+  // the buffer of block kb-1, released by the barrier.
   // One iteration for block kb, which sits in ring buffer j = kb % kRing (the
   // loop is unrolled by kRing so that j, and with it every LDS offset below,
   // is a compile-time constant).
@@ -265,7 +273,9 @@ void sa_gather_kernel(GatherParams p) {
   auto step = [&](const int kb, const int j) {
     uint32_t vm_next = 0u;
     if (kb + 1 < nb) {
-      wait_vmcnt<0>();  // block kb+1 has landed (kb+2 is issued below)
+      // Block kb+1 has landed once at most the younger blocks issued so far are outstanding.
+      if (kRing == 4 && kb + 2 < nb) wait_vmcnt<kUnits>();
+      else wait_vmcnt<0>();
       __syncthreads();  // block kb+1 is in LDS for every wave; block kb-1 is consumed
       if (kb + kRing - 1 < nb) issue((j + kRing - 1) % kRing, rv);
       vm_next = (uint32_t)__ballot(vslot >= 0);
@@ -340,7 +350,7 @@ void sa_gather_kernel(GatherParams p) {
     // One fragment is read ahead of its two products (the order is pinned below).
     __builtin_amdgcn_s_setprio(0);
     uint32_t vb_ = vbase;
-    asm volatile("" : "+v"(vb_));
+    if constexpr (kRing == 3) asm volatile("" : "+v"(vb_));
     auto rdv = [&](int i) {
       const int st = i >> 2, dt = i & 3;
       const uint32_t at = 8192u * j + 4096u * st;
@@ -359,19 +369,22 @@ void sa_gather_kernel(GatherParams p) {
       o[i & 3] = mfma32x32x16(va, phi[i >> 2], o[i & 3]);
       va = vn;
     }
-    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-#pragma unroll
-    for (int i = 0; i < 7; ++i) {
+    if constexpr (kRing == 3) {
       __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+      for (int i = 0; i < 7; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      }
       __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
     s_cur = s_next;
     vm_cur = vm_next;
   };
 
   if (nb > 0) {
-    if (nb >= 2) wait_vmcnt<kUnits>();
+    if (kRing == 4 && nb >= 3) wait_vmcnt<2 * kUnits>();
+    else if (nb >= 2) wait_vmcnt<kUnits>();
     else wait_vmcnt<0>();
     __syncthreads();
     vm_cur = (uint32_t)__ballot(vslot >= 0);
@@ -429,7 +442,7 @@ void sa_gather_kernel(GatherParams p) {
 // after the other (~0.8 us each), which the split divides; 8 tokens of 64 heads, 512 slots
 // of 8192 rows: 16.4 us with the blocks in sequence (sa_gather_kernel), 8.3 us with SP 4;
 // 2048 slots: 52.9 us, 17.1 us with SP 8. With many tokens SP 1 serves up to 32 heads:
-// 17 KB of LDS per wave instead of the 4-buffer ring's 33 KB keeps two waves on each SIMD
+// 17 KB of LDS per wave instead of a 4-buffer ring's 33 KB keeps two waves on each SIMD
 // (4,800 tokens of 16 heads, 256 slots: 57.1 -> 42.4 us). SP 2 was the best choice
 // nowhere by more than 8 %.
 constexpr int kSplitRing = 2;
@@ -715,16 +728,42 @@ void sa_gather_split_kernel(GatherParams p) {
 //    (64 slots: 5.8 -> 5.1);
 //  up to two groups per CU, 4 waves from 8 blocks on (512 slots, 512 groups: 16.8 -> 13.1);
 //    with fewer blocks the states cost what the split saves (128 slots: 7.7 -> 8.4);
-//  beyond that, 64 and more heads stay sequential, where the waves of a token share each
+//  beyond that, more than 32 heads stay sequential, where the waves of a token share each
 //    row's copy (512 slots, 1536 groups: 23.3, one wave 27.6), and up to 32 heads take one
 //    wave (512 slots, 8192 groups: 153.8 -> 108), or 4 where the slot list would leave
 //    room for fewer than 7 one-wave workgroups per CU (2048 slots, 3072 groups: one wave
 //    181, four 169).
+// Masked slots are not known here: where one block of a long list is valid the split costs up to
+// 1.7 us (8 tokens x 64 heads, 10 of 1024 slots 5.7 -> 7.3; 100 of them 7.9 -> 7.4).
 int gather_split(int64_t groups, int nw, int64_t nblk, int cu) {
   if (groups <= cu) return nblk >= 32 ? 8 : nblk >= 4 ? 4 : 1;
   if (groups <= 2 * (int64_t)cu && nblk >= 8) return 4;
   if (nw > 1) return 0;
   return nblk >= 48 ? 4 : 1;
+}
+
+// The form of sa_gather_kernel (kRing) for `tokens` workgroups of nw waves on cu CUs. The
+// three-wave form holds 12 waves per CU (6, 4, 3 workgroups of 2, 3, 4 waves) and the two-wave
+// form 8 (4, 2, 2), which a CU works off in 1.2 (32 slots) to 1.5 times (from 512) less time, so
+// what counts is in how many rounds the grid fits. Measured at 300 .. 8000 tokens and 32 .. 2048
+// slots (256 CUs; us, two waves -> three):
+//  one round of the two-wave form: that one (300 tokens x 64 heads, 1024 slots 33.3 -> 35.2;
+//    400 x 96, 512 20.7 -> 21.5; 400 x 128, 256 14.2 -> 14.9);
+//  4 waves, 3 to 4 tokens per CU: two rounds of either, two-wave (900 x 128, 2048 slots 157 ->
+//    169), else three waves (640: 136 -> 116; 4000, 512 slots: 197 -> 184);
+//  3 waves: three waves (900 x 96, 512 slots: 43 -> 38);
+//  2 waves: above 544 slots the slot list leaves LDS for five workgroups of the three-wave
+//    form, unevenly over the four SIMDs: two-wave (4000 x 64, 1024 slots: 184 -> 198; 1500: 81 ->
+//    89), but for the last block count, where it has room for three workgroups only and the
+//    three-wave form for four (900 x 64, 2048 slots: 126 -> 87; 1200: 136 -> 160). Up to 544
+//    slots three waves (1500 x 64, 512 slots: 47 -> 41; 8000: 201 -> 194) but where their second
+//    round is nearly empty (2000, 512 slots: 54 -> 58; 4 x 500 causal, 32 slots: 17.5 -> 20.9).
+int gather_ring(int64_t tokens, int nw, int64_t nblk, int cu) {
+  const auto rounds = [&](int per_cu) { return (tokens + per_cu * (int64_t)cu - 1) / (per_cu * (int64_t)cu); };
+  if (nw > 2) return tokens <= 2 * (int64_t)cu || (nw == 4 && rounds(3) == 2 && rounds(4) == 1) ? 4 : 3;
+  if (nblk == 64) return 4 * rounds(4) < 3 * rounds(3) ? 3 : 4;
+  if (nblk > 17 || rounds(4) == 1) return 4;
+  return rounds(6) == 2 && tokens < 8 * (int64_t)cu ? 4 : 3;
 }
 
 template <typename IdxT>
@@ -739,6 +778,26 @@ int launch_split(const GatherParams& p, int sp, unsigned blocks, size_t smem, hi
     DSA_GATHER_CASE(1)
     DSA_GATHER_CASE(4)
     DSA_GATHER_CASE(8)
+#undef DSA_GATHER_CASE
+    default:
+      return DSA_ERR_UNSUPPORTED;
+  }
+  return hipGetLastError() == hipSuccess ? DSA_OK : DSA_ERR_LAUNCH;
+}
+
+template <typename IdxT>
+int launch_ring(const GatherParams& p, int ring, int nw, unsigned tokens, size_t smem, hipStream_t stream) {
+  switch (4 * nw + ring) {
+#define DSA_GATHER_CASE(n, r)                                                                          \
+  case 4 * n + r:                                                                                      \
+    hipLaunchKernelGGL((sa_gather_kernel<n, IdxT, r>), dim3(tokens), dim3(64 * n), smem, stream, p);   \
+    break;
+    DSA_GATHER_CASE(2, 3)
+    DSA_GATHER_CASE(3, 3)
+    DSA_GATHER_CASE(4, 3)
+    DSA_GATHER_CASE(2, 4)
+    DSA_GATHER_CASE(3, 4)
+    DSA_GATHER_CASE(4, 4)
 #undef DSA_GATHER_CASE
     default:
       return DSA_ERR_UNSUPPORTED;
@@ -784,19 +843,7 @@ int dsa_sparse_attn_gather_launch(const void* q, const void* kv, const void* idx
     return idx64 ? launch_split<int64_t>(p, sp, (unsigned)blocks, smem, stream)
                  : launch_split<int32_t>(p, sp, (unsigned)blocks, smem, stream);
   }
-  const dim3 grid((unsigned)tokens);
-  if (idx64) {
-    switch (nw) {
-      case 2: hipLaunchKernelGGL((sa_gather_kernel<2, int64_t>), grid, dim3(128), smem, stream, p); break;
-      case 3: hipLaunchKernelGGL((sa_gather_kernel<3, int64_t>), grid, dim3(192), smem, stream, p); break;
-      default: hipLaunchKernelGGL((sa_gather_kernel<4, int64_t>), grid, dim3(256), smem, stream, p); break;
-    }
-  } else {
-    switch (nw) {
-      case 2: hipLaunchKernelGGL((sa_gather_kernel<2, int32_t>), grid, dim3(128), smem, stream, p); break;
-      case 3: hipLaunchKernelGGL((sa_gather_kernel<3, int32_t>), grid, dim3(192), smem, stream, p); break;
-      default: hipLaunchKernelGGL((sa_gather_kernel<4, int32_t>), grid, dim3(256), smem, stream, p); break;
-    }
-  }
-  return hipGetLastError() == hipSuccess ? DSA_OK : DSA_ERR_LAUNCH;
+  const int ring = gather_ring(tokens, nw, nblk, cu);
+  return idx64 ? launch_ring<int64_t>(p, ring, nw, (unsigned)tokens, smem, stream)
+               : launch_ring<int32_t>(p, ring, nw, (unsigned)tokens, smem, stream);
 }

@@ -297,6 +297,24 @@ def test_gather_split_edges(gpu, case):
     assert torch.equal(out64.view(torch.int16), out.view(torch.int16))
 
 
+# One workgroup per token: both rings on either side of each line of their rule (256 CUs), with the
+# slot blocks at the ends of the pipeline (1, 2, 3, 4 and 5 blocks).
+RING_CASES = [
+    # b, m, h, n_kv, topk
+    (1, 300, 64, 400, 1), (1, 300, 64, 400, 64), (1, 1024, 48, 400, 65), (1, 1025, 48, 400, 128), (1, 1536, 64, 400, 129),
+    (1, 1537, 64, 400, 33), (2, 1024, 64, 400, 97), (3, 700, 64, 400, 31), (1, 1100, 64, 900, 544),
+    (1, 1100, 64, 900, 545), (1, 900, 64, 2500, 2017), (1, 513, 96, 400, 96), (1, 512, 80, 400, 97),
+    (1, 512, 128, 400, 130), (1, 513, 112, 400, 64), (1, 769, 128, 400, 33), (1, 1025, 128, 400, 97),
+]
+
+
+@pytest.mark.parametrize("case", RING_CASES)
+def test_gather_ring_edges(gpu, case):
+    """Both forms of the one-workgroup-per-token kernel against the oracle, with whole blocks
+    masked, a token without any slot, and int64 slots giving the int32 result bit for bit."""
+    test_gather_split_edges(gpu, case)
+
+
 @pytest.mark.parametrize("variant", [_native.DSA_SA_GATHER, _native.DSA_SA_MULTIPLICITY])
 def test_neg_inf_sink_masked_leading_block(gpu, variant):
     """A -inf sink on half the heads with the first slot blocks of every token masked: no
