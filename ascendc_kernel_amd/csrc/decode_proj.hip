@@ -27,7 +27,9 @@
 //
 // The wl workgroups come first in the grid, so they start before the q ones. The weights
 // are read with plain loads: non-temporal ones bypass what the MALL holds of them (16
-// tokens 13.8 -> 9.7 us with one layer's weights, 14.2 -> 10.0 with four layers' in turn).
+// tokens 13.8 -> 9.7 us with one layer's weights, 14.2 -> 10.0 with four layers' in turn). With
+// 48 layers' in turn (1.25 GB, which no cache holds) plain loads are still the faster ones from
+// 5 tokens (5: 12.9 -> 11.7 us, 16: 15.4 -> 13.7) and 0.1-0.2 us behind up to 4 (1: 8.5 -> 8.8).
 // Up to 4 tokens take a finer work split (ix_decode_proj_few_kernel).
 #include "dsa_common.h"
 

@@ -24,7 +24,7 @@ class Model(nn.Module):
     #: kernel choice passed to the C ABI (auto = multiplicity kernel when n_kv <= 32)
     variant: int = _native.DSA_SA_AUTO
     # The native plan that serves further calls with the last calls' layouts (and whether it
-    # takes scratch memory), and the layout seen last on the way to building one.
+    # takes scratch memory), and the layout that the last call it did not serve had.
     _fast = None
     _fast_scratch = False
     _seen = None

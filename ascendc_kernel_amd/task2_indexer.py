@@ -216,7 +216,7 @@ class Model(nn.Module):
     #: which torch rounding of the RoPE complex product to reproduce
     rope_mode: int = _native.DSA_ROPE_TORCH_ROCM
     # The native plan that serves further calls with the last calls' layouts, and the layout
-    # seen last on the way to building one.
+    # that the last call it did not serve had.
     _fast = None
     _seen = None
 
