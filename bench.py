@@ -363,10 +363,10 @@ def main():
             _warm(torch, stepd, 2, 0.05)
             ms_de = _events_time(torch, stepd, nd, stream)
             eq = bool(torch.equal(outd.view(torch.int16), stepd().view(torch.int16)))
-            # the indexer's projections alone (its cached launch: both products in one
-            # kernel when the route is 'decode')
-            pl = ixd._plan
-            route_d = pl.route if pl is not None else None
+            # the indexer's projections alone (both products in one kernel when the route is
+            # 'decode'), prepared on this stream: the module's own plan may be of the side stream
+            pl = t2._IndexerPlan(ixd, xd, qrd, 8191, 0, None)
+            route_d = pl.route
             ms_dp = _events_time(torch, pl.proj, nd, stream) if route_d == "decode" else None
         dsa_decode = {
             "workload": "configs[4] decode: 1 new token at position 8191 of 8192; indexer 64x128 (qr[1,1,1536], "
