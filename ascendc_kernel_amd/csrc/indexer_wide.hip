@@ -488,17 +488,21 @@ __global__ __launch_bounds__(512) void ix_wide_kernel(WideParams p) {
   // go to LDS, one load per thread, so the rotation waits for one memory latency in all (read
   // pair by pair from memory it took 2.5 us of a decode step).
   // Waves of no token (three in four of a one-token step) read no rows: 8192 candidates without
-  // the table 16.1 -> 14.7 us at one token, 21.5 -> 18.9 at eight.
+  // the table 16.0 -> 14.9 us at one token, 21.5 -> 19.5 at eight.
   const int hq = head_of_row<KY>(col, y);
   bf16x8 qa[8];
   {
-    const uint16_t* qrow = p.q + (row_bt * kWH + hq) * kWD + 8 * hf;
+    // (one token's rows as a resource, empty for an absent token: in a branch the loads would be
+    // waited for at its end, 0.2-0.5 % at 300 tokens)
+    const int ts = t0 + (wis >> 1);
+    const __amdgpu_buffer_rsrc_t qrs =
+        buf_rsrc(p.q + ((int64_t)b * p.S + min(ts, p.S - 1)) * (kWH * kWD), ts < p.S ? (uint32_t)(kWH * kWD * 2) : 0u);
+    const int qoff = (hq * kWD + 8 * hf) * 2;
     const int half_rd = p.rd >> 1;
     const int rbase = kWD - p.rd;
     u32x4 v[8];
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks)
-      v[ks] = tok_ok ? *reinterpret_cast<const u32x4*>(qrow + 16 * ks) : u32x4{0u, 0u, 0u, 0u};
+    for (int ks = 0; ks < 8; ++ks) v[ks] = __builtin_amdgcn_raw_buffer_load_b128(qrs, qoff + 32 * ks, 0, 0);
     if (p.freqs != nullptr) {  // (rows of no token stay zero)
       float2* tab = reinterpret_cast<float2*>(hist);  // [kTok][rd / 2], at most 2 KB of the 8 KB
       const int rows = min(kTok, p.S - t0);
