@@ -278,11 +278,12 @@ class Model(nn.Module):
         dev = x.device
         # (A plan reads kv_cache and freqs_cis in place, so it sees their updates; it is kept
         # only where neither needs a contiguous copy, which would not.)
-        if (dev.type == _native.PLAN_DEVICE_TYPE and x.is_contiguous() and qr.is_contiguous() and kv.dim() == 3
-                and kv.stride(2) == 1 and kv.stride(1) == kv.shape[2] and fc.is_contiguous()):
+        kv_shape, kv_stride = kv.shape, kv.stride()
+        if (dev.type == _native.PLAN_DEVICE_TYPE and x.is_contiguous() and qr.is_contiguous() and len(kv_shape) == 3
+                and kv_stride[2] == 1 and kv_stride[1] == kv_shape[2] and fc.is_contiguous()):
             key = (x.data_ptr(), qr.data_ptr(), x.shape, qr.shape, x.dtype, qr.dtype, start_pos, offset,
-                   wq.data_ptr(), wq._version, wp.data_ptr(), wp._version, kv.data_ptr(), kv.shape,
-                   kv.stride(), kv.dtype, fc.data_ptr(), fc.shape, fc.dtype, _native.stream_handle(dev),
+                   wq.data_ptr(), wq._version, wp.data_ptr(), wp._version, kv.data_ptr(), kv_shape,
+                   kv_stride, kv.dtype, fc.data_ptr(), fc.shape, fc.dtype, _native.stream_handle(dev),
                    self.rope_mode, self.compress_ratio, self.index_topk, self.n_heads, self.n_local_heads,
                    self.head_dim, self.rope_head_dim, float(self.softmax_scale))
             plan = self._plan
